@@ -464,41 +464,55 @@ __device__ __forceinline__ Col<SymT> column(const SymT* sym, const uint32_t* blk
     return col;
 }
 
-// f(v, b, in) for the column symbols of ranks n-1, n-2, .., 0 (the column's
-// 16-symbol chunk k sits at p + 128 k), read with 16-byte loads issued one
-// chunk ahead.  b is the symbol's index in its chunk (a compile-time
-// constant after unrolling).  Only a column's top chunk can be partial.
-// Control flow is wave-uniform: the loop runs while any lane has chunks left,
-// takes the unconditional path when every lane holds a full chunk, the same
-// path with finished lanes masked off when every lane holds a full chunk or
-// none, and otherwise passes a per-lane predicate; f must leave its state
-// unchanged when in == false.
-template <typename SymT, typename F>
-__device__ __forceinline__ void for_each_rev(const SymT* p, int n, F&& f) {
-    int k = n > 0 ? (n - 1) >> 4 : -1;   // current chunk
-    Chunk16<SymT> cur = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)}, nxt = cur;
-    if (k >= 0) cur = gload_chunk(p + 128 * (int64_t)k);
-    if (k >= 1) nxt = gload_chunk(p + 128 * (int64_t)(k - 1));
-    while (__any(k >= 0)) {
-        const int hi_b = k < 0 ? 0 : (n - 16 * k < 16 ? n - 16 * k : 16);
-        if (__all(hi_b == 16)) {
+// f(e, b, in) for the column symbols of ranks n-1, n-2, .., 0 (the column's
+// 16-symbol chunk k sits at p + 128 k); entries(chunk, hi_b, e, whole) turns a chunk
+// into its 16 table entries, all read before the first is used, so a chunk's
+// serial chain waits for the LDS once and not per symbol (whole: hi_b is 16, or
+// 0 in lanes whose entries are not used).  b is the symbol's
+// index in its chunk (a compile-time constant after unrolling); after a
+// chunk's symbols done() runs.
+//
+// DEPTH chunks of 16-byte loads are in flight per lane: a chunk's registers
+// are reloaded, for the chunk DEPTH further down, as soon as its entries are
+// read.  The loads are unconditional (a lane past its last chunk reads chunk 0
+// again) and the trip count is uniform over the calling lanes (votes, not
+// shuffles: some of the wave's lanes may not be here): with a load under a condition, or
+// with registers that move from "next" to "current", the compiler waits for
+// the newest load before the symbols it was to be hidden behind (47,000 cycles
+// per block and wave against 18,000 here, one wave per SIMD).
+// Only a column's top chunk can be partial: it comes first, with a per-lane
+// predicate (f must leave its state unchanged when in == false); after it
+// lanes without chunks left are masked off.
+template <int DEPTH, typename SymT, typename E, typename F, typename D>
+__device__ __forceinline__ void for_each_rev(const SymT* p, int n, E&& entries, F&& f, D&& done) {
+    const int k = n > 0 ? (n - 1) >> 4 : -1;   // top chunk
+    if (!__any(k >= 0)) return;
+    auto at = [&](int i) { return gload_chunk(p + 128 * (i > 0 ? i : 0)); };
+    uint32_t e[16];
+    Chunk16<SymT> buf[DEPTH];
+    {
+        const Chunk16<SymT> top = at(k);
 #pragma unroll
-            for (int b = 15; b >= 0; b--) f(cur.get(b), b, true);
-        } else if (__all(hi_b == 16 || hi_b == 0)) {
-            // every lane holds a full chunk or has none left (the columns of a
-            // wave end at different chunks): the full path, finished lanes
-            // masked off
-            if (hi_b == 16) {
+        for (int j = 0; j < DEPTH; j++) buf[j] = at(k - 1 - j);
+        const int hi_b = k < 0 ? 0 : n - 16 * k;
+        entries(top, hi_b, e, false);
 #pragma unroll
-                for (int b = 15; b >= 0; b--) f(cur.get(b), b, true);
+        for (int b = 15; b >= 0; b--) f(e[b], b, b < hi_b);
+        done();
+    }
+    for (int it = 1; __any(it <= k); it += DEPTH) {
+#pragma unroll
+        for (int j = 0; j < DEPTH; j++) {
+            const bool live = it + j <= k;
+            if (!__any(live)) break;   // uniform over the calling lanes
+            entries(buf[j], live ? 16 : 0, e, true);   // every lane: no merge with the old entries
+            buf[j] = at(k - it - j - DEPTH);
+            if (live) {
+#pragma unroll
+                for (int b = 15; b >= 0; b--) f(e[b], b, true);
+                done();
             }
-        } else {
-#pragma unroll
-            for (int b = 15; b >= 0; b--) f(cur.get(b), b, b < hi_b);
         }
-        k--;
-        cur = nxt;
-        if (k >= 1) nxt = gload_chunk(p + 128 * (int64_t)(k - 1));
     }
 }
 
@@ -524,9 +538,22 @@ __host__ __device__ inline EncWork enc_layout(int64_t n_chunks, int64_t n_vector
 }
 
 constexpr int kEncBlocks = 16;   // blocks per encode workgroup (x 16 streams)
+constexpr int kEncRing = 8;      // scratch words per lane waiting in LDS
 
-// Grid: (block groups, chunks).  The scratch words of a task are collected in
-// a 4-word LDS queue per lane and stored as aligned 16-byte pieces.
+// Grid: (block groups, chunks).
+//
+// On a full chip the kernel issues VALU instructions nearly all the time; with
+// few blocks (a layer's prompt: one wave per SIMD or less) it waits for the
+// serial chain of its 256 or so symbols, their loads and lookups.  Encode and
+// offset scan, before / after the loads of for_each_rev and the branch-free
+// word output below: 102 blocks 38.1 / 25.4 us, 2048 blocks 47.6 / 32.4 us,
+// 131072 blocks (64 chunks of 8192 tokens) 412.7 / 364.1 us; the wide path's
+// 4096 blocks 84.9 / 60 us.  The bits of three symbols (at most 30) enter a 64-bit
+// accumulator, then the word they may have completed is written to the lane's
+// ring in LDS whether it is complete or not (an incomplete one is written
+// again, and overwritten, by the next three symbols): no branch and no
+// divergence per word.  Full groups of four words leave the ring once per
+// 16-symbol chunk as aligned 16-byte stores.
 template <typename SymT>
 __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ sym, const uint32_t* __restrict__ blk_n1,
                                                       int64_t nblk, int64_t V, const lq_table* __restrict__ tables,
@@ -540,9 +567,16 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
     // memory, so the workgroup's LDS stays that of the int8 encoder.
     constexpr bool kWide = sizeof(SymT) == 2;
     constexpr int kWin = kWide ? 256 : 264;
-    __shared__ uint32_t senc[LQ_STREAMS][kWin + 1];
+    // The ring comes first: lanes without a symbol look up whatever byte their
+    // chunk holds, at most 255 entries before or after their row's first.
+    __shared__ struct {
+        uint32_t sq[kEncRing][256];   // per-lane ring of scratch words
+        uint32_t senc[LQ_STREAMS][kWin + 1];
+    } sm;
+    static_assert(kWin + 1 > 257 || sizeof(SymT) == 2, "any byte's lookup stays inside the table rows");
+    auto& sq = sm.sq;
+    auto& senc = sm.senc;
     __shared__ int slo[LQ_STREAMS], snsym[LQ_STREAMS];
-    __shared__ uint32_t sq[4][256];   // per-lane queue of scratch words (4: seven workgroups fit a CU's LDS)
     const int tid = threadIdx.x;
     const int64_t chunk = blockIdx.y;
     // wave = one coset of 8 blocks (lanes: block-major, coordinate-minor), so
@@ -550,17 +584,18 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
     const int64_t g = (int64_t)blockIdx.x * kEncBlocks + ((tid >> 3) & 15);
     const int st = ((tid >> 7) << 3) | (tid & 7);
     const lq_table* T = tables + chunk * LQ_STREAMS;
-    // first alphabet entry of stream s's LDS window
-    auto win0 = [&](int s) -> int {
-        if constexpr (!kWide) return 0;
-        const int n = T[s].n_sym, w = -T[s].lo - kWin / 2;
-        return n <= kWin || w <= 0 ? 0 : (w < n - kWin ? w : n - kWin);
-    };
-    for (int i = tid; i < LQ_STREAMS * kWin; i += 256) {
-        const int s = i / kWin, j = i % kWin, w0 = win0(s);
-        senc[s][j] = j + w0 < T[s].n_sym ? encx_of(T[s].enc[j + w0]) : 0u;
+    {   // stage the tables: 16 threads per stream, its live entries only
+        const int s = tid >> 4;
+        const int n = T[s].n_sym, lo = T[s].lo;
+        int w0 = 0;   // first alphabet entry of the stream's LDS window
+        if constexpr (kWide) {
+            const int w = -lo - kWin / 2;
+            w0 = n <= kWin || w <= 0 ? 0 : (w < n - kWin ? w : n - kWin);
+        }
+        const int m = n - w0 < kWin ? n - w0 : kWin;
+        for (int j = tid & 15; j < m; j += 16) senc[s][j] = encx_of(T[s].enc[j + w0]);
+        if ((tid & 15) == 0) { slo[s] = lo + w0; snsym[s] = n; }
     }
-    if (tid < LQ_STREAMS) { slo[tid] = T[tid].lo + win0(tid); snsym[tid] = T[tid].n_sym; }
     __syncthreads();
     if (g >= nblk) return;
     const int64_t task = (chunk * LQ_STREAMS + st) * nblk + g;
@@ -570,20 +605,41 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
         return;
     }
     const int c = st >> 3, idx = st & 7;
-    const uint32_t* encs = senc[st];
     const int lo_sym = slo[st];   // symbol of the window's first entry (a valid symbol)
     const uint32_t* const genc = T[st].enc;
     const int glo = T[st].lo;
-    auto enc = [&](int v) -> uint32_t {   // entry of symbol value v
-        const uint32_t j = (uint32_t)(v - lo_sym);
+    const uint32_t row = (uint32_t)(uintptr_t)(lds_u32*)&senc[st][0];   // LDS byte address of the window
+    // the table entries of a chunk's first hi_b symbols (of the others: some
+    // entry)
+    auto entries = [&](const Chunk16<SymT>& ch, int hi_b, uint32_t e[16], bool whole) {
         if constexpr (!kWide) {
-            return encs[j];
+            // entry address of symbol value v: row + 4 (v - lo_sym), one 4-byte
+            // dot product with the symbol's byte picked by the weights
+            const int w[4] = {(int)ch.a.x, (int)ch.a.y, (int)ch.a.z, (int)ch.a.w};
+            const int base = (int)row - 4 * lo_sym;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                uint32_t a = (uint32_t)__builtin_amdgcn_sdot4(w[i >> 2], 4 << (8 * (i & 3)), base, false);
+                if (!whole) a = i < hi_b ? a : row;
+                e[i] = *(const lds_u32*)(uintptr_t)a;
+            }
         } else {
-            uint32_t e = encs[j < (uint32_t)kWin ? j : (uint32_t)kWin - 1u];
-            if (j >= (uint32_t)kWin) e = encx_of(genc[v - glo]);   // outside the window (rare)
-            return e;
+            uint32_t j[16], out = 0;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                j[i] = whole || i < hi_b ? (uint32_t)(ch.get(i) - lo_sym) : 0u;
+                const uint32_t jj = j[i] < (uint32_t)kWin ? j[i] : (uint32_t)kWin - 1u;
+                out |= j[i] >= (uint32_t)kWin ? 1u << i : 0u;
+                e[i] = *(const lds_u32*)(uintptr_t)(row + 4u * jj);
+            }
+            if (out && hi_b) {   // symbols outside the window (rare)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (out & (1u << i)) e[i] = encx_of(genc[(int)j[i] + lo_sym - glo]);
+            }
         }
     };
+    auto nothing = []() {};
 
     // ---- state entering block g (encode order runs from the stream end down)
     uint32_t x = kL;
@@ -606,77 +662,69 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
             const int cnt = (b == hb && !exact) ? need : col.n;
             if (lo == hi) {
                 uint32_t xx = lo, k;
-                for_each_rev(col.p, cnt, [&](int v, int, bool in) {
-                    const uint32_t xn = encx_step(xx, enc(in ? v : lo_sym), &k);
+                for_each_rev<1>(col.p, cnt, entries, [&](uint32_t e, int, bool in) {
+                    const uint32_t xn = encx_step(xx, e, &k);
                     xx = in ? xn : xx;
-                });
+                }, nothing);
                 lo = hi = xx;
             } else {
-                for_each_rev(col.p, cnt, [&](int v, int, bool in) {
+                for_each_rev<1>(col.p, cnt, entries, [&](uint32_t e, int, bool in) {
                     uint32_t l2 = lo, h2 = hi;
-                    hull_step(l2, h2, enc(in ? v : lo_sym));
+                    hull_step(l2, h2, e);
                     lo = in ? l2 : lo;
                     hi = in ? h2 : hi;
-                });
+                }, nothing);
             }
         }
         if (lo == hi) { x = lo; break; }
         window *= 8;
     }
 
-    // ---- encode block g, bits right-aligned in the task's scratch region
+    // ---- encode block g, bits right-aligned in the task's scratch region:
+    // words leave in decreasing address order from kCapW - 1
     Col<SymT> col = column(sym, blk_n1, chunk, nblk, V, g, c, idx);
     uint32_t* scr = scratch + task * (int64_t)kCapW;
-    // words leave in decreasing address order from kCapW - 1; word j of the
-    // current 4-word group waits in LDS at qcol[(3 - j) * 256] (this lane's
-    // column, so a wave's writes are contiguous) and the group leaves as one
-    // 16-byte store when full
-    uint32_t* const qcol = &sq[0][tid];
-    int nq = 0, gbase = kCapW - 4, nwords = 0;
-    auto push = [&](uint32_t word) {
-        qcol[(3 - nq) * 256] = word;
-        nwords++;
-        if (++nq == 4) {
-            *reinterpret_cast<uint4*>(scr + gbase) = make_uint4(qcol[0], qcol[256], qcol[512], qcol[768]);
-            gbase -= 4;
-            nq = 0;
-        }
-    };
+    uint32_t* const qcol = &sq[0][tid];   // ring slot s at qcol[256 s]: a wave's accesses are contiguous
     // Bit accumulator (ahi:alo): the emitted bits sit at the top, newest
-    // highest; a symbol's group (the k low bits of xin, bit k - 1 first in the
-    // final stream) enters by one funnel shift of (xin:ahi:alo) right by k, two
-    // v_alignbit (k <= 10; k = 0 leaves all three in place).  Below the bits a
-    // single 1 (the sentinel) marks their end, so no bit count is kept: 32 or
-    // more bits are held exactly when the low word is nonzero.  The oldest 32
-    // bits then leave as one word, bit-reversed so that the oldest bit is the
-    // word's most significant, as the stream order wants.
-    uint32_t ahi = 0x80000000u, alo = 0u;
-    auto take_word = [&]() {   // needs alo != 0
-        const uint32_t s = (uint32_t)__builtin_ctz(alo);   // sentinel position
-        const uint32_t raw = (uint32_t)((((uint64_t)ahi << 32) | alo) >> (s + 1u));
-        push(__builtin_bitreverse32(raw));
-        ahi = ((ahi >> s) | 1u) << s;   // sentinel moves up 32 bits (to bit s of the high word)
-        alo = 0u;
+    // highest; a symbol's group (the k low bits of x, bit k - 1 first in the
+    // final stream) enters by one funnel shift of (x:ahi:alo) right by k, two
+    // v_alignbit (k <= 10; k = 0 leaves all three in place).  total counts the
+    // bits; word w of the block holds bits 32 w .. 32 w + 31, so after a group
+    // of symbols the word being filled has n = (total & 31) + ks bits, the top
+    // n of the accumulator: bits past them are older words' and drop out.  The
+    // word is bit-reversed so that its oldest bit is the most significant, as
+    // the stream order wants.
+    uint32_t ahi = 0u, alo = 0u, total = 0u, ks = 0u, flushed = 0u;
+    auto emit = [&]() {   // ks <= 30: at most one word is completed
+        const uint32_t n = (total & 31u) + ks;
+        const uint32_t raw = (uint32_t)((((uint64_t)ahi << 32) | alo) >> ((0u - n) & 63u));
+        qcol[256u * ((total >> 5) & (kEncRing - 1))] = __builtin_bitreverse32(raw);
+        total += ks;
+        ks = 0u;
     };
-    for_each_rev(col.p, col.n, [&](int v, int b, bool in) {
+    auto store4 = [&]() {   // words flushed .. flushed + 3 of the block, as one 16-byte store
+        const uint32_t* q = qcol + 256u * (flushed & 4u);
+        *reinterpret_cast<uint4*>(scr + (kCapW - 4 - (int)flushed)) = make_uint4(q[768], q[512], q[256], q[0]);
+        flushed += 4u;
+    };
+    // fewer than 4 words wait before a chunk and it completes at most 5: 8 fit the ring
+    for_each_rev<4>(col.p, col.n, entries, [&](uint32_t e, int b, bool in) {
         uint32_t k;
         const uint32_t xin = x;
-        const uint32_t xn = encx_step(xin, enc(in ? v : lo_sym), &k);
+        const uint32_t xn = encx_step(xin, e, &k);
         k = in ? k : 0u;
         x = in ? xn : xin;
         alo = __builtin_amdgcn_alignbit(ahi, alo, k);
         ahi = __builtin_amdgcn_alignbit(xin, ahi, k);
-        // at most 3 symbols (<= 30 bits) since the last check: <= 61 bits and the sentinel
-        if (b % 3 == 0 && alo != 0u) take_word();
+        ks += k;
+        if (b % 3 == 0) emit();
+    }, [&]() {
+        while ((total >> 5) >= flushed + 4u) store4();
     });
-    if (alo != 0u) take_word();   // the range may end between check points
-    // fewer than 32 bits left: the sentinel is in the high word
-    const uint32_t nacc = 31u - (uint32_t)__builtin_ctz(ahi);
-    const uint32_t total = 32u * (uint32_t)nwords + nacc;
-    if (nacc) push(__builtin_bitreverse32(ahi >> (32u - nacc)));
-    if (nq) {   // the last, partial group: its words sit in the top nq slots
-        *reinterpret_cast<uint4*>(scr + gbase) = make_uint4(qcol[0], qcol[256], qcol[512], qcol[768]);
-    }
+    const uint32_t nacc = total & 31u;
+    if (nacc) qcol[256u * ((total >> 5) & (kEncRing - 1))] = __builtin_bitreverse32(ahi >> (32u - nacc));
+    // the last, partial group's words sit in the top slots of its 16 bytes
+    while (((total + 31u) >> 5) > flushed) store4();
     blk_bits[task] = total;
     blk_state[task] = (uint16_t)x;
 }

@@ -283,6 +283,7 @@ __global__ __launch_bounds__(kTileThreads) void k_compact_encode(
     __shared__ int64_t s_excl;
     __shared__ float s_sc[2], s_sf[2];
     __shared__ int s_fd[2], s_bad[2];
+    __shared__ double sp[SC ? 2 : 1][SC ? kPartsLds : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid == 0) s_t = (int)atomicAdd(ticket, 1u);
     __syncthreads();
@@ -295,19 +296,7 @@ __global__ __launch_bounds__(kTileThreads) void k_compact_encode(
         const int nhd = (int)(last / bph - h0) + 1;   // 1 or 2
         if (wave < nhd) {
             const int64_t h = h0 + wave;
-            const double* wp = as.work + h * as.parts;
-            double acc = 0.0;
-            for (int p0 = 0; p0 < as.parts; p0 += 64) {
-                const double v = p0 + lane < as.parts ? wp[p0 + lane] : 0.0;
-                const int m = as.parts - p0 < 64 ? as.parts - p0 : 64;
-                const uint64_t vb = __builtin_bit_cast(uint64_t, v);
-                const int lo = (int)(uint32_t)vb, hi = (int)(uint32_t)(vb >> 32);
-                for (int i = 0; i < m; i++) {
-                    const uint64_t b = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(lo, i) |
-                                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi, i) << 32);
-                    acc += __builtin_bit_cast(double, b);
-                }
-            }
+            const double acc = parts_sum(as.work + h * as.parts, as.parts, lane, sp[SC ? wave : 0]);
             if (lane == 0) {
                 float s2;
                 const float s = head_scale(acc, bph * 8, as.scale_bits, &s2);

@@ -99,21 +99,23 @@ __device__ void fastdiv_check(float s, int32_t* word) {
 }
 
 // sigma^2, scales (llm/compressed_kv_cache.py:189-196) and fast-division flag.
-__global__ void k_head_finalize(const double* __restrict__ work, int parts, int64_t elems_per_head,
+__global__ __launch_bounds__(256) void k_head_finalize(const double* __restrict__ work, int parts, int64_t elems_per_head,
                                 int64_t n_heads, const int32_t* __restrict__ chunk_bits, int dtype,
                                 float* __restrict__ sigma2, float* __restrict__ scale32,
                                 uint16_t* __restrict__ scale16, int32_t* __restrict__ fastdiv) {
     int64_t h = blockIdx.x;
     __shared__ float sc;
-    if (threadIdx.x == 0) {
-        double acc = 0.0;
-        for (int p = 0; p < parts; p++) acc += work[h * parts + p];
-        float s2;
-        const float s = head_scale(acc, elems_per_head, chunk_bits[h / n_heads], &s2);
-        sigma2[h] = s2;
-        scale32[h] = s;
-        scale16[h] = f2h(s);
-        sc = s;
+    __shared__ double sp[kPartsLds];
+    if (threadIdx.x < 64) {
+        const double acc = parts_sum(work + h * parts, parts, (int)threadIdx.x, sp);
+        if (threadIdx.x == 0) {
+            float s2;
+            const float s = head_scale(acc, elems_per_head, chunk_bits[h / n_heads], &s2);
+            sigma2[h] = s2;
+            scale32[h] = s;
+            scale16[h] = f2h(s);
+            sc = s;
+        }
     }
     __syncthreads();
     if (dtype == LQ_F16) {

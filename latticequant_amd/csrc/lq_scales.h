@@ -108,6 +108,37 @@ __device__ __forceinline__ void head_sumsq_part(const void* __restrict__ x, int 
     if (threadIdx.x == 0) work[h * parts + p] = red[0];
 }
 
+// w[0] + w[1] + .. + w[parts - 1] in that order (one rounding order for every
+// launch shape), in every lane of the calling wave (lane: its lane id; lds: 512
+// doubles of the wave's own).  A load per term would put a memory latency into
+// every link of the serial chain; 512 terms at a time are loaded together and
+// staged in LDS, from where they reach the chain eight ahead of their use (the
+// finalisation of 512 parts: 31.8 -> 7.3 us, of 128: 10.0 -> 4.0 us).
+constexpr int kPartsLds = 512;
+__device__ __forceinline__ double parts_sum(const double* __restrict__ w, int parts, int lane, double* lds) {
+    double acc = 0.0;
+    for (int p0 = 0; p0 < parts; p0 += kPartsLds) {
+        const int m = parts - p0 < kPartsLds ? parts - p0 : kPartsLds;
+        double v[kPartsLds / 64];
+#pragma unroll
+        for (int u = 0; u < kPartsLds / 64; u++) v[u] = 64 * u + lane < m ? w[p0 + 64 * u + lane] : 0.0;
+#pragma unroll
+        for (int u = 0; u < kPartsLds / 64; u++) lds[64 * u + lane] = v[u];
+        __builtin_amdgcn_wave_barrier();
+        int i = 0;
+        for (; i + 8 <= m; i += 8) {
+            double t[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) t[j] = lds[i + j];
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc += t[j];
+        }
+        for (; i < m; i++) acc += lds[i];
+        __builtin_amdgcn_wave_barrier();
+    }
+    return acc;
+}
+
 // Exhaustive check that the three-op division equals IEEE division for every
 // fp16 significand M in [1, 2047] (every fp16 value is M * 2^E, and both forms
 // are invariant under that power of two), by the whole workgroup; bad: an LDS

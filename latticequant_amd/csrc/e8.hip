@@ -137,14 +137,13 @@ __global__ void k_scale_fastdiv(const float* __restrict__ scale32, int dtype, in
 // -------------------------------------------------------- chunk quantize --
 
 constexpr int kQThreads = 256;
-constexpr int kQBlocksPerWG = 8;
+constexpr int kQBlocksPerWG = 8;   // at most (quant_blocks_per_wg)
 // LDS histogram row of one stream: 256 bins indexed by the symbol's low byte,
 // padded so consecutive rows start 8 banks apart
 constexpr int kHRow = 256 + 8;
 constexpr int64_t kMaxBph = 1 << 30;   // vectors per head (2^27 tokens of 128 dims): in-head offsets stay int32
 
-// One workgroup quantizes kQBlocksPerWG consecutive LQ_BLK-vector blocks of one
-// chunk.  Per block it writes the coset bitmap (wave ballots, i.e. the
+// One workgroup quantizes bpw consecutive LQ_BLK-vector blocks of one chunk.  Per block it writes the coset bitmap (wave ballots, i.e. the
 // reference's LSB-first pack_coset_bits layout), the coset-1 count and the
 // symbols in the interleaved column layout of sym_pos (element index; int8
 // symbols, or int16 for the wide path), staged in LDS so the global stores are
@@ -233,7 +232,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
     const float* __restrict__ scale32, const int32_t* __restrict__ fastdiv, SymT* __restrict__ sym,
     uint8_t* __restrict__ coset_bits, uint32_t* __restrict__ blk_n1, uint32_t* __restrict__ hist,
     int32_t* __restrict__ minmax, int32_t* __restrict__ status, void* __restrict__ deq, int deq_dtype,
-    const int64_t* __restrict__ dseed, const float* __restrict__ signs, int lpr, float rdiv) {
+    const int64_t* __restrict__ dseed, const float* __restrict__ signs, int lpr, float rdiv, int bpw) {
     constexpr bool kWide = sizeof(SymT) == 2;
     constexpr int kSymMin = kWide ? -32768 : -128, kSymMax = kWide ? 32767 : 127;
     __shared__ uint32_t shist[kWide ? 1 : LQ_STREAMS * kHRow];
@@ -247,9 +246,9 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t wg_per_chunk = (nblk + kQBlocksPerWG - 1) / kQBlocksPerWG;
+    const int64_t wg_per_chunk = (nblk + bpw - 1) / bpw;
     const int64_t chunk = blockIdx.x / wg_per_chunk;
-    const int64_t b0 = (blockIdx.x % wg_per_chunk) * kQBlocksPerWG;
+    const int64_t b0 = (blockIdx.x % wg_per_chunk) * bpw;
     const int64_t V = n_heads * bph;
 
     if constexpr (!kWide) {
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
     int tmin[2] = {INT_MAX, INT_MAX}, tmax[2] = {INT_MIN, INT_MIN};
 
     int flag = 0;
-    for (int bi = 0; bi < kQBlocksPerWG; bi++) {
+    for (int bi = 0; bi < bpw; bi++) {
         const int64_t blk = b0 + bi;
         if (blk >= nblk) break;
         const int64_t vbase = blk * kBlk;
@@ -567,6 +566,20 @@ __global__ __launch_bounds__(256) void k_chunk_hist_wide(const int16_t* __restri
     }
 }
 
+// Blocks per quantizer workgroup.  A workgroup takes its blocks one after the
+// other (about 5 us each on an idle chip) and adds its histogram to the
+// chunk's at the end (contended atomics), so few blocks are spread over many
+// workgroups and many blocks over 8 each: one more block per 1024 blocks in
+// the launch (four workgroups per CU).  Measured, fp16 with dequantised rows,
+// 1 / 2 / 4 / 8 blocks per workgroup: 102 blocks 11.2 / 15.4 / 23.8 / 40.6 us,
+// 2048 blocks 41 / 29.5 / 32.2 / 46.0 us, 4096 blocks 67 / 52 / 46.8 / 53.8 us,
+// 8192 blocks 121 / 81 / 67.7 / 65.7 us; 131072 blocks (no rows) 865 / 673 /
+// 589 / 561 us.
+inline int quant_blocks_per_wg(int64_t n_chunks, int64_t nblk) {
+    const int64_t b = (n_chunks * nblk + 1023) / 1024;
+    return (int)(b < kQBlocksPerWG ? b : kQBlocksPerWG);
+}
+
 inline int launch_status() { return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_LAUNCH; }
 
 }  // namespace
@@ -686,16 +699,17 @@ int lq_chunk_quantize(const void* d_x, int dtype, int64_t n_chunks, int64_t n_he
     if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || bph > kMaxBph || dtype < 0 || dtype > 2) return LQ_ERR_ARG;
     const int64_t V = n_heads * bph;
     const int64_t nblk = (V + kBlk - 1) / kBlk;
-    const int64_t wg = n_chunks * ((nblk + kQBlocksPerWG - 1) / kQBlocksPerWG);
+    const int bpw = quant_blocks_per_wg(n_chunks, nblk);
+    const int64_t wg = n_chunks * ((nblk + bpw - 1) / bpw);
     if (d_dither_seed)
         hipLaunchKernelGGL((k_chunk_quantize<int8_t, true>), dim3((unsigned)wg), dim3(kQThreads), 0, s, d_x, dtype,
                            n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1, d_hist, nullptr,
-                           d_status, d_deq, deq_dtype, d_dither_seed, nullptr, 1, 1.0f);
+                           d_status, d_deq, deq_dtype, d_dither_seed, nullptr, 1, 1.0f, bpw);
     else if (bph >= kBlk && !d_deq) {
 #define LQ_LEAN(DT)                                                                                              \
         hipLaunchKernelGGL((k_chunk_quantize<int8_t, false, true, false, DT>), dim3((unsigned)wg), dim3(kQThreads),  \
                            0, s, d_x, dtype, n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1, \
-                           d_hist, nullptr, d_status, nullptr, deq_dtype, nullptr, nullptr, 1, 1.0f)
+                           d_hist, nullptr, d_status, nullptr, deq_dtype, nullptr, nullptr, 1, 1.0f, bpw)
         if (dtype == LQ_F16) LQ_LEAN(LQ_F16);
         else if (dtype == LQ_BF16) LQ_LEAN(LQ_BF16);
         else LQ_LEAN(LQ_F32);
@@ -704,7 +718,7 @@ int lq_chunk_quantize(const void* d_x, int dtype, int64_t n_chunks, int64_t n_he
     else
         hipLaunchKernelGGL((k_chunk_quantize<int8_t, false>), dim3((unsigned)wg), dim3(kQThreads), 0, s, d_x, dtype,
                            n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1, d_hist, nullptr,
-                           d_status, d_deq, deq_dtype, nullptr, nullptr, 1, 1.0f);
+                           d_status, d_deq, deq_dtype, nullptr, nullptr, 1, 1.0f, bpw);
     return launch_status();
 }
 
@@ -720,13 +734,14 @@ int lq_chunk_quantize_rht(const void* d_x, int dtype, int64_t n_chunks, int64_t 
     if (head_dim < 8 || head_dim > 128 || (head_dim & (head_dim - 1)) || bph % (head_dim / 8)) return LQ_ERR_ARG;
     const int64_t V = n_heads * bph;
     const int64_t nblk = (V + kBlk - 1) / kBlk;
-    const int64_t wg = n_chunks * ((nblk + kQBlocksPerWG - 1) / kQBlocksPerWG);
+    const int bpw = quant_blocks_per_wg(n_chunks, nblk);
+    const int64_t wg = n_chunks * ((nblk + bpw - 1) / bpw);
     const float div = (float)sqrt((double)head_dim);
     const int lpr = head_dim / 8;
 #define LQ_ROT(DI, LE, DT, LP)                                                                                    \
     hipLaunchKernelGGL((k_chunk_quantize<int8_t, DI, LE, true, DT, LP>), dim3((unsigned)wg), dim3(kQThreads), 0, s,  \
                        d_x, dtype, n_heads, bph, nblk, d_scale32, nullptr, d_sym, d_coset_bits, d_blk_n1, d_hist,      \
-                       nullptr, d_status, nullptr, (int)LQ_F32, d_dither_seed, d_signs, lpr, div)
+                       nullptr, d_status, nullptr, (int)LQ_F32, d_dither_seed, d_signs, lpr, div, bpw)
 #define LQ_ROT_LP(DI, DT)                                                                                         \
     if (lpr == 16) LQ_ROT(DI, true, DT, 16);                                                                      \
     else LQ_ROT(DI, true, DT, 0)
@@ -751,16 +766,17 @@ int lq_chunk_quantize_wide(const void* d_x, int dtype, int64_t n_chunks, int64_t
         return LQ_ERR_ARG;
     const int64_t V = n_heads * bph;
     const int64_t nblk = (V + kBlk - 1) / kBlk;
-    const int64_t wg = n_chunks * ((nblk + kQBlocksPerWG - 1) / kQBlocksPerWG);
+    const int bpw = quant_blocks_per_wg(n_chunks, nblk);
+    const int64_t wg = n_chunks * ((nblk + bpw - 1) / bpw);
     if (d_dither_seed)
         hipLaunchKernelGGL((k_chunk_quantize<int16_t, true>), dim3((unsigned)wg), dim3(kQThreads), 0, s, d_x, dtype,
                            n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1, nullptr, d_minmax,
-                           d_status, d_deq, deq_dtype, d_dither_seed, nullptr, 1, 1.0f);
+                           d_status, d_deq, deq_dtype, d_dither_seed, nullptr, 1, 1.0f, bpw);
     else if (bph >= kBlk && !d_deq) {
 #define LQ_LEAN(DT)                                                                                               \
         hipLaunchKernelGGL((k_chunk_quantize<int16_t, false, true, false, DT>), dim3((unsigned)wg), dim3(kQThreads),  \
                            0, s, d_x, dtype, n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1,  \
-                           nullptr, d_minmax, d_status, nullptr, deq_dtype, nullptr, nullptr, 1, 1.0f)
+                           nullptr, d_minmax, d_status, nullptr, deq_dtype, nullptr, nullptr, 1, 1.0f, bpw)
         if (dtype == LQ_F16) LQ_LEAN(LQ_F16);
         else if (dtype == LQ_BF16) LQ_LEAN(LQ_BF16);
         else LQ_LEAN(LQ_F32);
@@ -769,7 +785,7 @@ int lq_chunk_quantize_wide(const void* d_x, int dtype, int64_t n_chunks, int64_t
     else
         hipLaunchKernelGGL((k_chunk_quantize<int16_t, false>), dim3((unsigned)wg), dim3(kQThreads), 0, s, d_x, dtype,
                            n_heads, bph, nblk, d_scale32, d_fastdiv, d_sym, d_coset_bits, d_blk_n1, nullptr, d_minmax,
-                           d_status, d_deq, deq_dtype, nullptr, nullptr, 1, 1.0f);
+                           d_status, d_deq, deq_dtype, nullptr, nullptr, 1, 1.0f, bpw);
     return launch_status();
 }
 

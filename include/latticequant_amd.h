@@ -240,7 +240,8 @@ int lq_chunk_pack(int64_t n_chunks, int64_t n_vectors, const lq_table *d_tables,
                   const int64_t *d_chunk_base, uint32_t *d_words, hipStream_t s);
 
 /* Decode + dequantize a batch of chunks to (B, H, T, hd) in out_dtype:
- * fp16(q * float(scale16[head])).  d_lut_work: n_chunks * 16 * 1024 uint32.
+ * fp16(q * float(scale16[head])).  d_lut_work is not used and may be null (the
+ * decoder builds its LUTs in LDS).
  * d_words must have 2 readable words after the last chunk's last stream.
  * d_dither_seed (nullable): the seeds the chunks were quantized with; the
  * output is then (q - d) * scale16 (fp32 arithmetic, then out_dtype).
@@ -276,9 +277,9 @@ int lq_chunk_decode_rht(const uint32_t *d_words, const int64_t *d_chunk_base, co
                         uint32_t *d_lut_work, void *d_out, int out_dtype, const int64_t *d_dither_seed, hipStream_t s);
 
 /* Decoder LUTs of every stream of a chunk batch (n_chunks * 16 * 1024 uint32:
- * per slot: 31 - k | k << 5 | symbol index << 9 | (row * 1024 + (x' << k) - 1024) << 19,
+ * per slot: k | symbol index << 6 | (row * 1024 + (x' << k) - 1024) << 18,
  * with x' = freq + slot - cum, k its renormalisation bits and row = stream & 7),
- * as lq_chunk_decode builds them internally.  Part of the table stage of core/gpu_ans.py:88-95 (lookup). */
+ * as lq_decode_attention reads them.  Part of the table stage of core/gpu_ans.py:88-95 (lookup). */
 int lq_chunk_luts(const lq_table *d_tables, int64_t n_chunks, uint32_t *d_lut, hipStream_t s);
 
 /* ---------------------------------------------------- decode attention --- */

@@ -661,14 +661,13 @@ def decode_batch(enc: EncodedBatch, out_dtype: torch.dtype = torch.float16, out:
     fp16(q * float(scale16[head])) as _decompress_chunk computes it
     (llm/compressed_kv_cache.py:289-332).  rht_signs (C*B*H, hd): the rows are
     rotated back (inverse RHT of the fp32 dequantised rows, then out_dtype)
-    inside the decoder for hd <= 128, else by a separate pass."""
+    inside the decoder for hd <= 128, else by a separate pass.  lut_work is
+    accepted and not used (the decoder builds its LUTs on chip)."""
     lib = L.lib()
     dev = enc.words.device
     C = enc.n_chunks
     if out is None:
         out = torch.empty((C,) + tuple(enc.shape), dtype=out_dtype, device=dev)
-    if lut_work is None:
-        lut_work = _empty(C * L.LQ_STREAMS * L.LQ_L, torch.int32, dev)
     # an escape plan still on its way to the host is not waited for: the
     # escaped decoder reads the shifts on the device (k_j = 0 decodes plainly)
     esc = enc.extra.get("esc")
@@ -688,7 +687,7 @@ def decode_batch(enc: EncodedBatch, out_dtype: torch.dtype = torch.float16, out:
                                             enc.blk_state.data_ptr(), enc.coset_bits.data_ptr(), enc.tables.data_ptr(),
                                             enc.scale16.data_ptr(), C, enc.n_heads, enc.bph,
                                             hd if rht_signs is not None else 0, L.ptr(rht_signs), esc.k.data_ptr(),
-                                            esc.off.data_ptr(), esc.fine.data_ptr(), lut_work.data_ptr(),
+                                            esc.off.data_ptr(), esc.fine.data_ptr(), L.ptr(lut_work),
                                             out.data_ptr(), L.dtype_code(out.dtype),
                                             L.ptr(enc.extra.get("dither_seed")), L.stream_ptr(dev)),
                 "lq_chunk_decode_escaped")
@@ -697,7 +696,7 @@ def decode_batch(enc: EncodedBatch, out_dtype: torch.dtype = torch.float16, out:
         L.check(lib.lq_chunk_decode_rht(enc.words.data_ptr(), enc.chunk_base.data_ptr(), enc.stream_woff.data_ptr(),
                                         enc.blk_off.data_ptr(), enc.stream_nbits.data_ptr(), enc.blk_state.data_ptr(),
                                         enc.coset_bits.data_ptr(), enc.tables.data_ptr(), enc.scale16.data_ptr(), C,
-                                        enc.n_heads, enc.bph, hd, rht_signs.data_ptr(), lut_work.data_ptr(),
+                                        enc.n_heads, enc.bph, hd, rht_signs.data_ptr(), L.ptr(lut_work),
                                         out.data_ptr(), L.dtype_code(out.dtype),
                                         L.ptr(enc.extra.get("dither_seed")), L.stream_ptr(dev)), "lq_chunk_decode_rht")
         return out
@@ -705,7 +704,7 @@ def decode_batch(enc: EncodedBatch, out_dtype: torch.dtype = torch.float16, out:
                                 enc.blk_off.data_ptr(), enc.stream_nbits.data_ptr(), enc.blk_state.data_ptr(),
                                 enc.coset_bits.data_ptr(),
                                 enc.blk_n1.data_ptr(), enc.tables.data_ptr(), enc.scale16.data_ptr(), C, enc.n_heads,
-                                enc.bph, lut_work.data_ptr(), out.data_ptr(), L.dtype_code(out.dtype),
+                                enc.bph, L.ptr(lut_work), out.data_ptr(), L.dtype_code(out.dtype),
                                 L.ptr(enc.extra.get("dither_seed")), L.stream_ptr(dev)), "lq_chunk_decode")
     return out
 

@@ -434,7 +434,7 @@ __global__ __launch_bounds__(128) void k_attn_combine(const float* __restrict__ 
 }
 
 struct AttnWork {
-    int64_t lut_k, lut_v, s0, s1, vdec, rec, total;
+    int64_t lut_k, s0, s1, vdec, rec, total;
 };
 
 __host__ inline AttnWork attn_layout(int64_t n_chunks, int64_t n_heads, int64_t bph, int G) {
@@ -444,8 +444,7 @@ __host__ inline AttnWork attn_layout(int64_t n_chunks, int64_t n_heads, int64_t 
     const int64_t n_tsplit = (1024 + kSplit - 1) / kSplit;   // records reserved for the largest tail
     auto al = [](int64_t b) { return ((b + 255) / 256) * 256; };
     w.lut_k = 0;
-    w.lut_v = al(w.lut_k + n_chunks * LQ_STREAMS * kL * 4);
-    w.s0 = al(w.lut_v + n_chunks * LQ_STREAMS * kL * 4);
+    w.s0 = al(w.lut_k + n_chunks * LQ_STREAMS * kL * 4);
     w.s1 = al(w.s0 + n_heads * G * n_chunks * T * 4);
     w.vdec = al(w.s1 + n_heads * G * n_chunks * T * 4);
     w.rec = al(w.vdec + n_chunks * n_heads * bph * 8 * 2);
@@ -497,7 +496,6 @@ int lq_decode_attention(const lq_chunk_batch* k, const lq_chunk_batch* v, const 
     const AttnWork w = attn_layout(k->n_chunks, k->n_heads, k->bph, group);
     char* base = reinterpret_cast<char*>(d_work);
     uint32_t* lut_k = reinterpret_cast<uint32_t*>(base + w.lut_k);
-    uint32_t* lut_v = reinterpret_cast<uint32_t*>(base + w.lut_v);
     float* S0 = reinterpret_cast<float*>(base + w.s0);
     float* S1 = reinterpret_cast<float*>(base + w.s1);
     uint16_t* vdec = reinterpret_cast<uint16_t*>(base + w.vdec);
@@ -506,7 +504,7 @@ int lq_decode_attention(const lq_chunk_batch* k, const lq_chunk_batch* v, const 
     if (rc) return rc;
     // V: decode + dequantise to fp16 (n_chunks, n_heads, T, 128)
     rc = lq_chunk_decode(v->words, v->chunk_base, v->stream_woff, v->blk_off, v->stream_nbits, v->blk_state,
-                         v->coset_bits, v->blk_n1, v->tables, v->scale16, v->n_chunks, v->n_heads, v->bph, lut_v, vdec,
+                         v->coset_bits, v->blk_n1, v->tables, v->scale16, v->n_chunks, v->n_heads, v->bph, nullptr, vdec,
                          LQ_F16, nullptr, s);
     if (rc) return rc;
     const BatchArgs ak = to_args(k, lut_k);

@@ -365,15 +365,13 @@ __device__ __forceinline__ uint4 deq_staged_f16(const uint4& r, const half2_t lo
 // needs no per-coset constants: the biases are even (the parity of the seven
 // free fields is that of c0..c6), 2 u7 + parity = c7 + 512, and every field
 // u < 1024, so fp16 (1024 + u) - 1536 is the coordinate exactly.
-__device__ __forceinline__ bool chunk_biased(const lq_table* T16) {
-    bool ok = true;
-#pragma unroll
-    for (int st = 0; st < LQ_STREAMS; st++) {
-        const int n = T16[st].n_sym, lo = T16[st].lo;
-        const int lim = (st & 7) < 7 ? 512 : 256;
-        ok = ok && (n == 0 || (lo >= -lim && lo + n - 1 < lim));
-    }
-    return ok;
+// The calling wave (all 64 lanes) looks at one stream per lane: the sixteen
+// loads are in flight together.
+__device__ __forceinline__ bool chunk_biased(const lq_table* T16, int lane) {
+    const int st = lane & (LQ_STREAMS - 1);
+    const int n = T16[st].n_sym, lo = T16[st].lo;
+    const int lim = (st & 7) < 7 ? 512 : 256;
+    return __all(n == 0 || (lo >= -lim && lo + n - 1 < lim));
 }
 
 // A staged vector of biased fields dequantised to 8 fp16 values, packed in

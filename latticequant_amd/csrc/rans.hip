@@ -1047,14 +1047,10 @@ __global__ __launch_bounds__(256) void k_chunk_pack(int64_t n_streams_total, int
 
 // ------------------------------------------------------------ chunk decode --
 
-// Decoder LUT of every chunk stream (lut_entry format, lq_decode.h).
-// mode 0 (decode attention): stream st of a chunk sits at row st & 7 (the 8
-// LUTs of one coset form one LDS block) and the symbol field is the alphabet
-// index.  mode 1 (chunk decoder): row st & 15 (the 16 LUTs of a chunk form
-// one LDS block), and the symbol field is biased (chunk_biased) when the
-// chunk's alphabets allow it.
-__global__ __launch_bounds__(256) void k_chunk_lut(const lq_table* __restrict__ tables, uint32_t* __restrict__ lut,
-                                                   int mode) {
+// Decoder LUTs of every chunk stream for decode attention (lut_entry format,
+// lq_decode.h): stream st of a chunk sits at row st & 7 (the 8 LUTs of one
+// coset form one LDS block) and the symbol field is the alphabet index.
+__global__ __launch_bounds__(256) void k_chunk_lut(const lq_table* __restrict__ tables, uint32_t* __restrict__ lut) {
     __shared__ int32_t fr[LQ_MAXSYM];
     __shared__ int32_t cum[LQ_MAXSYM + 1];
     const int64_t sid = blockIdx.x;
@@ -1064,24 +1060,88 @@ __global__ __launch_bounds__(256) void k_chunk_lut(const lq_table* __restrict__ 
     for (int i = threadIdx.x; i < n; i += 256) fr[i] = (int32_t)enc_f(T->enc[i]);
     __syncthreads();
     exclusive_scan_array<BlockGroup>(fr, n, cum);
-    const int st = (int)(sid % LQ_STREAMS);
-    const uint32_t row = (uint32_t)st & (mode ? 15u : 7u);
-    uint32_t bias = 0;
-    if (mode && chunk_biased(tables + (sid - st))) bias = (uint32_t)(T->lo + ((st & 7) < 7 ? 512 : 256));
+    const uint32_t row = (uint32_t)(sid % LQ_STREAMS) & 7u;
     for (int slot = threadIdx.x; slot < kL; slot += 256) {
         int lo = 0, hi = n - 1;   // largest s with cum[s] <= slot
         while (lo < hi) {
             int mid = (lo + hi + 1) >> 1;
             if (cum[mid] <= slot) lo = mid; else hi = mid - 1;
         }
-        lut[sid * kL + slot] = lut_entry((uint32_t)lo + bias, (uint32_t)(fr[lo] + slot - cum[lo]), row);
+        lut[sid * kL + slot] = lut_entry((uint32_t)lo, (uint32_t)(fr[lo] + slot - cum[lo]), row);
     }
+}
+
+// Inclusive maximum over the lanes below and at each lane of a wave (all 64
+// active), the moves of wave_incl_scan.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
+    auto up = [](uint32_t v, uint32_t u) { return u > v ? u : v; };
+    int v = (int)x;
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));   // row_shr:1
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));   // row_shr:2
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));   // row_shr:4
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));   // row_shr:8
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = (int)up((uint32_t)v, (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return (uint32_t)v;
+}
+
+// The chunk decoder's LUT of one stream (lut_entry format, symbol field biased
+// by `bias`), built in LDS by one wave: every symbol writes one word (its cum,
+// index and frequency, ordered by cum) at its first slot, a running maximum
+// hands it to the slots up to the next symbol's, and each slot's entry follows
+// from it.  Lane l owns slots 16 l .. 16 l + 15.
+__device__ __forceinline__ void wave_lut(const lq_table* __restrict__ T, uint32_t row, uint32_t bias, uint32_t* lut,
+                                         int lane) {
+    // the first 256 entries are loaded with n_sym, not after it (entries past
+    // n_sym are allocated, and not used)
+    uint32_t e[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) e[u] = T->enc[64 * u + lane];
+    const int n = T->n_sym < kL ? T->n_sym : kL;
+    if (n <= 0) return;   // absent stream: no lane looks its row up
+    uint4* const mine = reinterpret_cast<uint4*>(lut + 16 * lane);
+#pragma unroll
+    for (int i = 0; i < 4; i++) mine[i] = make_uint4(0u, 0u, 0u, 0u);
+    WaveGroup::sync();
+    for (int j0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int j = j0 + 64 * u + lane;
+            const uint32_t f = enc_f(e[u]), cum = enc_c(e[u]);
+            if (j < n && f) lut[cum] = (cum << 21) | ((uint32_t)j << 11) | f;
+        }
+        j0 += 256;
+        if (j0 >= n) break;
+#pragma unroll
+        for (int u = 0; u < 4; u++) e[u] = j0 + 64 * u + lane < n ? T->enc[j0 + 64 * u + lane] : 0u;
+    }
+    WaveGroup::sync();
+    uint32_t v[16];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint4 q = mine[i];
+        v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+    }
+#pragma unroll
+    for (int i = 1; i < 16; i++) v[i] = v[i] > v[i - 1] ? v[i] : v[i - 1];
+    const uint32_t below = (uint32_t)__shfl_up((int)wave_incl_max(v[15]), 1, 64);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const uint32_t m = lane && below > v[i] ? below : v[i];
+        const uint32_t xp = (m & 0x7ffu) + (uint32_t)(16 * lane + i) - (m >> 21);
+        // as lut_entry; xp >= 1 in a valid table (a malformed one gives in-range garbage)
+        const int z = __clz((int)(xp | 1u)) - 21;
+        const uint32_t k = z > 0 ? (uint32_t)z : 0u;
+        v[i] = k | ((((m >> 11) & 1023u) + bias) << 6) | ((row * (uint32_t)kL + (((xp << k) - (uint32_t)kL) & (kL - 1u))) << 18);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) mine[i] = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
 
 // Whole-line chunk decoder.
 //
-// Workgroup: 64 consecutive blocks of one chunk, 16 lanes per block (one
-// wave holds 4 blocks): lane (block b, coset c, coordinate idx) decodes stream
+// A wave decodes 4 consecutive blocks of one chunk at a time (a task), 16
+// lanes per block: lane (block b, coset c, coordinate idx) decodes stream
 // c * 8 + idx of block b with LineLane, in phases of 8 steps.  Step j of a
 // phase stages the symbol index of coset-c vector `st + j` of the block at
 // rank slot (st + j) % 16 of the (block, coset) staging, so no lane walks the
@@ -1100,7 +1160,7 @@ __global__ __launch_bounds__(256) void k_chunk_lut(const lq_table* __restrict__ 
 // HEADS_ALIGNED: bph is a multiple of the block size, so a block lies in one
 // head.  DITHER: the chunk's dither (dither8, seed dseed[chunk]) is
 // subtracted from each lattice point before scaling.
-constexpr int kDecBlocks = 64;                  // blocks per decode workgroup
+constexpr int kDecBlocks = 64;                  // blocks in flight per decode workgroup (4 per wave)
 constexpr int kDecThreads = 16 * kDecBlocks;    // 1024
 constexpr int kDecStage = 16;                   // staged vectors per (block, coset)
 // Staging of (block b, coset c): group b * 2 + c, 16 slots of 8 u16, padded to
@@ -1117,8 +1177,8 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
         const uint32_t* __restrict__ words, const int64_t* __restrict__ chunk_base, const int64_t* __restrict__ stream_woff,
         const uint32_t* __restrict__ blk_off, const int64_t* __restrict__ stream_nbits,
         const uint16_t* __restrict__ blk_state, const uint8_t* __restrict__ coset_bits,
-        const lq_table* __restrict__ tables, const uint16_t* __restrict__ scale16, const uint32_t* __restrict__ lutg,
-        int64_t n_chunks, int64_t n_heads, int64_t bph, int64_t nblk, int64_t gpw, void* __restrict__ out,
+        const lq_table* __restrict__ tables, const uint16_t* __restrict__ scale16,
+        int64_t n_chunks, int64_t n_heads, int64_t bph, int64_t nblk, int64_t tpw, int wpc, void* __restrict__ out,
         const int64_t* __restrict__ dseed, const float* __restrict__ signs, int lpr, float rdiv,
         const int32_t* __restrict__ esc_k, const int64_t* __restrict__ fine_off, const uint32_t* __restrict__ fine) {
     __shared__ uint32_t lut[LQ_STREAMS * kL];                               // 64 KB
@@ -1128,27 +1188,32 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
     const int tid = threadIdx.x;
     const float rrcp = ROT ? 1.0f / rdiv : 1.0f;   // the rotation's RN(1 / sqrt(head_dim))
     const int64_t V = n_heads * bph;
-    const int64_t groups = (nblk + kDecBlocks - 1) / kDecBlocks;   // per chunk
-    const int64_t total = n_chunks * groups;
-    const int64_t first = (int64_t)blockIdx.x * gpw;
-    const int64_t last = first + gpw < total ? first + gpw : total;
-    const int wave = tid >> 6, lane = tid & 63;
-    int64_t lut_chunk = -1;
-    // The workgroup walks groups first .. last - 1 (64 blocks each); its LUTs
-    // are reloaded, between two barriers, only when the chunk changes.  Each
-    // wave stages its own 4 blocks' bitmaps and moves to its next blocks
-    // without waiting for the other waves.
-    for (int64_t gi = first; gi < last; gi++) {
-    const int64_t chunk = gi / groups;
-    const int64_t gbase = (gi % groups) * kDecBlocks;
-    if (chunk != lut_chunk) {
-        __syncthreads();   // every wave is done with the previous chunk's LUTs
-        const uint4* src = reinterpret_cast<const uint4*>(lutg + chunk * LQ_STREAMS * kL);
-        uint4* dst = reinterpret_cast<uint4*>(lut);
-        for (int i = tid; i < LQ_STREAMS * kL / 4; i += kDecThreads) dst[i] = src[i];
-        __syncthreads();
-        lut_chunk = chunk;
+    const int64_t per_chunk = (nblk + 3) / 4;   // tasks
+    const int64_t total = n_chunks * per_chunk;
+    // wpc > 0: wpc workgroups to a chunk, tpw tasks each; else tpw tasks each
+    // of the whole batch's
+    const int64_t wc = wpc > 0 ? (int64_t)blockIdx.x / wpc : 0;
+    const int64_t first = wc * per_chunk + ((int64_t)blockIdx.x - wc * wpc) * tpw;
+    const int64_t lim = wpc > 0 ? (wc + 1) * per_chunk : total;
+    const int64_t last = first + tpw < lim ? first + tpw : lim;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // The workgroup walks tasks first .. last - 1, chunk by chunk; wave w builds
+    // the LUT of the chunk's stream w, between two barriers, and takes the
+    // chunk's tasks w, w + 16, ..  Each wave stages its own 4 blocks' bitmaps
+    // and moves to its next task without waiting for the other waves.
+    for (int64_t t0 = first; t0 < last;) {
+    const int64_t chunk = t0 / per_chunk;
+    const int64_t tend = (chunk + 1) * per_chunk < last ? (chunk + 1) * per_chunk : last;
+    const bool lut_biased = chunk_biased(tables + chunk * LQ_STREAMS, lane);   // the LUTs' symbol fields
+    if (t0 != first) __syncthreads();   // every wave is done with the previous chunk's LUTs
+    {
+        const lq_table* T = tables + chunk * LQ_STREAMS + wave;
+        wave_lut(T, (uint32_t)wave, lut_biased ? (uint32_t)(T->lo + ((wave & 7) < 7 ? 512 : 256)) : 0u,
+                 lut + wave * kL, lane);
     }
+    __syncthreads();
+    for (int64_t task4 = t0 + wave; task4 < tend; task4 += kDecThreads / 64) {
+    const int64_t gbase = (task4 - chunk * per_chunk) * 4 - wave * 4;   // block b of the workgroup: gbase + b
     __builtin_amdgcn_wave_barrier();
     for (int i = lane; i < 4 * (kBlk / 32 + 1); i += 64) {
         const int bl = wave * 4 + i / (kBlk / 32 + 1), w = i % (kBlk / 32 + 1);
@@ -1186,7 +1251,6 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
 #pragma unroll
         for (int j = 0; j < 8; j++) esc = esc || ec.k[j] != 0;
     }
-    const bool lut_biased = chunk_biased(T);   // the LUT's symbol fields (k_chunk_lut decides the same way)
     const bool biased = !esc && lut_biased;
     CosetConsts cc0, cc1;   // per-coset alphabet lows, for chunks whose fields are not biased
     if (!biased) {
@@ -1229,17 +1293,21 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
     float pend[ROT ? 8 : 1];         // ROT: butterfly stages of a deferred first half-row (lanes 0..7)
     int st = 0;                      // vectors of my coset staged (symbols of my stream decoded)
     int fpos = 0, fr0 = 0, fr1 = 0;  // flushed block positions and flushed ranks per coset (block-uniform)
+    d.boundary(n > 0);
     while (fpos < valid) {
         __builtin_amdgcn_wave_barrier();
-        const bool more = st < n;
-        d.boundary(more);
-        if (more && st - (c ? fr1 : fr0) <= kDecStage - 8) {
+        if (st < n && st - (c ? fr1 : fr0) <= kDecStage - 8) {
             // st % 8 == 0 here, so the phase's slots do not wrap; a last phase
             // with fewer than 8 symbols stages garbage in slots of ranks >= n,
             // which hold no unflushed rank (st + 8 - flushed <= 16) and are never read
             d.phase(my_stg + (st & (kDecStage - 1)) * 8, lutb);
             st = n - st < kPhase ? n : st + kPhase;
         }
+        // The boundary comes between the steps and the flush: the wait for the
+        // top-up also waits for older stores, and here those are a phase old
+        // (before the steps it waited for the stores just issued: 131072 blocks
+        // 520 us, here 493).
+        d.boundary(st < n);
         __builtin_amdgcn_wave_barrier();
         const int st_o = dpp_ror8(st);
         const int s0 = c ? st_o : st, s1 = c ? st : st_o;
@@ -1369,6 +1437,8 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
         fpos += F;
     }
     }
+    }
+    t0 = tend;
     }
 }
 
@@ -1601,11 +1671,24 @@ static int chunk_decode_launch(const uint32_t* d_words, const int64_t* d_chunk_b
     if (d_esc_k && (!d_fine_off || !d_fine)) return LQ_ERR_ARG;
     const int64_t V = n_heads * bph;
     const int64_t nblk = (V + kBlk - 1) / kBlk;
-    hipLaunchKernelGGL(k_chunk_lut, dim3((unsigned)(n_chunks * LQ_STREAMS)), dim3(256), 0, s, d_tables, d_lut_work, 1);
-    const int64_t groups = n_chunks * ((nblk + kDecBlocks - 1) / kDecBlocks);
+    (void)d_lut_work;   // the decoder builds its LUTs in LDS
+    // One workgroup per CU, whose waves share its tasks: up to 1024 tasks (4096
+    // blocks) each has a SIMD to itself.  With 64 blocks per workgroup whatever
+    // the size, and the LUTs from a launch of their own, 512 blocks (a chunk of
+    // 2048 tokens) took 65.2 us, 8192 blocks 72.3 and 131072 blocks 525; now
+    // 39.4, 49.0 and 493.  Either every chunk is cut into equal
+    // parts (no workgroup crosses a chunk boundary), or the whole batch is cut
+    // into one part per CU, and a workgroup that crosses a boundary waits for
+    // its slowest wave there and builds the next chunk's LUTs, about what a
+    // round of 16 tasks costs: the equal parts unless they are 16 tasks longer.
+    const int64_t per_chunk = (nblk + 3) / 4, tasks = n_chunks * per_chunk;
     const int64_t cus = device_cus();
-    const int64_t gpw = (groups + cus - 1) / cus;   // groups per workgroup: one workgroup per CU
-    const dim3 grid((unsigned)((groups + gpw - 1) / gpw));
+    const int64_t parts = n_chunks < cus ? cus / n_chunks : 1;
+    const int64_t tpw_c = (per_chunk + parts - 1) / parts, tpw_b = (tasks + cus - 1) / cus;
+    const bool by_chunk = tpw_c <= tpw_b + 16;
+    const int64_t tpw = by_chunk ? tpw_c : tpw_b;
+    const int wpc = by_chunk ? (int)((per_chunk + tpw - 1) / tpw) : 0;
+    const dim3 grid((unsigned)(by_chunk ? n_chunks * wpc : (tasks + tpw - 1) / tpw));
     const bool aligned = bph % kBlk == 0;
     const int lpr = d_signs ? head_dim / 8 : 1;
     const float div = d_signs ? (float)sqrt((double)head_dim) : 1.0f;
@@ -1614,7 +1697,7 @@ static int chunk_decode_launch(const uint32_t* d_words, const int64_t* d_chunk_b
 #define LQ_DECODE_E(DT, AL, DI, RO, ES)                                                                           \
     hipLaunchKernelGGL((k_chunk_decode<DT, AL, DI, RO, ES>), grid, dim3(kDecThreads), 0, s, d_words, d_chunk_base,      \
                        d_stream_woff, d_blk_off, d_stream_nbits, d_blk_state, d_coset_bits, d_tables, d_scale16,       \
-                       d_lut_work, n_chunks, n_heads, bph, nblk, gpw, d_out, d_dither_seed, d_signs, lpr, div,         \
+                       n_chunks, n_heads, bph, nblk, tpw, wpc, d_out, d_dither_seed, d_signs, lpr, div,         \
                        d_esc_k, d_fine_off, d_fine)
 #define LQ_DECODE(DT, AL, DI, RO)                                                                                 \
     do {                                                                                                          \
@@ -1679,7 +1762,7 @@ int lq_chunk_decode_rht(const uint32_t* d_words, const int64_t* d_chunk_base, co
 
 int lq_chunk_luts(const lq_table* d_tables, int64_t n_chunks, uint32_t* d_lut, hipStream_t s) {
     if (n_chunks <= 0 || !d_tables || !d_lut) return LQ_ERR_ARG;
-    hipLaunchKernelGGL(k_chunk_lut, dim3((unsigned)(n_chunks * LQ_STREAMS)), dim3(256), 0, s, d_tables, d_lut, 0);
+    hipLaunchKernelGGL(k_chunk_lut, dim3((unsigned)(n_chunks * LQ_STREAMS)), dim3(256), 0, s, d_tables, d_lut);
     return launch_status();
 }
 

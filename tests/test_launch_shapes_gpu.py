@@ -1,0 +1,81 @@
+"""Batches at the edges of the launch rules: how the blocks of a batch are cut
+into workgroups (quantizer, decoder) and how a head's partial sums are added
+must not show in any output."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _x(C, H, T, hd, seed, dtype=torch.float16):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(C, 1, H, T, hd, generator=g)
+    x[..., :2] *= 6.0
+    return x.to(dtype).cuda()
+
+
+# blocks per chunk x chunks: a task is 4 blocks, a workgroup walks the tasks of
+# one part of a chunk, or (many or uneven chunks) crosses chunk boundaries
+@pytest.mark.parametrize("C,H,T,hd", [
+    (1, 1, 3, 8),          # less than one block
+    (1, 2, 260, 128),      # 17 blocks: a task of one block
+    (3, 8, 203, 128),      # a partial last block, three parts per chunk
+    (300, 1, 40, 64),      # more chunks than compute units
+    (100, 8, 260, 128),    # 17 tasks per chunk, two parts
+    (7, 8, 2100, 128),     # 132 tasks per chunk over 36 parts
+    (129, 2, 1024, 128),   # one part of 16 tasks per chunk
+])
+def test_decode_parts_gpu(C, H, T, hd):
+    """Every chunk decoded in the batch equals the chunk decoded alone, and the
+    oracle's rows at both ends of the batch."""
+    from latticequant_amd import codec
+    x = _x(C, H, T, hd, C + T)
+    enc, _ = codec.encode_batch(x, 4)
+    out = codec.decode_batch(enc)
+    for c in sorted({0, 1 % C, C // 2, C - 1}):
+        assert torch.equal(out[c], codec.decode_batch(enc.select(c))[0])
+    for c in {0, C - 1}:
+        ch = O.compress_chunk(x[c].cpu().numpy(), 4, scales_f32=enc.scale32.view(C, -1)[c].cpu().numpy())
+        base, nw = int(enc.chunk_base[c]), int(enc.chunk_words[c])
+        assert np.array_equal(enc.words[base:base + nw].cpu().numpy().view(np.uint32), ch.bitstream)
+        assert np.array_equal(out[c].cpu().numpy(), O.decompress_chunk(ch))
+
+
+# heads x vectors per head: 1, 8, 512, 513 .. partial sums per head (one per 512
+# vectors, about 4096 in all)
+@pytest.mark.parametrize("C,H,T,dtype", [
+    (1, 3, 33, torch.float16), (1, 8, 256, torch.bfloat16), (1, 4, 16400, torch.float16), (1, 1, 33000, torch.float16),
+])
+def test_scale_parts_gpu(C, H, T, dtype):
+    """sigma^2 against 64-bit sums: the partial sums are 64-bit, so one fp32
+    rounding (2^-24) is all that may separate them, twice that being allowed
+    for the sum's own rounding falling on the other side."""
+    from latticequant_amd import codec
+    x = _x(C, H, T, 128, T, dtype)
+    _, _, _, s2 = codec.quantize_batch(x, 4, with_sigma2=True)
+    want = x.double().square().mean((-1, -2)).reshape(-1)
+    assert float(((s2.double() - want) / want).abs().max()) <= 2.0 ** -23
+
+
+# blocks in the launch: 1, 2 .. 8 blocks per quantizer workgroup, and counts one
+# off a multiple
+@pytest.mark.parametrize("C,H,T", [(1, 1, 32), (2, 1, 1025), (1, 8, 4100), (2, 8, 4096), (9, 8, 1500), (20, 8, 3300)])
+@pytest.mark.parametrize("deq", [False, True])
+def test_quantizer_workgroups_gpu(C, H, T, deq):
+    """Histograms, counts and symbols do not depend on the blocks per
+    workgroup: the batch equals its chunks encoded one at a time (other launch
+    shapes), word for word."""
+    from latticequant_amd import codec
+    x = _x(C, H, T, 128, 7 * T)
+    enc, d = codec.encode_batch(x, 4, deq_out=deq)
+    for c in sorted({0, C - 1}):
+        one, d1 = codec.encode_batch(x[c:c + 1], 4, deq_out=deq)
+        base, nw = int(enc.chunk_base[c]), int(enc.chunk_words[c])
+        assert nw == int(one.chunk_words[0])
+        assert torch.equal(enc.words[base:base + nw], one.words[:nw])
+        assert torch.equal(enc.coset_bits[c], one.coset_bits[0]) and torch.equal(enc.blk_n1[c], one.blk_n1[0])
+        if deq:
+            assert torch.equal(d[c], d1[0])

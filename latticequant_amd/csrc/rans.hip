@@ -59,11 +59,35 @@ struct WaveGroup {
     static constexpr bool kWave = true;
 };
 
+// Inclusive scan over the 64 lanes of a wave in DPP moves: Hillis-Steele
+// within each 16-lane row (row_shr 1, 2, 4, 8; lanes shifted in from outside
+// the row read 0), then row 0's last lane added to row 1 and row 2's to row 3
+// (row_bcast:15), then lane 31 added to rows 2 and 3 (row_bcast:31).
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+    int v = (int)x;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, rows 2 and 3
+    return (uint32_t)v;
+}
+
+// Sum of v over a wave (64 active lanes), in every lane.
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(v), 63);
+}
+
 // Block-wide sum of v (G::size() multiple of 64, <= 1024).
 template <typename G>
 __device__ int64_t block_sum(int64_t v) {
+    if constexpr (G::kWave) {   // |v| < 2^42 (counts of one chunk): two halves of 21 bits, sums below 2^31
+        const uint64_t lo = wave_sum((uint32_t)v & 0x1fffffu);
+        const int64_t hi = (int64_t)(int32_t)wave_sum((uint32_t)(int32_t)(v >> 21));
+        return hi * (int64_t)(1 << 21) + (int64_t)lo;
+    }
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if constexpr (G::kWave) return v;
     __shared__ int64_t part[16];
     G::sync();
     if ((G::tid() & 63) == 0) part[G::tid() >> 6] = v;
@@ -73,7 +97,7 @@ __device__ int64_t block_sum(int64_t v) {
     return s;
 }
 
-// Block-wide maximum of v (G::size() multiple of 64, <= 1024).
+// Group-wide maximum of v >= 0.
 template <typename G>
 __device__ int64_t block_max(int64_t v) {
     for (int o = 32; o > 0; o >>= 1) {
@@ -138,6 +162,115 @@ __device__ bool adjust_pass_sorted(int n, const int32_t* freqs, int diff, int fu
     return block_sum<G>(matters) != 0;
 }
 
+// np_net_sort's network (n <= 256 keys) with the pairs in a wave's registers
+// instead of LDS: element e sits in slot e / 64 of lane e % 64, as
+// (key << 8) | index with keys below 2^23 (the padding's is larger), and every
+// stage pairs e with e ^ m, so one lane exchange per slot and stage replaces
+// the stage's LDS reads, writes and waits.  v: -key (counts or frequencies),
+// vmax >= every v.  Sets inset[] of the first rem sorted entries to 1, of the
+// others to 0.
+__device__ void net_sort_inset(const uint32_t vin[4], uint32_t vmax, int n, int rem, int8_t* inset) {
+    const int lane = WaveGroup::tid();
+    uint32_t v[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int e = 64 * s + lane;
+        v[s] = (e < n ? vmax - vin[s] : 0xffffffu) << 8 | (uint32_t)e;
+    }
+    auto stage = [&](int m) {   // m < 64, or 64, 127, 255: slot partner s, s ^ 1, s ^ 1, s ^ 3
+        const int src = (lane ^ (m & 63)) << 2;
+        auto cx = [&](uint32_t own, uint32_t other, bool lower) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)other);
+            const bool take = lower ? (own >> 8) > (o >> 8) : (o >> 8) > (own >> 8);   // equal keys stay
+            return take ? o : own;
+        };
+        uint32_t r[4];
+        if (m < 64) {
+            const bool lower = (lane & (1 << (31 - __builtin_clz((unsigned)m)))) == 0;
+#pragma unroll
+            for (int s = 0; s < 4; s++) r[s] = cx(v[s], v[s], lower);
+        } else if (m < 128) {
+#pragma unroll
+            for (int s = 0; s < 4; s++) r[s] = cx(v[s], v[s ^ 1], (s & 1) == 0);
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) r[s] = cx(v[s], v[s ^ 3], (s & 2) == 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) v[s] = r[s];
+    };
+    int nv = 1;
+    while (nv * 8 < n) nv *= 2;
+    stage(1); stage(3); stage(1); stage(7); stage(2); stage(1);
+    for (int per = 2; per <= nv; per *= 2) {
+        stage(8 * per - 1);
+        for (int num = per / 2; num >= 2; num /= 2) stage(4 * num);
+        stage(4); stage(2); stage(1);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        if (64 * s + lane < n) inset[v[s] & 255u] = 64 * s + lane < rem ? 1 : 0;
+}
+
+// adjust_pass for one wave and at most 320 entries: the members of the set
+// that do not depend on the tie order, from the rem-th smallest key kstar (all
+// keys below it are in, all above out, those equal to it straddle the cut
+// unless they end exactly there), found by a search over the key's bits with
+// the keys in registers and a vote per entry and step.  Counting every entry's
+// rank instead (n^2 LDS reads) took most of the table kernel: on alphabets of
+// about 180 symbols it fell from 29.8 to 21.7 us with this search, and to 17.0
+// with the network in registers (launch included).  If a different subset of the straddling group would
+// change a frequency and the alphabet is at most 256 symbols with keys below
+// 2^23, numpy's network order settles it here (net_sort_inset); returns (wave
+// uniform) whether the caller has to.
+__device__ bool adjust_pass_select(int n, const int32_t* freqs, int diff, int full, int rem, const int64_t* kk,
+                                   int8_t* inset) {
+    constexpr int kPer = 5;
+    const int lane = WaveGroup::tid();
+    uint32_t v[kPer];   // -key: counts or frequencies, below 2^32
+    uint32_t any = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const int i = 64 * u + lane;
+        v[u] = i < n ? (uint32_t)(-kk[i]) : 0u;
+        any |= v[u];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) any |= (uint32_t)__shfl_xor((int)any, o, 64);
+    any = (uint32_t)__builtin_amdgcn_readfirstlane((int)any);
+    auto at_least = [&](uint32_t t) {   // entries with v >= t
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; u++) c += __builtin_popcountll(__ballot(64 * u + lane < n && v[u] >= t));
+        return c;
+    };
+    // the largest t with more than rem entries >= t: position rem of the
+    // descending order holds t (rem < n, so t = 0 has n > rem entries)
+    uint32_t t = 0;
+    for (int b = 31 - __builtin_clz(any | 1u); b >= 0; b--) {
+        const uint32_t c = t | (1u << b);
+        if (at_least(c) > rem) t = c;
+    }
+    // keys above t: all in.  Equal to t: in the straddling group, or (none of
+    // them before the cut) out
+    const int above = t == 0xffffffffu ? 0 : at_least(t + 1u);
+    const bool straddles = above < rem;
+    bool mt = false;
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const int i = 64 * u + lane;
+        if (i < n) {
+            inset[i] = v[u] > t ? 1 : (v[u] == t && straddles ? 2 : 0);
+            mt = mt || (v[u] == t && straddles && (diff > 0 || freqs[i] - full > 1));
+        }
+    }
+    if (!__any(mt)) return false;
+    if (n > 256 || any >= 1u << 23) return true;
+    WaveGroup::sync();
+    net_sort_inset(v, any, n, rem, inset);
+    return false;
+}
+
 // One pass of the build_rans_table adjustment loop (core/gpu_ans.py:73-84)
 // with m = |diff|: j = 0 .. m-1 visits order[j % n], i.e. every entry
 // `full` = m / n times plus the first rem = m % n entries of the argsort order
@@ -153,7 +286,9 @@ __device__ void adjust_pass(const int64_t* counts, int n, int32_t* freqs, int di
     for (int i = G::tid(); i < n; i += G::size()) kk[i] = diff > 0 ? -counts[i] : -(int64_t)freqs[i];
     G::sync();
     bool matters;
-    if (n > 256 && sk) {
+    if constexpr (G::kWave) {
+        matters = adjust_pass_select(n, freqs, diff, full, rem, kk, inset);
+    } else if (n > 256 && sk) {
         matters = adjust_pass_sorted<G>(n, freqs, diff, full, rem, kk, a, inset, sk);
     } else {
         int mt = 0;
@@ -249,12 +384,12 @@ __device__ void normalise(const int64_t* counts, int n, int32_t* freqs, int16_t*
 // Inclusive scan of v over the block (G::size() <= 1024, multiple of 64).
 template <typename G>
 __device__ int block_incl_scan(int v) {
+    if constexpr (G::kWave) return (int)wave_incl_scan((uint32_t)v);
     const int lane = G::tid() & 63, w = G::tid() >> 6;
     for (int o = 1; o < 64; o <<= 1) {
         int t = __shfl_up(v, o, 64);
         if (lane >= o) v += t;
     }
-    if constexpr (G::kWave) return v;
     __shared__ int wsum[16];
     G::sync();
     if (lane == 63) wsum[w] = v;
@@ -273,7 +408,7 @@ __device__ void exclusive_scan_array(const int32_t* in, int n, int32_t* out) {
             const int v = i < n ? in[i] : 0;
             const int incl = block_incl_scan<G>(v);
             if (i < n) out[i] = carry + incl - v;
-            carry += __shfl(incl, 63, 64);
+            carry += __builtin_amdgcn_readlane(incl, 63);
         }
         if (G::tid() == 0) out[n] = carry;
         G::sync();
@@ -395,33 +530,40 @@ __global__ __launch_bounds__(64 * kTabWaves) void k_chunk_tables_wave(const uint
     lq_table* T = tables + sid;
     const uint32_t* hs = hist + sid * 256;
     uint32_t hv[4];
-    int mn = 256, mx = -1;
+    int mn, mx;
     uint32_t tl = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int b = lane + 64 * j;
         hv[j] = hs[b];
-        if (hv[j]) {
-            mn = b < mn ? b : mn;
-            mx = b > mx ? b : mx;
-            tl += hv[j];
+        tl += hv[j];
+    }
+    // a bin with a count, in each quarter of the bins: first and last by ballot
+    mn = 256;
+    mx = -1;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint64_t m = __ballot(hv[j] != 0);
+        if (m) {
+            mx = 64 * j + 63 - __builtin_clzll(m);
+            if (mn == 256) mn = 64 * j + __builtin_ctzll(m);
         }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int a = __shfl_xor(mn, o, 64), c = __shfl_xor(mx, o, 64);
-        mn = a < mn ? a : mn;
-        mx = c > mx ? c : mx;
-        tl += __shfl_xor(tl, o, 64);
-    }
+    tl = wave_sum(tl);
     if (mx < 0) {   // absent stream (empty coset)
         if (lane == 0) { T->lo = 0; T->n_sym = 0; T->n_symbols = 0; T->status = 0; }
         return;
     }
     const int lo = mn - 128 - 2, n = mx - mn + 5;
-    for (int i = lane; i < n; i += 64) {
-        const int b = lo + i + 128;
-        counts[w][i] = (b >= 0 && b < 256) ? (int64_t)hs[b] : 0;
+    // bin b is alphabet entry b - 128 - lo; the guard entries have no counts
+    if (lane < 2) {
+        counts[w][lane] = 0;
+        counts[w][n - 1 - lane] = 0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = lane + 64 * j - 128 - lo;
+        if (i >= 2 && i < n - 2) counts[w][i] = (int64_t)hv[j];
     }
     if (lane == 0) s_st[w] = 0;
     WaveGroup::sync();
@@ -735,21 +877,6 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
 // offsets (n_words + 1 words per present stream) and total.  Replaces
 // k_chunk_scan + k_chunk_offsets for such batches.
 constexpr int kScanRounds = 32;   // rounds of 64 blocks whose loads are in flight together
-
-// Inclusive scan over the 64 lanes of a wave in DPP moves: Hillis-Steele
-// within each 16-lane row (row_shr 1, 2, 4, 8; lanes shifted in from outside
-// the row read 0), then row 0's last lane added to row 1 and row 2's to row 3
-// (row_bcast:15), then lane 31 added to rows 2 and 3 (row_bcast:31).
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-    int v = (int)x;
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, rows 2 and 3
-    return (uint32_t)v;
-}
 
 __global__ __launch_bounds__(1024) void k_chunk_scan_offsets(const uint32_t* __restrict__ blk_bits,
                                                              const uint16_t* __restrict__ blk_state,

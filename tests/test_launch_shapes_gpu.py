@@ -79,3 +79,46 @@ def test_quantizer_workgroups_gpu(C, H, T, deq):
         assert torch.equal(enc.coset_bits[c], one.coset_bits[0]) and torch.equal(enc.blk_n1[c], one.blk_n1[0])
         if deq:
             assert torch.equal(d[c], d1[0])
+
+
+def _tie_heavy(rng, n, kind):
+    if kind == 0:
+        return rng.integers(1, 4, n)                                  # three counts: large tie groups
+    if kind == 1:
+        return (1 + 2000 * np.exp(-0.5 * ((np.arange(n) - n / 2) / (0.1 * n + 1)) ** 2)).astype(np.int64)
+    if kind == 2:
+        return np.where(rng.random(n) < 0.02, 100000, rng.integers(1, 3, n))   # an excess: the decrement branch
+    return rng.integers(1, 4, n) * (1 << 22) + (rng.random(n) < 0.5)  # keys beyond 2^23
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+def test_int8_tables_tie_order_gpu(kind):
+    """Every table of the int8 path against the oracle (numpy's argsort order
+    on ties) at alphabets of 5 .. 260 symbols, around the network's sizes (8,
+    16, .. 256) and the wave's quarters."""
+    from latticequant_amd import codec, _lib as L
+    rng = np.random.default_rng(kind)
+    spans = [1, 2, 3, 4, 5, 11, 12, 13, 27, 28, 59, 60, 61, 100, 123, 124, 125, 150, 187, 188, 200, 220, 251, 252, 253,
+             255, 256, 64, 65, 128, 192, 230]
+    hist = np.zeros((len(spans), 256), np.int64)
+    for i, m in enumerate(spans):
+        b0 = int(rng.integers(0, 256 - m + 1))
+        hist[i, b0:b0 + m] = _tie_heavy(rng, m, kind)
+    C = len(spans) // 16
+    d = torch.from_numpy(hist.astype(np.uint32).view(np.int32)).cuda()
+    tables = torch.zeros(C * 16 * L.TABLE_BYTES, dtype=torch.uint8, device="cuda")
+    st = torch.zeros(C, dtype=torch.int32, device="cuda")
+    L.check(L.lib().lq_chunk_tables(d.data_ptr(), C, tables.data_ptr(), st.data_ptr(), L.stream_ptr(d.device)),
+            "lq_chunk_tables")
+    t = tables.view(torch.int32).view(-1, L.TABLE_BYTES // 4).cpu().numpy()
+    assert not st.any()
+    for i, m in enumerate(spans):
+        b0 = int(np.flatnonzero(hist[i])[0])
+        lo, n = b0 - 128 - 2, m + 4
+        assert (int(t[i, 0]), int(t[i, 1])) == (lo, n)
+        counts = np.zeros(n, np.int64)
+        counts[2:-2] = hist[i, b0:b0 + m]
+        want = O.build_rans_table(counts, list(range(lo, lo + n))).freqs
+        got = t[i, 4:4 + n].view(np.uint32)
+        assert np.array_equal(got & 0x7ff, want), (kind, m)
+        assert np.array_equal((got >> 11) & 0x3ff, (np.cumsum(want) - want) & 0x3ff)

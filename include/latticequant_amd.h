@@ -327,7 +327,8 @@ int lq_build_tables(const int64_t *d_counts, const int64_t *d_count_off, const i
                     int32_t n_tables, int32_t *d_freqs, int32_t *d_cum, int32_t *d_lookup, int32_t *d_status,
                     hipStream_t s);
 
-/* Serial rANS encode of n_streams streams of symbol indices (one lane each).
+/* rANS encode of n_streams streams of symbol indices (one workgroup each; the
+ * tables are lq_build_tables': frequencies in [1, L] summing to L).
  * Stream t: d_idx + d_sym_off[t], length d_n[t], table freqs/cum at
  * d_tab_off[t].  Words go to d_words + d_word_off[t] (capacity
  * 10*n/32 + 2 words each); state and n_bits per stream.
@@ -337,7 +338,7 @@ int lq_rans_encode_streams(const int32_t *d_idx, const int64_t *d_sym_off, const
                            int32_t n_streams, uint32_t *d_scratch, uint32_t *d_words, const int64_t *d_word_off,
                            int64_t *d_state, int64_t *d_nbits, hipStream_t s);
 
-/* One lane per stream decode with the reference's bit-position guard; writes
+/* Decode (one workgroup per stream) with the reference's bit-position guard; writes
  * int64 symbol values.  Replaces _rans_decode_kernel (core/gpu_ans.py:175-235). */
 int lq_rans_decode_streams(const int32_t *d_bits, const int32_t *d_bit_off, const int32_t *d_nbits,
                            const int32_t *d_init, const int32_t *d_ndec, const int32_t *d_lookup,

@@ -105,7 +105,7 @@ def _contiguous(alphabet) -> bool:
 
 
 def _encode_many(symbol_lists, tables, dev):
-    """Encode several streams in one launch (one lane per stream)."""
+    """Encode several streams in one launch (one workgroup per stream)."""
     lib = L_.lib()
     s = L_.stream_ptr(dev)
     n_s = len(symbol_lists)
@@ -260,7 +260,7 @@ def prepare_gpu_decode(streams: List[RANSStream], device: str = "cuda") -> Prepa
 
 
 def run_gpu_decode_kernel(prep: PreparedGPUDecode):
-    """Decode every stream, one lane each (core/gpu_ans.py:345-354)."""
+    """Decode every stream, one workgroup each (core/gpu_ans.py:345-354)."""
     dev = prep.d_out.device
     with torch.cuda.device(dev):
         prep.d_out.zero_()

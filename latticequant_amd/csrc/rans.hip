@@ -1610,16 +1610,32 @@ __global__ __launch_bounds__(256) void k_build_tables(const int64_t* __restrict_
 
 // ------------------------------------------------------ generic streams --
 
-// Serial encode of one stream per lane, then the bits are laid out in the
-// reference's word order (n_words + 1 words, last zero).
-__global__ void k_encode_streams(const int32_t* __restrict__ idx, const int64_t* __restrict__ sym_off,
-                                 const int64_t* __restrict__ nsym, const int32_t* __restrict__ freqs,
-                                 const int32_t* __restrict__ cum, const int64_t* __restrict__ tab_off, int32_t n_streams,
-                                 uint32_t* __restrict__ scratch, uint32_t* __restrict__ words,
-                                 const int64_t* __restrict__ word_off, int64_t* __restrict__ state_out,
-                                 int64_t* __restrict__ nbits_out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_streams) return;
+// Encode of arbitrary streams, one workgroup per stream.  The stream is cut
+// into segments of kSegSyms symbols, one lane each; a lane finds the exact
+// state entering its segment as the chunk encoder does (an interval of states,
+// run over a growing window of the symbols behind the segment until it is one
+// state or the window reaches the stream's end, where the state is L), encodes
+// the segment into its LDS column, and the segments' bits are joined by a scan
+// of their counts.  Encoding runs from the stream's end, so a segment's place
+// is known from the end: the joined bits are right-aligned in the stream's
+// scratch words, and a last pass shifts them to the reference's layout (n_words
+// + 1 words, last zero).  Streams longer than kSegLanes segments take that
+// many at a time, from the end.  One lane per stream, symbol by symbol, took
+// 9278 us for 16 streams of 32768 symbols; this takes 52 us.
+// The tables are build_rans_table's (frequencies in [1, L], summing to L).
+constexpr int kSegSyms = 64;
+constexpr int kSegWords = 10 * kSegSyms / 32;   // at most 10 bits per symbol
+constexpr int kSegLanes = 1024;
+
+__global__ __launch_bounds__(kSegLanes) void k_encode_streams(
+        const int32_t* __restrict__ idx, const int64_t* __restrict__ sym_off, const int64_t* __restrict__ nsym,
+        const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum, const int64_t* __restrict__ tab_off,
+        uint32_t* __restrict__ scratch, uint32_t* __restrict__ words, const int64_t* __restrict__ word_off,
+        int64_t* __restrict__ state_out, int64_t* __restrict__ nbits_out) {
+    __shared__ uint32_t seg[kSegWords][kSegLanes];   // 80 KB: a lane's bits, right-aligned in its column
+    __shared__ uint32_t wsum[kSegLanes / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t t = blockIdx.x;
     const int64_t n = nsym[t];
     const int32_t* id = idx + sym_off[t];
     const int32_t* F = freqs + tab_off[t];
@@ -1627,51 +1643,153 @@ __global__ void k_encode_streams(const int32_t* __restrict__ idx, const int64_t*
     const int64_t cap = (10 * n + 31) / 32 + 2;
     uint32_t* scr = scratch + word_off[t];
     uint32_t* out = words + word_off[t];
-    int64_t wpos = cap - 1;
-    uint64_t acc = 0;
-    uint32_t nacc = 0;
-    int64_t total = 0;
-    uint32_t x = kL;
-    for (int64_t j = n - 1; j >= 0; j--) {
-        uint32_t f = (uint32_t)F[id[j]], cf = (uint32_t)C[id[j]];
-        uint32_t e = enc_pack(f, cf);
-        uint32_t k, xin = x;
-        x = enc_step(x, e, &k);
-        uint64_t r = ((uint64_t)__builtin_bitreverse32(xin) << k) >> 32;
-        acc = (acc << k) | r;
-        nacc += k;
-        total += k;
-        if (nacc >= 32) { nacc -= 32; scr[wpos--] = (uint32_t)(acc >> nacc); }
+    for (int64_t w = tid; w < cap; w += kSegLanes) scr[w] = 0u;
+    const int64_t nseg = (n + kSegSyms - 1) / kSegSyms;
+    int64_t done = 0;   // bits of the segments behind the current ones
+    // f(entry, in) for symbols j1 - 1 .. j0, 16 at a time with their loads together
+    auto rev = [&](int64_t j0, int64_t j1, auto&& f) {
+        for (int64_t j = j1; j > j0; j -= 16) {
+            uint32_t e[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                const int64_t p = j - 1 - u > j0 ? j - 1 - u : j0;
+                e[u] = (uint32_t)id[p];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; u++) e[u] = encx_of(enc_pack((uint32_t)F[e[u]], (uint32_t)C[e[u]]));
+#pragma unroll
+            for (int u = 0; u < 16; u++) f(e[u], j - 1 - u >= j0);
+        }
+    };
+    for (int64_t s1 = nseg; s1 > 0; s1 -= kSegLanes) {
+        const int64_t s0 = s1 > kSegLanes ? s1 - kSegLanes : 0;
+        const int64_t g = s0 + tid;
+        uint32_t total = 0;
+        int capw = 0;
+        if (g < s1) {
+            const int64_t b = g * kSegSyms, e = b + kSegSyms < n ? b + kSegSyms : n;
+            uint32_t x = kL;
+            for (int64_t window = 16; e < n; window *= 4) {
+                const int64_t top = e + window < n ? e + window : n;
+                uint32_t lo = kL, hi = top == n ? (uint32_t)kL : 2u * kL - 1u;
+                rev(e, top, [&](uint32_t en, bool in) {
+                    uint32_t l2 = lo, h2 = hi;
+                    hull_step(l2, h2, en);
+                    lo = in ? l2 : lo;
+                    hi = in ? h2 : hi;
+                });
+                x = lo;
+                if (lo == hi) break;   // always so once the window ends at n
+            }
+            capw = (int)((10 * (e - b) + 31) / 32);
+            int wpos = capw - 1;
+            uint64_t acc = 0;
+            uint32_t nacc = 0;
+            rev(b, e, [&](uint32_t en, bool in) {
+                uint32_t k;
+                const uint32_t xin = x, xn = encx_step(xin, en, &k);
+                if (in) {
+                    acc = (acc << k) | (((uint64_t)__builtin_bitreverse32(xin) << k) >> 32);
+                    nacc += k;
+                    total += k;
+                    x = xn;
+                    if (nacc >= 32) {
+                        nacc -= 32;
+                        seg[wpos][tid] = (uint32_t)(acc >> nacc);
+                        wpos = wpos > 0 ? wpos - 1 : 0;   // never below 0 with tables of the kind above
+                    }
+                }
+            });
+            if (nacc) seg[wpos][tid] = (uint32_t)(acc << (32 - nacc));
+            total = total < 32u * (uint32_t)capw ? total : 32u * (uint32_t)capw;
+            if (g == 0) state_out[t] = x;
+        }
+        // bits of the segments behind mine in this tile
+        const uint32_t incl = wave_incl_scan(total);
+        // the cleared words reach the L2, where the atomics below work; wsum of
+        // the previous tile is read
+        if (s1 == nseg) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __syncthreads();
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        uint32_t upto = 0, tile = 0;
+#pragma unroll
+        for (int w = 0; w < kSegLanes / 64; w++) {
+            const uint32_t v = wsum[w];
+            upto += w < wave ? v : 0u;
+            tile += v;
+        }
+        const int64_t behind = done + (int64_t)(tile - (upto + incl));
+        // my bits go to bits D .. D + total - 1 of the scratch words; words shared
+        // with other segments are merged with atomics
+        const int64_t D = cap * 32 - behind - total;
+        const int sp0 = capw * 32 - (int)total;   // first bit in my column
+        for (int64_t w = D >> 5; total && w <= (D + total - 1) >> 5; w++) {
+            const int64_t lo = w * 32 > D ? w * 32 : D, hi = w * 32 + 32 < D + total ? w * 32 + 32 : D + total;
+            const int sp = sp0 + (int)(lo - D), take = (int)(hi - lo), wi = sp >> 5, sh = sp & 31;
+            uint64_t v = seg[wi][tid];
+            if (sh + take > 32) v |= (uint64_t)seg[wi + 1][tid] << 32;
+            const uint32_t bits = (uint32_t)(v >> sh);
+            if (take == 32) scr[w] = bits;
+            else atomicOr(scr + w, (bits & ((1u << take) - 1u)) << (int)(lo - w * 32));
+        }
+        done += tile;
     }
-    if (nacc) scr[wpos] = (uint32_t)(acc << (32 - nacc));
-    const int64_t nw = (total + 31) / 32;
-    const int64_t base = cap * 32 - total;   // scratch bit position of stream bit 0
-    for (int64_t w = 0; w < nw; w++) {
-        int64_t sp = base + 32 * w;
-        int64_t wi = sp >> 5;
-        int sh = (int)(sp & 31);
-        int take = (int)(total - 32 * w < 32 ? total - 32 * w : 32);
-        uint64_t v = scr[wi];
-        if (sh + take > 32) v |= (uint64_t)scr[wi + 1] << 32;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    const int64_t nw = (done + 31) / 32, base = cap * 32 - done;   // scratch bit of the stream's first
+    for (int64_t w = tid; w < nw; w += kSegLanes) {
+        const int64_t sp = base + 32 * w, wi = sp >> 5;
+        const int sh = (int)(sp & 31), take = (int)(done - 32 * w < 32 ? done - 32 * w : 32);
+        uint64_t v = __hip_atomic_load(scr + wi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sh + take > 32) v |= (uint64_t)__hip_atomic_load(scr + wi + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) << 32;
         v >>= sh;
         out[w] = take == 32 ? (uint32_t)v : (uint32_t)v & ((1u << take) - 1u);
     }
-    out[nw] = 0u;
-    state_out[t] = x;
-    nbits_out[t] = total;
+    if (tid == 0) {
+        out[nw] = 0u;
+        nbits_out[t] = done;
+        if (n == 0) state_out[t] = kL;
+    }
 }
 
-// _rans_decode_kernel semantics (core/gpu_ans.py:175-235): one stream per lane,
-// renormalisation reads min(needed, n_bits - bit_pos) bits.
-__global__ void k_decode_streams(const int32_t* __restrict__ bits, const int32_t* __restrict__ bit_off,
-                                 const int32_t* __restrict__ nbits, const int32_t* __restrict__ init,
-                                 const int32_t* __restrict__ ndec, const int32_t* __restrict__ lookup,
-                                 const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum,
-                                 const int32_t* __restrict__ alphabet, const int32_t* __restrict__ tid_,
-                                 int32_t max_sym, const int32_t* __restrict__ out_off, int32_t n_streams,
-                                 int64_t* __restrict__ out) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_streams) return;
+// _rans_decode_kernel semantics (core/gpu_ans.py:175-235), one workgroup per
+// stream: renormalisation reads min(needed, n_bits - bit_pos) bits.
+//
+// A stream is one serial chain (every step needs the state before it), so the
+// kernel is arranged around that chain's latency: tables in LDS, bits in a
+// register buffer refilled from words the wave holds one per lane, the chain
+// computed by all lanes alike, and everything else (symbol values, stores)
+// done by 64 lanes at once from the trace of 64 steps.  A step takes one LDS
+// read and a few shifts.  PAIR: the table is indexed by the slot and the next
+// kAhead stream bits, and a step covers two symbols whenever the first one's
+// renormalisation needs no more than those bits; it fills a CU's LDS, so it is
+// taken for up to two streams per CU, and the one-symbol table (many
+// workgroups per CU) beyond.  One lane per stream with the tables in global
+// memory, bit by bit, took 30771 us for 16 streams of 32768 symbols; this takes
+// 1436 us.
+// The chain's tables hold for states in [L, 2L) and tables whose steps stay
+// there; anything else, and the stream's last bits, take plain_step.
+constexpr int kAhead = 5;
+constexpr int kWordRing = 256;   // stream words in LDS
+
+template <bool PAIR>
+__global__ __launch_bounds__(256) void k_decode_streams(
+        const int32_t* __restrict__ bits, const int32_t* __restrict__ bit_off, const int32_t* __restrict__ nbits,
+        const int32_t* __restrict__ init, const int32_t* __restrict__ ndec, const int32_t* __restrict__ lookup,
+        const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum, const int32_t* __restrict__ alphabet,
+        const int32_t* __restrict__ tid_, int32_t max_sym, const int32_t* __restrict__ out_off,
+        int64_t* __restrict__ out) {
+    // one[slot]: k | symbol index << 6 | next slot before the k bits << 16
+    __shared__ uint32_t one[kL];
+    // two[slot << kAhead | next bits]: k1 | (64 - kAhead - k2) << 6 | next slot << 22, the
+    // pair's first shift and second read; k1 = 0 and the first symbol's own k and slot
+    // where it needs more than kAhead bits
+    __shared__ uint32_t two[PAIR ? kL << kAhead : 1];
+    __shared__ uint32_t ring[kWordRing];
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int t = blockIdx.x;
     const uint32_t* wb = reinterpret_cast<const uint32_t*>(bits);
     const int64_t boff = bit_off[t];
     const int64_t nb = nbits[t];
@@ -1682,18 +1800,160 @@ __global__ void k_decode_streams(const int32_t* __restrict__ bits, const int32_t
     const int32_t* C = cum + (int64_t)tb * max_sym;
     const int32_t* A = alphabet + (int64_t)tb * max_sym;
     int64_t* o = out + out_off[t];
+    if (n <= 0) return;   // uniform
     uint32_t x = (uint32_t)init[t];
-    int64_t pos = 0;
-    for (int i = 0; i < n; i++) {
-        uint32_t slot = x & (kL - 1);
-        int si = LU[slot];
-        o[i] = A[si];
+    if (tid == 0) s_bad = x < (uint32_t)kL || x >= 2u * kL ? 1 : 0;
+    __syncthreads();
+    for (int slot = tid; slot < kL; slot += 256) {
+        const int si = LU[slot];
+        int64_t xp = 0;
+        if (si >= 0 && si < max_sym && si < kL) xp = (int64_t)F[si] + slot - C[si];
+        if (xp < 1 || xp >= 2 * kL) {
+            s_bad = 1;
+            one[slot] = 0u;
+        } else {
+            const uint32_t k = xp >= kL ? 0u : (uint32_t)(__clz((int)xp) - 21);
+            one[slot] = k | ((uint32_t)si << 6) | ((((uint32_t)xp << k) - (uint32_t)kL) << 16);
+        }
+    }
+    __syncthreads();
+    if constexpr (PAIR) {
+        for (int i = tid; i < kL << kAhead; i += 256) {
+            uint32_t e = one[i >> kAhead], ks = 0u;
+            const uint32_t k1 = e & 63u;
+            if (k1 <= (uint32_t)kAhead) {
+                ks = k1;
+                e = one[(e >> 16) + ((uint32_t)(i & ((1 << kAhead) - 1)) >> (kAhead - k1))];
+            }
+            two[i] = ks | ((uint32_t)(64 - kAhead) - (e & 63u)) << 6 | (e >> 16) << 22;
+        }
+        __syncthreads();
+    }
+    if (tid >= 64) return;   // the first wave decodes
+
+    int i = 0;         // symbols done
+    int64_t pos = 0;   // bits read
+    if (!s_bad && nb > 0) {
+        // Words from the one holding the stream's first bit (past the stream's
+        // last: its last) reach the chain through a ring in LDS, topped up with
+        // 64 of them per batch (load at its start, store at its end), and, within
+        // a batch, a register: lane l holds the batch's l-th word, read by
+        // readlane.  A batch takes at most 31 of them.
+        const int64_t first = boff >> 5, lastw = (boff + nb - 1) >> 5;
+        auto load = [&](int64_t w) { return wb[first + w < lastw ? first + w : lastw]; };
+        ring[lane] = load(lane);
+        ring[64 + lane] = load(64 + lane);
+        int64_t cur = 0, filled = 128;   // words taken before this batch, words in the ring
+        int r = 0;                       // words taken in this batch
+        uint32_t w = 0, q = 0;
+        bool more = false;
+        auto open = [&]() {
+            more = filled - cur < 128;   // at least 64 left
+            if (more) q = load(filled + lane);
+            w = ring[(cur + lane) & (kWordRing - 1)];
+        };
+        auto close = [&]() {
+            cur += r;
+            r = 0;
+            if (more) {
+                ring[(filled + lane) & (kWordRing - 1)] = q;
+                filled += 64;
+            }
+        };
+        BitBuf bb;
+        auto refill = [&]() {   // at least 32 bits in the buffer
+            if (__builtin_amdgcn_readfirstlane((int)(uint32_t)bb.buf) == 0)
+                bb.push((uint32_t)__builtin_amdgcn_readlane((int)w, r++));
+        };
+        auto bits_read = [&]() -> int64_t {   // words taken, less the buffered bits
+            return (cur + r) * 32 - (boff & 31) - (63 - __builtin_ctzll(bb.buf));
+        };
+        // 0, but not known to be alike in all lanes: a lookup at + zero stays in a
+        // vector register until its readfirstlane (a lookup the compiler knows to
+        // be uniform is read to a scalar, and waited for, at once)
+        uint32_t zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        open();
+        bb.init((uint32_t)__builtin_amdgcn_readlane((int)w, r++), (uint32_t)(boff & 31));
+        refill();
+        close();
+        uint32_t slot = x - (uint32_t)kL;
+        if constexpr (PAIR) {
+            uint32_t ix = (slot << kAhead) | (uint32_t)(bb.buf >> (64 - kAhead));
+            // 64 steps read at most 15 bits and decode at most two symbols each
+            while (n - i >= 128 && nb - bits_read() >= 64 * 15 + 64) {
+                open();
+                uint32_t trace = 0, e = two[ix];
+#pragma unroll 8
+                for (int j = 0; j < 64; j++) {
+                    const uint64_t v = bb.buf << (e & 63u);
+                    const uint32_t rs = (e >> 6) & 63u, now = ix;
+                    ix = (uint32_t)(v >> rs) + (e >> 17);
+                    const uint32_t ev = two[ix + zero];   // in flight while the buffer is seen to
+                    __builtin_amdgcn_sched_barrier(0);
+                    trace = lane == j ? now : trace;
+                    bb.buf = v << ((uint32_t)(64 - kAhead) - rs);
+                    refill();
+                    e = (uint32_t)__builtin_amdgcn_readfirstlane((int)ev);
+                }
+                close();
+                const uint32_t e1 = one[trace >> kAhead], k1 = e1 & 63u;
+                const bool both = k1 <= (uint32_t)kAhead;
+                const uint32_t incl = wave_incl_scan(both ? 2u : 1u);
+                int64_t* p = o + i + (incl - (both ? 2u : 1u));
+                p[0] = A[(e1 >> 6) & 1023u];
+                if (both) {
+                    const uint32_t e2 = one[(e1 >> 16) + ((trace & ((1u << kAhead) - 1u)) >> (kAhead - k1))];
+                    p[1] = A[(e2 >> 6) & 1023u];
+                }
+                i += __builtin_amdgcn_readlane((int)incl, 63);
+            }
+            slot = ix >> kAhead;
+        }
+        // one symbol per step, while a step's 10 bits are there: 64 at a time,
+        // then one by one
+        while (n - i >= 64 && nb - bits_read() >= 64 * 10) {
+            open();
+            uint32_t trace = 0, e = one[slot];
+#pragma unroll 8
+            for (int j = 0; j < 64; j++) {
+                const uint32_t now = e;
+                slot = (e >> 16) + (uint32_t)(((uint64_t)(uint32_t)(bb.buf >> 32) << (e & 63u)) >> 32);
+                const uint32_t ev = one[slot + zero];
+                __builtin_amdgcn_sched_barrier(0);
+                trace = lane == j ? now : trace;
+                bb.buf <<= (now & 63u);
+                refill();
+                e = (uint32_t)__builtin_amdgcn_readfirstlane((int)ev);
+            }
+            close();
+            o[i + lane] = A[(trace >> 6) & 1023u];
+            i += 64;
+        }
+        while (i < n && nb - bits_read() >= 10) {
+            open();
+            for (int j = 0; j < 64 && i < n && nb - bits_read() >= 10; j++, i++) {
+                const uint32_t e = one[slot];
+                if (lane == 0) o[i] = A[(e >> 6) & 1023u];
+                slot = (e >> 16) + bb.take(e);
+                refill();
+            }
+            close();
+        }
+        pos = bits_read();
+        x = slot + (uint32_t)kL;
+    }
+    // the plain step (all lanes alike)
+    for (; i < n; i++) {
+        const uint32_t slot = x & (kL - 1);
+        const int si = LU[slot];
+        if (lane == 0) o[i] = A[si];
         x = (uint32_t)F[si] * (x >> 10) + slot - (uint32_t)C[si];
         if (x < (uint32_t)kL) {
             int64_t k = (int64_t)__clz((int)x) - 21;
             if (k > nb - pos) k = nb - pos;
             for (int64_t q = 0; q < k; q++) {
-                int64_t ab = boff + pos + q;
+                const int64_t ab = boff + pos + q;
                 x = (x << 1) | ((wb[ab >> 5] >> (ab & 31)) & 1u);
             }
             pos += k;
@@ -1906,8 +2166,8 @@ int lq_rans_encode_streams(const int32_t* d_idx, const int64_t* d_sym_off, const
                            uint32_t* d_words, const int64_t* d_word_off, int64_t* d_state, int64_t* d_nbits,
                            hipStream_t s) {
     if (n_streams <= 0) return LQ_ERR_ARG;
-    hipLaunchKernelGGL(k_encode_streams, dim3((unsigned)((n_streams + 63) / 64)), dim3(64), 0, s, d_idx, d_sym_off, d_n,
-                       d_freqs, d_cum, d_tab_off, n_streams, d_scratch, d_words, d_word_off, d_state, d_nbits);
+    hipLaunchKernelGGL(k_encode_streams, dim3((unsigned)n_streams), dim3(kSegLanes), 0, s, d_idx, d_sym_off, d_n, d_freqs,
+                       d_cum, d_tab_off, d_scratch, d_words, d_word_off, d_state, d_nbits);
     return launch_status();
 }
 
@@ -1916,8 +2176,12 @@ int lq_rans_decode_streams(const int32_t* d_bits, const int32_t* d_bit_off, cons
                            const int32_t* d_alphabet, const int32_t* d_tid, int32_t max_sym, const int32_t* d_out_off,
                            int32_t n_streams, int64_t* d_out, hipStream_t s) {
     if (n_streams <= 0 || max_sym <= 0) return LQ_ERR_ARG;
-    hipLaunchKernelGGL(k_decode_streams, dim3((unsigned)((n_streams + 63) / 64)), dim3(64), 0, s, d_bits, d_bit_off, d_nbits,
-                       d_init, d_ndec, d_lookup, d_freqs, d_cum, d_alphabet, d_tid, max_sym, d_out_off, n_streams, d_out);
+    if (n_streams <= 2 * device_cus())
+        hipLaunchKernelGGL(k_decode_streams<true>, dim3((unsigned)n_streams), dim3(256), 0, s, d_bits, d_bit_off, d_nbits,
+                           d_init, d_ndec, d_lookup, d_freqs, d_cum, d_alphabet, d_tid, max_sym, d_out_off, d_out);
+    else
+        hipLaunchKernelGGL(k_decode_streams<false>, dim3((unsigned)n_streams), dim3(256), 0, s, d_bits, d_bit_off, d_nbits,
+                           d_init, d_ndec, d_lookup, d_freqs, d_cum, d_alphabet, d_tid, max_sym, d_out_off, d_out);
     return launch_status();
 }
 

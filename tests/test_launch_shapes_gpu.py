@@ -122,3 +122,63 @@ def test_int8_tables_tie_order_gpu(kind):
         got = t[i, 4:4 + n].view(np.uint32)
         assert np.array_equal(got & 0x7ff, want), (kind, m)
         assert np.array_equal((got >> 11) & 0x3ff, (np.cumsum(want) - want) & 0x3ff)
+
+
+def _stream(rng, n, spread):
+    s = np.rint(rng.normal(0.0, spread, n)).astype(np.int64) if spread else np.zeros(n, np.int64)
+    lo, hi = (int(s.min()), int(s.max())) if n else (0, 0)
+    pad = 2 if spread else 0    # spread 0: one symbol with all of L, no bits
+    counts = np.bincount(s - lo, minlength=hi - lo + 1)
+    alphabet = list(range(lo - pad, hi + pad + 1))
+    return s, np.concatenate([np.zeros(pad, np.int64), counts if n else np.ones(1, np.int64), np.zeros(pad, np.int64)]), alphabet
+
+
+# lengths around a segment (64), the window behind it (16, 64), a decoder batch
+# (64, 128) and a tile of segments (65536); spreads from no bits per symbol to
+# alphabets near L
+@pytest.mark.parametrize("spread", [0.0, 0.3, 3.0, 40.0, 100.0])
+def test_stream_coder_lengths_gpu(spread):
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(int(10 * spread) + 1)
+    lens = [0, 1, 2, 15, 16, 17, 63, 64, 65, 80, 127, 128, 129, 191, 192, 193, 500, 1000, 4097, 65535, 65536, 65537, 70001]
+    parts = [_stream(rng, n, spread) for n in lens]
+    tabs = gpu_ans.build_rans_tables([p[1] for p in parts], [p[2] for p in parts])
+    enc = gpu_ans.rans_encode_many([p[0] for p in parts], tabs)
+    for (s, counts, alphabet), (words, state, nbits) in zip(parts, enc):
+        want = O.rans_encode(s, O.build_rans_table(counts, alphabet))
+        assert (state, nbits) == (int(want[1]), int(want[2])), len(s)
+        assert np.array_equal(words, want[0]), len(s)
+    streams = [gpu_ans.RANSStream(w, nb, st, len(p[0]), t) for (w, st, nb), p, t in zip(enc, parts, tabs)]
+    for got, p in zip(gpu_ans.gpu_rans_decode(streams), parts):
+        assert np.array_equal(got, p[0]), len(p[0])
+    # more streams than the two-symbol tables are taken for
+    many = gpu_ans.gpu_rans_decode([streams[i % 19] for i in range(600)])
+    for i, got in enumerate(many):
+        assert np.array_equal(got, parts[i % 19][0])
+
+
+def test_stream_decoder_truncated_gpu():
+    """A stream with fewer bits than its symbols need is decoded to its length
+    with the reference's rule (a step reads min(needed, bits left)), from any
+    state, as the plain step written out below."""
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(5)
+    s, counts, alphabet = _stream(rng, 700, 9.0)
+    tab = gpu_ans.build_rans_tables([counts], [alphabet])[0]
+    words, state, nbits = gpu_ans.rans_encode_many([s], [tab])[0]
+    cases = [(nbits, state, 700), (nbits - 1, state, 700), (nbits // 2, state, 700), (9, state, 60), (0, state, 40),
+             (nbits, 1024, 700), (nbits, 77, 700), (nbits, state, 760)]
+    streams = [gpu_ans.RANSStream(words, nb, st, n, tab) for nb, st, n in cases]
+    for (nb, st, n), got in zip(cases, gpu_ans.gpu_rans_decode(streams)):
+        x, pos, want = st, 0, []
+        for _ in range(n):
+            slot = x & 1023
+            si = int(tab.lookup[slot])
+            want.append(tab.alphabet[si])
+            x = (int(tab.freqs[si]) * (x >> 10) + slot - int(tab.cumfreqs[si])) & 0xffffffff
+            if x < 1024:
+                k = min((32 - x.bit_length()) - 21, nb - pos)
+                for q in range(pos, pos + k):
+                    x = (x << 1) | (int(words[q >> 5]) >> (q & 31) & 1)
+                pos += max(k, 0)
+        assert np.array_equal(got, np.array(want)), (nb, st, n)

@@ -239,6 +239,32 @@ int lq_chunk_pack(int64_t n_chunks, int64_t n_vectors, const lq_table *d_tables,
                   const uint32_t *d_blk_off, const int64_t *d_stream_nbits, const int64_t *d_stream_woff,
                   const int64_t *d_chunk_base, uint32_t *d_words, hipStream_t s);
 
+/* The int8 write path as one call: lq_head_scales (or, scales_given: the fp16
+ * copies and fast-division words of the d_scale32 the caller filled in),
+ * lq_chunk_quantize, lq_chunk_tables, lq_chunk_encode, the chunk bases
+ * (d_chunk_base: exclusive prefix of d_chunk_words) and, when d_words is given,
+ * lq_chunk_pack.  d_signs (nullable) selects the rotated forms (head_dim as
+ * there; d_deq must be null then).  d_hist, d_status and the counters are
+ * cleared here.  skip_overflowed: when a chunk has LQ_ST_SYM_OVERFLOW, every
+ * chunk gets empty streams (the caller will take the wide path).  d_work:
+ * lq_encode_chunks_workspace bytes, 256-byte aligned; lq_encode_chunks_pack is
+ * the pack alone, from the same workspace, for a caller that sizes d_words by
+ * d_chunk_words first.  h_status, h_words (nullable, host memory): the call
+ * returns once the OR of the chunks' status bits, and the sum of d_chunk_words,
+ * are there (it waits for the table, or the offset, launch; those behind it run
+ * on).  Without them it does not wait.  Replaces llm/compressed_kv_cache.py:188-263. */
+int64_t lq_encode_chunks_workspace(int64_t n_chunks, int64_t n_heads, int64_t bph);
+int lq_encode_chunks(const void *d_x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph, int head_dim,
+                     const float *d_signs, const int64_t *d_dither_seed, const int32_t *d_chunk_bits, int scales_given,
+                     float *d_sigma2, float *d_scale32, uint16_t *d_scale16, uint8_t *d_coset_bits, uint32_t *d_blk_n1,
+                     void *d_deq, uint32_t *d_hist, int32_t *d_status, lq_table *d_tables, uint32_t *d_blk_off,
+                     uint16_t *d_blk_state, int64_t *d_stream_nbits, int32_t *d_stream_state, int64_t *d_stream_woff,
+                     int64_t *d_chunk_words, int64_t *d_chunk_base, uint32_t *d_words, int skip_overflowed, void *d_work,
+                     int64_t *h_status, int64_t *h_words, hipStream_t s);
+int lq_encode_chunks_pack(int64_t n_chunks, int64_t n_heads, int64_t bph, const lq_table *d_tables, const void *d_work,
+                          const uint32_t *d_blk_off, const int64_t *d_stream_nbits, const int64_t *d_stream_woff,
+                          const int64_t *d_chunk_base, uint32_t *d_words, hipStream_t s);
+
 /* Decode + dequantize a batch of chunks to (B, H, T, hd) in out_dtype:
  * fp16(q * float(scale16[head])).  d_lut_work is not used and may be null (the
  * decoder builds its LUTs in LDS).

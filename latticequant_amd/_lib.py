@@ -56,6 +56,9 @@ _SIGS = {
     "lq_chunk_encode_wide": ([_P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P], _INT),
     "lq_chunk_encode_workspace": ([_I64, _I64], _I64),
     "lq_chunk_encode": ([_P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P], _INT),
+    "lq_encode_chunks_workspace": ([_I64, _I64, _I64], _I64),
+    "lq_encode_chunks": ([_P, _INT, _I64, _I64, _I64, _INT, _P, _P, _P, _INT] + [_P] * 17 + [_INT, _P, _P, _P, _P], _INT),
+    "lq_encode_chunks_pack": ([_I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P], _INT),
     "lq_chunk_pack": ([_I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P], _INT),
     "lq_chunk_decode": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _INT, _P, _P], _INT),
     "lq_build_tables": ([_P, _P, _P, _I32, _P, _P, _P, _P, _P], _INT),

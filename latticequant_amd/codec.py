@@ -19,6 +19,7 @@ for.  All compute runs in the kernels of liblatticequant_amd.so.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -551,75 +552,158 @@ def encode_batch(x: torch.Tensor, bits, scale32: Optional[torch.Tensor] = None, 
             w = rotate_rows(x, rht_signs, inverse=False)
             return encode_batch(w, bits, scale32, deq_out, exact_size, words_out, wide, dither_seed,
                                 escape=escape)
+    if wide is not True:
+        enc, deq = _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, wide == "auto", dither_seed, rht_signs)
+        if enc.words is not None:
+            return enc, deq
+        # a chunk's symbols left int8: the int16 path, with the same scales (it
+        # reads the materialised rotation)
+        if rht_signs is not None:
+            w = rotate_rows(x, rht_signs, inverse=False)
+            return encode_batch(w, bits, enc.scale32, deq_out, exact_size, words_out, wide, dither_seed, escape=escape)
+        scales = (enc.bits, enc.scale32, enc.scale16, enc.sigma2)
+    else:
+        scales = None
+    return _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide, dither_seed, escape)
+
+
+def _dither_tensor(dither_seed, C: int, dev) -> Optional[torch.Tensor]:
+    if dither_seed is None:
+        return None
+    ds = [int(dither_seed)] * C if isinstance(dither_seed, int) else [int(v) for v in dither_seed]
+    if len(ds) != C:
+        raise ValueError("dither_seed must be an int or one seed per chunk")
+    # from pinned memory: a copy from pageable memory waits for the stream's earlier work
+    return torch.tensor(ds, dtype=torch.int64, pin_memory=True).to(dev, non_blocking=True)
+
+
+def _arena(words_out: Optional[torch.Tensor], C: int, V: int, dev) -> torch.Tensor:
+    """The caller's arena, checked, or one at the upper bound."""
+    bound = words_bound(C, V)
+    if words_out is None:
+        return _empty(bound, torch.int32, dev)
+    if words_out.numel() < bound:
+        raise ValueError(f"words_out holds {words_out.numel()} words, needs {bound}")
+    return words_out
+
+
+def _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, auto, dither_seed, rht_signs):
+    """encode_batch on int8 symbols: one native call (lq_encode_chunks), which
+    also reads back the chunks' status (auto) and total size (for an arena of
+    its own, exact_size); `auto` and a symbol outside int8: words is None."""
+    lib = L.lib()
+    C, B, H, T, hd = x.shape
+    dev = x.device
+    nh, bph = B * H, T * hd // 8
+    V = nh * bph
+    S = L.LQ_STREAMS
+    nblk = (V + L.LQ_BLK - 1) // L.LQ_BLK
+    n = C * nh
+    given = scale32 is not None
+    if given:
+        scale32 = scale32.to(device=dev, dtype=torch.float32).contiguous().view(-1)
+        if scale32.numel() != n:
+            raise ValueError("scale32 must hold one scale per head of every chunk")
+    dt = L.dtype_code(x.dtype)
+    bits_t = _bits_tensor(bits, C, dev)
+    dseed = _dither_tensor(dither_seed, C, dev)
+    sized = exact_size and words_out is None   # the arena waits for the sizes
+    words = None if sized else _arena(words_out, C, V, dev)
+    # the batch's arrays, cut from one buffer per element type (each part 256-byte aligned)
+    chunk_words, stream_nbits, stream_woff, chunk_base = _cut(torch.int64, dev, (C, S * C, S * C, C))
+    blk_n1, blk_off, stream_state, status, hist = _cut(torch.int32, dev, (C * nblk, C * S * nblk, C * S, C, C * S * 256))
+    coset_bits, tables = _cut(torch.uint8, dev, (C * nblk * L.LQ_BLK // 8, C * S * L.TABLE_BYTES))
+    blk_state = _empty(C * S * nblk, torch.int16, dev)
+    if given:
+        sigma2, scale16 = None, _empty(n, torch.float16, dev)
+    else:
+        sigma2, scale32, s16 = _cut(torch.float32, dev, (n, n, (n + 1) // 2))
+        scale16 = s16.view(torch.float16)[:n]
+    deq = torch.empty_like(x) if deq_out else None
+    work = _empty(lib.lq_encode_chunks_workspace(C, nh, bph), torch.uint8, dev)
+    s = L.stream_ptr(dev)
+    host = (ctypes.c_int64 * 2)()   # status bits, total words: read back where asked for
+    at = ctypes.addressof(host)
+    L.check(lib.lq_encode_chunks(x.data_ptr(), dt, C, nh, bph, hd, L.ptr(rht_signs), L.ptr(dseed), bits_t.data_ptr(),
+                                 1 if given else 0, L.ptr(sigma2), scale32.data_ptr(), scale16.data_ptr(),
+                                 coset_bits.data_ptr(), blk_n1.data_ptr(), L.ptr(deq), hist.data_ptr(),
+                                 status.data_ptr(), tables.data_ptr(), blk_off.data_ptr(), blk_state.data_ptr(),
+                                 stream_nbits.data_ptr(), stream_state.data_ptr(), stream_woff.data_ptr(),
+                                 chunk_words.data_ptr(), chunk_base.data_ptr(), L.ptr(words), 1 if auto else 0,
+                                 work.data_ptr(), at if auto else None, at + 8 if sized else None, s),
+            "lq_encode_chunks")
+    overflow = auto and bool(host[0] & L.LQ_ST_SYM_OVERFLOW)
+    if sized and not overflow:
+        words = _empty(host[1] + 2, torch.int32, dev)   # decoder read-ahead slack
+        L.check(lib.lq_encode_chunks_pack(C, nh, bph, tables.data_ptr(), work.data_ptr(), blk_off.data_ptr(),
+                                          stream_nbits.data_ptr(), stream_woff.data_ptr(), chunk_base.data_ptr(),
+                                          words.data_ptr(), s), "lq_encode_chunks_pack")
+    return EncodedBatch(n_chunks=C, n_heads=nh, bph=bph, shape=(B, H, T, hd), bits=bits_t, scale32=scale32,
+                        scale16=scale16, sigma2=sigma2, coset_bits=coset_bits.view(C, -1), blk_n1=blk_n1.view(C, -1),
+                        tables=tables, blk_off=blk_off, blk_state=blk_state, stream_nbits=stream_nbits,
+                        stream_state=stream_state, stream_woff=stream_woff, chunk_words=chunk_words,
+                        chunk_base=chunk_base, words=None if overflow else words, status=status, hist=hist,
+                        extra={"wide": False, "dither_seed": dseed, "esc": None}), deq
+
+
+def _cut(dtype, dev, sizes):
+    """Uninitialised device arrays of `sizes` elements, cut from one buffer,
+    each 256-byte aligned."""
+    unit = 256 // dtype.itemsize
+    padded = [(n + unit - 1) // unit * unit for n in sizes]
+    parts = torch.empty(sum(padded), dtype=dtype, device=dev).split(padded)
+    return [p if p.numel() == n else p[:n] for p, n in zip(parts, sizes)]
+
+
+def _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide, dither_seed, escape):
+    """encode_batch on int16 symbols.  scales: (bits, scale32, scale16, sigma2)
+    of the int8 attempt, or None."""
+    lib = L.lib()
+    C, B, H, T, hd = x.shape
     dev = x.device
     nh, bph = B * H, T * hd // 8
     V = nh * bph
     nblk = (V + L.LQ_BLK - 1) // L.LQ_BLK
     dt = L.dtype_code(x.dtype)
     s = L.stream_ptr(dev)
-    bits_t, scale32, scale16, sigma2, fastdiv = _head_scales(x, bits, scale32, rht_signs)
+    if scales is None:
+        bits_t, scale32, scale16, sigma2, fastdiv = _head_scales(x, bits, scale32)
+    else:
+        bits_t, scale32, scale16, sigma2 = scales
+        fastdiv = _empty(C * nh, torch.int32, dev)
+        L.check(lib.lq_scale_fastdiv(scale32.data_ptr(), C * nh, dt, fastdiv.data_ptr(), s), "lq_scale_fastdiv")
     # every block's 64 bytes of coset bits are written by the quantizer (bits of
     # vectors past the end are zero), so no fill
     coset_bits = _empty(C * nblk * L.LQ_BLK // 8, torch.uint8, dev)
     blk_n1 = _empty(C * nblk, torch.int32, dev)
-    use_wide = wide is True
-    esc = None
-    # one zero fill: the status flags, the int8 path's histogram and a leading
-    # zero before the chunks' word counts (so that one inclusive scan of
-    # [0, w_0 .. w_{C-2}] gives the chunk bases)
-    status, hist, cwz = _zero_views(dev, (C, torch.int32), (0 if use_wide else C * L.LQ_STREAMS * 256, torch.int32),
-                                    (C + 1, torch.int64))
+    # one zero fill: the status flags and a leading zero before the chunks' word
+    # counts (so that one inclusive scan of [0, w_0 .. w_{C-2}] gives the chunk bases)
+    status, cwz, hist = _zero_views(dev, (C, torch.int32), (C + 1, torch.int64), (C * L.LQ_STREAMS * L.LQ_L, torch.int32))
     deq = torch.empty_like(x) if deq_out else None
     tables = _empty(C * L.LQ_STREAMS * L.TABLE_BYTES, torch.uint8, dev)
-    dseed = None
-    if dither_seed is not None:
-        ds = [int(dither_seed)] * C if isinstance(dither_seed, int) else [int(v) for v in dither_seed]
-        if len(ds) != C:
-            raise ValueError("dither_seed must be an int or one seed per chunk")
-        dseed = torch.tensor(ds, dtype=torch.int64).to(dev)
-    if not use_wide:
-        sym = _empty(C * nblk * L.LQ_SYM_STRIDE, torch.int8, dev)
-        if rht_signs is not None:
-            L.check(lib.lq_chunk_quantize_rht(x.data_ptr(), dt, C, nh, bph, hd, rht_signs.data_ptr(),
-                                              scale32.data_ptr(), sym.data_ptr(), coset_bits.data_ptr(),
-                                              blk_n1.data_ptr(), hist.data_ptr(), status.data_ptr(), L.ptr(dseed), s),
-                    "lq_chunk_quantize_rht")
-        else:
-            L.check(lib.lq_chunk_quantize(x.data_ptr(), dt, C, nh, bph, scale32.data_ptr(), fastdiv.data_ptr(),
-                                          sym.data_ptr(), coset_bits.data_ptr(), blk_n1.data_ptr(), hist.data_ptr(),
-                                          status.data_ptr(), L.ptr(deq), dt, L.ptr(dseed), s), "lq_chunk_quantize")
-        if wide == "auto" and _status_or(status) & L.LQ_ST_SYM_OVERFLOW:
-            if rht_signs is not None:   # the int16 path reads the materialised rotation
-                w = rotate_rows(x, rht_signs, inverse=False)
-                return encode_batch(w, bits, scale32, deq_out, exact_size, words_out, wide, dither_seed,
-                                    escape=escape)
-            use_wide = True
-            status.zero_()
-        else:
-            L.check(lib.lq_chunk_tables(hist.data_ptr(), C, tables.data_ptr(), status.data_ptr(), s), "lq_chunk_tables")
-    if use_wide:
-        sym = _empty(C * nblk * L.LQ_SYM_STRIDE, torch.int16, dev)
-        minmax = torch.empty(C * L.LQ_STREAMS, 2, dtype=torch.int32, device=dev)
-        minmax[:, 0] = 2 ** 31 - 1
-        minmax[:, 1] = -2 ** 31
-        hist = _zeros(C * L.LQ_STREAMS * L.LQ_L, torch.int32, dev)
-        L.check(lib.lq_chunk_quantize_wide(x.data_ptr(), dt, C, nh, bph, scale32.data_ptr(), fastdiv.data_ptr(),
-                                           sym.data_ptr(), coset_bits.data_ptr(), blk_n1.data_ptr(), minmax.data_ptr(),
-                                           status.data_ptr(), L.ptr(deq), dt, L.ptr(dseed), s),
-                "lq_chunk_quantize_wide")
-        if escape:
-            esc, minmax = _plan_escape(minmax, C, nblk, V, sym, coset_bits, blk_n1, status, dev, s)
-        L.check(lib.lq_chunk_hist_wide(sym.data_ptr(), blk_n1.data_ptr(), C, V, minmax.data_ptr(), hist.data_ptr(), s),
-                "lq_chunk_hist_wide")
-        L.check(lib.lq_chunk_tables_wide(hist.data_ptr(), minmax.data_ptr(), C, tables.data_ptr(), status.data_ptr(), s),
-                "lq_chunk_tables_wide")
-        if wide == "auto" or exact_size:
-            st = _status_or(status)
-            if st & L.LQ_ST_ALPHABET:
-                raise AlphabetError("a stream's alphabet exceeds L = 1024 symbols (the reference's table "
-                                    "normalisation never terminates there); use more bits or smaller chunks")
-            if st & L.LQ_ST_SYM_OVERFLOW:
-                raise AlphabetError("a lattice symbol does not fit int16")
+    dseed = _dither_tensor(dither_seed, C, dev)
+    sym = _empty(C * nblk * L.LQ_SYM_STRIDE, torch.int16, dev)
+    minmax = torch.empty(C * L.LQ_STREAMS, 2, dtype=torch.int32, device=dev)
+    minmax[:, 0] = 2 ** 31 - 1
+    minmax[:, 1] = -2 ** 31
+    L.check(lib.lq_chunk_quantize_wide(x.data_ptr(), dt, C, nh, bph, scale32.data_ptr(), fastdiv.data_ptr(),
+                                       sym.data_ptr(), coset_bits.data_ptr(), blk_n1.data_ptr(), minmax.data_ptr(),
+                                       status.data_ptr(), L.ptr(deq), dt, L.ptr(dseed), s),
+            "lq_chunk_quantize_wide")
+    esc = None
+    if escape:
+        esc, minmax = _plan_escape(minmax, C, nblk, V, sym, coset_bits, blk_n1, status, dev, s)
+    L.check(lib.lq_chunk_hist_wide(sym.data_ptr(), blk_n1.data_ptr(), C, V, minmax.data_ptr(), hist.data_ptr(), s),
+            "lq_chunk_hist_wide")
+    L.check(lib.lq_chunk_tables_wide(hist.data_ptr(), minmax.data_ptr(), C, tables.data_ptr(), status.data_ptr(), s),
+            "lq_chunk_tables_wide")
+    if wide == "auto" or exact_size:
+        st = _status_or(status)
+        if st & L.LQ_ST_ALPHABET:
+            raise AlphabetError("a stream's alphabet exceeds L = 1024 symbols (the reference's table "
+                                "normalisation never terminates there); use more bits or smaller chunks")
+        if st & L.LQ_ST_SYM_OVERFLOW:
+            raise AlphabetError("a lattice symbol does not fit int16")
     ws = lib.lq_chunk_encode_workspace(C, V)
     work = _empty(ws, torch.uint8, dev)
     ntask = C * L.LQ_STREAMS * nblk
@@ -629,21 +713,15 @@ def encode_batch(x: torch.Tensor, bits, scale32: Optional[torch.Tensor] = None, 
     stream_state = _empty(C * L.LQ_STREAMS, torch.int32, dev)
     stream_woff = _empty(C * L.LQ_STREAMS, torch.int64, dev)
     chunk_words = cwz[1:]
-    enc_fn = lib.lq_chunk_encode_wide if use_wide else lib.lq_chunk_encode
-    L.check(enc_fn(sym.data_ptr(), blk_n1.data_ptr(), C, V, tables.data_ptr(), work.data_ptr(),
-                   blk_off.data_ptr(), blk_state.data_ptr(), stream_nbits.data_ptr(),
-                   stream_state.data_ptr(), stream_woff.data_ptr(), chunk_words.data_ptr(), s),
-            "lq_chunk_encode_wide" if use_wide else "lq_chunk_encode")
+    L.check(lib.lq_chunk_encode_wide(sym.data_ptr(), blk_n1.data_ptr(), C, V, tables.data_ptr(), work.data_ptr(),
+                                     blk_off.data_ptr(), blk_state.data_ptr(), stream_nbits.data_ptr(),
+                                     stream_state.data_ptr(), stream_woff.data_ptr(), chunk_words.data_ptr(), s),
+            "lq_chunk_encode_wide")
     chunk_base = torch.cumsum(cwz[:C], 0)
-    bound = words_bound(C, V)
-    if words_out is not None:
-        if words_out.numel() < bound:
-            raise ValueError(f"words_out holds {words_out.numel()} words, needs {bound}")
-        words = words_out
-    elif exact_size:
+    if exact_size and words_out is None:
         words = _empty(int(chunk_words.sum().item()) + 2, torch.int32, dev)   # decoder read-ahead slack
     else:
-        words = _empty(bound, torch.int32, dev)
+        words = _arena(words_out, C, V, dev)
     L.check(lib.lq_chunk_pack(C, V, tables.data_ptr(), work.data_ptr(), blk_off.data_ptr(), stream_nbits.data_ptr(),
                               stream_woff.data_ptr(), chunk_base.data_ptr(), words.data_ptr(), s), "lq_chunk_pack")
     enc = EncodedBatch(n_chunks=C, n_heads=nh, bph=bph, shape=(B, H, T, hd), bits=bits_t, scale32=scale32,
@@ -651,7 +729,7 @@ def encode_batch(x: torch.Tensor, bits, scale32: Optional[torch.Tensor] = None, 
                        tables=tables, blk_off=blk_off, blk_state=blk_state, stream_nbits=stream_nbits,
                        stream_state=stream_state, stream_woff=stream_woff, chunk_words=chunk_words,
                        chunk_base=chunk_base, words=words, status=status, hist=hist,
-                       extra={"wide": use_wide, "dither_seed": dseed, "esc": esc})
+                       extra={"wide": True, "dither_seed": dseed, "esc": esc})
     return enc, deq
 
 

@@ -2,6 +2,7 @@
 // per-head scales and the chunk quantizer of the compressed-KV write path.
 #include <climits>
 
+#include "lq_launch.h"
 #include "lq_scales.h"
 
 using namespace lq;
@@ -83,12 +84,24 @@ __global__ void k_quantize_heads(const void* __restrict__ x, int dtype, int64_t 
 
 // ---------------------------------------------------------- head scales --
 
+// Clears c's words, thread i of n.
+__device__ __forceinline__ void clear_words(const Clear& c, int64_t i, int64_t n) {
+    for (int64_t j = i; j < c.n_hist; j += n) c.hist[j] = 0u;
+    for (int64_t j = i; j < c.n_status; j += n) c.status[j] = 0;
+    if (c.counter && i == 0) *c.counter = 0u;
+}
+
 // Partial sums of x^2 per head in double: grid (heads, parts).  ROT: of the
-// forward-rotated rows (lq_scales.h head_sumsq_part); LPR > 0: lpr known.
+// forward-rotated rows (lq_scales.h head_sumsq_part); LPR > 0: lpr known.  On
+// the side it clears the words of `clear` (a launch of their own took 2.3 us
+// and its gap).
 template <bool ROT, int LPR = 0>
 __global__ void k_head_sumsq(const void* __restrict__ x, int dtype, int64_t vec_per_head, int parts,
-                             double* __restrict__ work, const float* __restrict__ signs, int lpr, float rdiv) {
+                             double* __restrict__ work, const float* __restrict__ signs, int lpr, float rdiv,
+                             Clear clear) {
     __shared__ double red[256];
+    clear_words(clear, ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x,
+                (int64_t)gridDim.x * gridDim.y * blockDim.x);
     head_sumsq_part<ROT, LPR>(x, dtype, vec_per_head, parts, blockIdx.x, blockIdx.y, work, red, signs, lpr, rdiv);
 }
 
@@ -125,8 +138,11 @@ __global__ __launch_bounds__(256) void k_head_finalize(const double* __restrict_
     }
 }
 
-__global__ void k_scale_fastdiv(const float* __restrict__ scale32, int dtype, int32_t* __restrict__ fastdiv) {
+__global__ void k_scale_fastdiv(const float* __restrict__ scale32, int dtype, int32_t* __restrict__ fastdiv,
+                                uint16_t* __restrict__ scale16, Clear clear) {
     int64_t h = blockIdx.x;
+    clear_words(clear, h * blockDim.x + threadIdx.x, (int64_t)gridDim.x * blockDim.x);
+    if (scale16 && threadIdx.x == 0) scale16[h] = f2h(scale32[h]);
     if (dtype == LQ_F16) {
         fastdiv_check(scale32[h], fastdiv + h);
     } else if (threadIdx.x == 0) {
@@ -584,6 +600,43 @@ inline int launch_status() { return hipGetLastError() == hipSuccess ? LQ_OK : LQ
 
 }  // namespace
 
+namespace lq {
+
+int head_scales_launch(const void* x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph, int head_dim,
+                       const float* signs, const int32_t* bits, double* work, float* sigma2, float* scale32,
+                       uint16_t* scale16, int32_t* fastdiv, const Clear& clear, hipStream_t s) {
+    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || dtype < 0 || dtype > 2) return LQ_ERR_ARG;
+    if (signs && (head_dim < 8 || head_dim > 128 || (head_dim & (head_dim - 1)) || bph % (head_dim / 8)))
+        return LQ_ERR_ARG;
+    const int64_t H = n_chunks * n_heads;
+    const int parts = head_parts(H, bph);
+    const float div = signs ? (float)sqrt((double)head_dim) : 1.0f;
+    const int lpr = signs ? head_dim / 8 : 1;
+    const dim3 grid((unsigned)H, parts);
+    if (!signs)
+        hipLaunchKernelGGL((k_head_sumsq<false, 0>), grid, dim3(256), 0, s, x, dtype, bph, parts, work, nullptr, lpr, div,
+                           clear);
+    else if (head_dim == 128)
+        hipLaunchKernelGGL((k_head_sumsq<true, 16>), grid, dim3(256), 0, s, x, dtype, bph, parts, work, signs, lpr, div,
+                           clear);
+    else
+        hipLaunchKernelGGL((k_head_sumsq<true, 0>), grid, dim3(256), 0, s, x, dtype, bph, parts, work, signs, lpr, div,
+                           clear);
+    // rotated rows are fp32: no fast-division word
+    hipLaunchKernelGGL(k_head_finalize, dim3((unsigned)H), dim3(256), 0, s, work, parts, bph * 8, n_heads, bits,
+                       signs ? (int)LQ_F32 : dtype, sigma2, scale32, scale16, fastdiv);
+    return launch_status();
+}
+
+int scale_fastdiv_launch(const float* scale32, int64_t n, int dtype, int32_t* fastdiv, uint16_t* scale16,
+                         const Clear& clear, hipStream_t s) {
+    if (n <= 0) return LQ_ERR_ARG;
+    hipLaunchKernelGGL(k_scale_fastdiv, dim3((unsigned)n), dim3(256), 0, s, scale32, dtype, fastdiv, scale16, clear);
+    return launch_status();
+}
+
+}  // namespace lq
+
 extern "C" {
 
 int lq_e8_encode_f32(const float* d_x, int64_t n, int mode, float* d_out, hipStream_t s) {
@@ -610,14 +663,8 @@ int lq_symbols_to_e8(const int32_t* d_coset, const int32_t* d_sym8, int64_t n, f
 int lq_head_scales(const void* d_x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph,
                    const int32_t* d_chunk_bits, double* d_work, float* d_sigma2, float* d_scale32,
                    uint16_t* d_scale16, int32_t* d_fastdiv, hipStream_t s) {
-    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || dtype < 0 || dtype > 2) return LQ_ERR_ARG;
-    const int64_t H = n_chunks * n_heads;
-    const int parts = head_parts(H, bph);
-    hipLaunchKernelGGL(k_head_sumsq<false>, dim3((unsigned)H, parts), dim3(256), 0, s, d_x, dtype, bph, parts, d_work,
-                       nullptr, 1, 1.0f);
-    hipLaunchKernelGGL(k_head_finalize, dim3((unsigned)H), dim3(256), 0, s, d_work, parts, bph * 8, n_heads,
-                       d_chunk_bits, dtype, d_sigma2, d_scale32, d_scale16, d_fastdiv);
-    return launch_status();
+    return head_scales_launch(d_x, dtype, n_chunks, n_heads, bph, 0, nullptr, d_chunk_bits, d_work, d_sigma2, d_scale32,
+                              d_scale16, d_fastdiv, Clear{}, s);
 }
 
 // Small updates without entropy coding: lq_head_scales, then the quantizer
@@ -661,26 +708,13 @@ int lq_quantize_deq(const void* d_x, int dtype, int64_t n_chunks, int64_t n_head
 int lq_head_scales_rht(const void* d_x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph, int head_dim,
                        const float* d_signs, const int32_t* d_chunk_bits, double* d_work, float* d_sigma2,
                        float* d_scale32, uint16_t* d_scale16, int32_t* d_fastdiv, hipStream_t s) {
-    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || dtype < 0 || dtype > 2 || !d_signs) return LQ_ERR_ARG;
-    if (head_dim < 8 || head_dim > 128 || (head_dim & (head_dim - 1)) || bph % (head_dim / 8)) return LQ_ERR_ARG;
-    const int64_t H = n_chunks * n_heads;
-    const int parts = head_parts(H, bph);
-    const float div = (float)sqrt((double)head_dim);
-    if (head_dim == 128)
-        hipLaunchKernelGGL((k_head_sumsq<true, 16>), dim3((unsigned)H, parts), dim3(256), 0, s, d_x, dtype, bph, parts,
-                           d_work, d_signs, 16, div);
-    else
-        hipLaunchKernelGGL((k_head_sumsq<true, 0>), dim3((unsigned)H, parts), dim3(256), 0, s, d_x, dtype, bph, parts,
-                           d_work, d_signs, head_dim / 8, div);
-    hipLaunchKernelGGL(k_head_finalize, dim3((unsigned)H), dim3(256), 0, s, d_work, parts, bph * 8, n_heads,
-                       d_chunk_bits, (int)LQ_F32, d_sigma2, d_scale32, d_scale16, d_fastdiv);
-    return launch_status();
+    if (!d_signs) return LQ_ERR_ARG;
+    return head_scales_launch(d_x, dtype, n_chunks, n_heads, bph, head_dim, d_signs, d_chunk_bits, d_work, d_sigma2,
+                              d_scale32, d_scale16, d_fastdiv, Clear{}, s);
 }
 
 int lq_scale_fastdiv(const float* d_scale32, int64_t n_heads_total, int dtype, int32_t* d_fastdiv, hipStream_t s) {
-    if (n_heads_total <= 0) return LQ_ERR_ARG;
-    hipLaunchKernelGGL(k_scale_fastdiv, dim3((unsigned)n_heads_total), dim3(256), 0, s, d_scale32, dtype, d_fastdiv);
-    return launch_status();
+    return scale_fastdiv_launch(d_scale32, n_heads_total, dtype, d_fastdiv, nullptr, Clear{}, s);
 }
 
 int lq_e8_quantize_heads(const void* d_x, int dtype, int64_t n_heads, int64_t bph, const float* d_scale32,

@@ -15,9 +15,12 @@
 // the end of the stream where the state is exactly L.  Results are therefore
 // exact, and identical to a serial encode.
 #include <climits>
+#include <mutex>
+#include <vector>
 
 #include "lq_argsort.h"
 #include "lq_decode.h"
+#include "lq_launch.h"
 
 using namespace lq;
 
@@ -513,9 +516,14 @@ __global__ __launch_bounds__(256) void k_chunk_tables(const uint32_t* __restrict
 constexpr int kTabWaves = 4;
 constexpr int kCap8 = 264;   // range(min - 2, max + 2) of int8 values: at most 260 symbols
 
+// skip: when a chunk's symbols left int8 (LQ_ST_SYM_OVERFLOW, set by the launch
+// before) every stream of the batch is left empty, so that the launches that
+// follow do nothing.  host (nullable, host memory): the OR of the chunks' status
+// words so far.
 __global__ __launch_bounds__(64 * kTabWaves) void k_chunk_tables_wave(const uint32_t* __restrict__ hist,
                                                                       int64_t n_streams, lq_table* __restrict__ tables,
-                                                                      int32_t* __restrict__ status) {
+                                                                      int32_t* __restrict__ status, int skip,
+                                                                      int64_t* __restrict__ host) {
     __shared__ int64_t counts[kTabWaves][kCap8];
     __shared__ int32_t freqs[kTabWaves][kCap8];
     __shared__ NpScratch ns[kTabWaves];
@@ -550,7 +558,18 @@ __global__ __launch_bounds__(64 * kTabWaves) void k_chunk_tables_wave(const uint
         }
     }
     tl = wave_sum(tl);
-    if (mx < 0) {   // absent stream (empty coset)
+    if (host && sid == 0) {
+        int32_t all = 0;
+        for (int64_t c = lane; c * LQ_STREAMS < n_streams; c += 64) all |= status[c];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) all |= __shfl_xor(all, o, 64);
+        if (lane == 0) *host = all;
+    }
+    bool out = false;
+    if (skip)
+        for (int64_t c0 = 0; c0 * LQ_STREAMS < n_streams; c0 += 64)
+            out = out || __any((c0 + lane) * LQ_STREAMS < n_streams && (status[c0 + lane] & LQ_ST_SYM_OVERFLOW));
+    if (mx < 0 || out) {   // absent stream (empty coset)
         if (lane == 0) { T->lo = 0; T->n_sym = 0; T->n_symbols = 0; T->status = 0; }
         return;
     }
@@ -878,6 +897,28 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
 // k_chunk_scan + k_chunk_offsets for such batches.
 constexpr int kScanRounds = 32;   // rounds of 64 blocks whose loads are in flight together
 
+// chunk_base[c] = chunk_words[0] + .. + chunk_words[c - 1], by one wave.
+// total (nullable, host memory): the sum of them all.
+__device__ __forceinline__ void chunk_bases(const int64_t* chunk_words, int64_t n_chunks, int64_t* chunk_base, int lane,
+                                            int64_t* total) {
+    int64_t carry = 0;
+    for (int64_t c0 = 0; c0 < n_chunks; c0 += 64) {
+        const int64_t c = c0 + lane;
+        const int64_t v = c < n_chunks ? __hip_atomic_load(chunk_words + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        int64_t incl = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t u = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += u;
+        }
+        if (c < n_chunks) chunk_base[c] = carry + incl - v;
+        carry += __shfl(incl, 63, 64);
+    }
+    if (total && lane == 0) *total = carry;
+}
+
+// chunk_base (nullable; counter is then a cleared word): the workgroup that
+// finishes last also writes the chunks' bases.
 __global__ __launch_bounds__(1024) void k_chunk_scan_offsets(const uint32_t* __restrict__ blk_bits,
                                                              const uint16_t* __restrict__ blk_state,
                                                              const lq_table* __restrict__ tables, int64_t nblk,
@@ -885,7 +926,11 @@ __global__ __launch_bounds__(1024) void k_chunk_scan_offsets(const uint32_t* __r
                                                              int64_t* __restrict__ stream_nbits,
                                                              int32_t* __restrict__ stream_state,
                                                              int64_t* __restrict__ stream_woff,
-                                                             int64_t* __restrict__ chunk_words) {
+                                                             int64_t* __restrict__ chunk_words,
+                                                             int64_t* __restrict__ chunk_base,
+                                                             uint32_t* __restrict__ counter,
+                                                             int64_t* __restrict__ total) {
+    __shared__ int s_last;
     __shared__ int64_t s_nbits[LQ_STREAMS];
     __shared__ int s_present[LQ_STREAMS];
     const int64_t c = blockIdx.x;
@@ -923,8 +968,16 @@ __global__ __launch_bounds__(1024) void k_chunk_scan_offsets(const uint32_t* __r
             stream_woff[c * LQ_STREAMS + k] = w;
             if (s_present[k]) w += (s_nbits[k] + 31) / 32 + 1;
         }
-        chunk_words[c] = w;
+        if (!chunk_base) {
+            chunk_words[c] = w;
+        } else {   // the release orders the count before the counter's step
+            __hip_atomic_store(chunk_words + c, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x;
+        }
     }
+    if (!chunk_base) return;
+    __syncthreads();
+    if (s_last && st == 0) chunk_bases(chunk_words, gridDim.x, chunk_base, lane, total);
 }
 
 // Tiled scan of long streams.  Tile t of stream sid covers blocks
@@ -1007,18 +1060,34 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__
     }
 }
 
-// per chunk: word offset of each present stream (n_words + 1 words each) and chunk total
-__global__ void k_chunk_offsets(const int64_t* __restrict__ stream_nbits, const lq_table* __restrict__ tables,
-                                int64_t n_chunks, int64_t* __restrict__ stream_woff, int64_t* __restrict__ chunk_words) {
-    int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n_chunks) return;
-    int64_t w = 0;
-    for (int st = 0; st < LQ_STREAMS; st++) {
-        int64_t sid = c * LQ_STREAMS + st;
-        stream_woff[sid] = w;
-        if (tables[sid].n_sym > 0) w += (stream_nbits[sid] + 31) / 32 + 1;
+// per chunk: word offset of each present stream (n_words + 1 words each) and
+// chunk total; one workgroup.  chunk_base: nullable.
+__global__ __launch_bounds__(256) void k_chunk_offsets(const int64_t* __restrict__ stream_nbits,
+                                                       const lq_table* __restrict__ tables, int64_t n_chunks,
+                                                       int64_t* __restrict__ stream_woff,
+                                                       int64_t* __restrict__ chunk_words,
+                                                       int64_t* __restrict__ chunk_base,
+                                                       int64_t* __restrict__ total) {
+    for (int64_t c = threadIdx.x; c < n_chunks; c += 256) {
+        int64_t nb[LQ_STREAMS];
+        int ns[LQ_STREAMS];
+#pragma unroll
+        for (int st = 0; st < LQ_STREAMS; st++) {
+            nb[st] = stream_nbits[c * LQ_STREAMS + st];
+            ns[st] = tables[c * LQ_STREAMS + st].n_sym;
+        }
+        int64_t w = 0;
+#pragma unroll
+        for (int st = 0; st < LQ_STREAMS; st++) {
+            stream_woff[c * LQ_STREAMS + st] = w;
+            if (ns[st] > 0) w += (nb[st] + 31) / 32 + 1;
+        }
+        __hip_atomic_store(chunk_words + c, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    chunk_words[c] = w;
+    if (!chunk_base) return;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    if (threadIdx.x < 64) chunk_bases(chunk_words, n_chunks, chunk_base, (int)threadIdx.x, total);
 }
 
 // One wave per (stream, group of 32 blocks).  The group owns the stream
@@ -1965,7 +2034,7 @@ template <typename SymT>
 int encode_launch(const SymT* d_sym, const uint32_t* d_blk_n1, int64_t n_chunks, int64_t n_vectors,
                   const lq_table* d_tables, void* d_work, uint32_t* d_blk_off, uint16_t* d_blk_state,
                   int64_t* d_stream_nbits, int32_t* d_stream_state, int64_t* d_stream_woff, int64_t* d_chunk_words,
-                  hipStream_t s) {
+                  int64_t* d_chunk_base, uint32_t* d_counter, int64_t* h_total, hipStream_t s) {
     if (n_chunks <= 0 || n_vectors <= 0) return LQ_ERR_ARG;
     const int64_t nblk = (n_vectors + kBlk - 1) / kBlk;
     EncWork w = enc_layout(n_chunks, n_vectors);
@@ -1982,26 +2051,173 @@ int encode_launch(const SymT* d_sym, const uint32_t* d_blk_n1, int64_t n_chunks,
         hipLaunchKernelGGL(k_scan_top, dim3((unsigned)(n_chunks * LQ_STREAMS)), dim3(256), 0, s, tsum, tiles, d_blk_state,
                            nblk, d_tables, d_stream_nbits, d_stream_state);
         hipLaunchKernelGGL(k_scan_apply, tg, dim3(256), 0, s, bits, nblk, tiles, tsum, d_blk_off);
-        hipLaunchKernelGGL(k_chunk_offsets, dim3((unsigned)((n_chunks + 63) / 64)), dim3(64), 0, s, d_stream_nbits,
-                           d_tables, n_chunks, d_stream_woff, d_chunk_words);
+        hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(256), 0, s, d_stream_nbits, d_tables, n_chunks, d_stream_woff,
+                           d_chunk_words, d_chunk_base, h_total);
     } else {
         hipLaunchKernelGGL(k_chunk_scan_offsets, dim3((unsigned)n_chunks), dim3(64 * LQ_STREAMS), 0, s, bits,
                            d_blk_state, d_tables, nblk, d_blk_off, d_stream_nbits, d_stream_state, d_stream_woff,
-                           d_chunk_words);
+                           d_chunk_words, d_chunk_base, d_counter, h_total);
     }
     return launch_status();
+}
+
+int tables_launch(const uint32_t* d_hist, int64_t n_chunks, lq_table* d_tables, int32_t* d_status, int skip,
+                  int64_t* h_status, hipStream_t s) {
+    if (n_chunks <= 0) return LQ_ERR_ARG;
+    const int64_t ns = n_chunks * LQ_STREAMS;
+    hipLaunchKernelGGL(k_chunk_tables_wave, dim3((unsigned)((ns + kTabWaves - 1) / kTabWaves)), dim3(64 * kTabWaves), 0,
+                       s, d_hist, ns, d_tables, d_status, skip, h_status);
+    return launch_status();
+}
+
+// What lq_encode_chunks reads back: two words of pinned host memory that the
+// launches write, and an event after the launch that writes the last one.
+// Slots are taken for one call and given back at its end: as many exist as
+// calls were ever under way together on a device (the event's).
+struct ReadSlot {
+    int64_t* host = nullptr;
+    hipEvent_t event = nullptr;
+    int device = -1;
+};
+
+struct ReadPool {
+    std::mutex m;
+    std::vector<ReadSlot> free;
+
+    bool take(ReadSlot* out) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        {
+            std::lock_guard<std::mutex> g(m);
+            for (size_t i = 0; i < free.size(); i++)
+                if (free[i].device == dev) {
+                    *out = free[i];
+                    free.erase(free.begin() + i);
+                    return true;
+                }
+        }
+        ReadSlot s;
+        s.device = dev;
+        if (hipHostMalloc(reinterpret_cast<void**>(&s.host), 2 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
+            return false;
+        if (hipEventCreateWithFlags(&s.event, hipEventDisableTiming) != hipSuccess) {
+            (void)hipHostFree(s.host);
+            return false;
+        }
+        *out = s;
+        return true;
+    }
+    void give(const ReadSlot& s) {
+        std::lock_guard<std::mutex> g(m);
+        free.push_back(s);
+    }
+};
+
+ReadPool& read_pool() {
+    static ReadPool* p = new ReadPool;   // never destroyed: the HIP runtime may be gone by then
+    return *p;
+}
+
+struct WriteWork {   // offsets into lq_encode_chunks' workspace
+    int64_t sums, fastdiv, counter, sym, enc, total;
+};
+
+inline WriteWork write_layout(int64_t n_chunks, int64_t n_heads, int64_t bph) {
+    auto al = [](int64_t b) { return (b + 255) / 256 * 256; };
+    const int64_t H = n_chunks * n_heads, V = n_heads * bph, nblk = (V + kBlk - 1) / kBlk;
+    WriteWork w;
+    w.sums = 0;
+    w.fastdiv = w.sums + al((4096 + H) * 8);
+    w.counter = w.fastdiv + al(H * 4);
+    w.sym = w.counter + 256;
+    w.enc = w.sym + al(n_chunks * nblk * kSymStride);
+    w.total = w.enc + enc_layout(n_chunks, V).total;
+    return w;
 }
 
 }  // namespace
 
 extern "C" {
 
+int64_t lq_encode_chunks_workspace(int64_t n_chunks, int64_t n_heads, int64_t bph) {
+    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0) return -1;
+    return write_layout(n_chunks, n_heads, bph).total;
+}
+
+int lq_encode_chunks(const void* d_x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph, int head_dim,
+                     const float* d_signs, const int64_t* d_dither_seed, const int32_t* d_chunk_bits, int scales_given,
+                     float* d_sigma2, float* d_scale32, uint16_t* d_scale16, uint8_t* d_coset_bits, uint32_t* d_blk_n1,
+                     void* d_deq, uint32_t* d_hist, int32_t* d_status, lq_table* d_tables, uint32_t* d_blk_off,
+                     uint16_t* d_blk_state, int64_t* d_stream_nbits, int32_t* d_stream_state, int64_t* d_stream_woff,
+                     int64_t* d_chunk_words, int64_t* d_chunk_base, uint32_t* d_words, int skip_overflowed, void* d_work,
+                     int64_t* h_status, int64_t* h_words, hipStream_t s) {
+    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || !d_work || !d_status || !d_hist || !d_scale32 || !d_scale16 ||
+        !d_chunk_base || (d_signs && d_deq))
+        return LQ_ERR_ARG;
+    const int64_t H = n_chunks * n_heads, V = n_heads * bph;
+    const WriteWork w = write_layout(n_chunks, n_heads, bph);
+    char* const base = static_cast<char*>(d_work);
+    int32_t* const fastdiv = reinterpret_cast<int32_t*>(base + w.fastdiv);
+    uint32_t* const counter = reinterpret_cast<uint32_t*>(base + w.counter);
+    int8_t* const sym = reinterpret_cast<int8_t*>(base + w.sym);
+    Clear clear;
+    clear.hist = d_hist;
+    clear.n_hist = n_chunks * LQ_STREAMS * 256;
+    clear.status = d_status;
+    clear.n_status = n_chunks;
+    clear.counter = counter;
+    const bool reads = h_status || h_words;
+    ReadSlot slot;
+    if (reads && !read_pool().take(&slot)) return LQ_ERR_LAUNCH;
+    auto run = [&]() -> int {
+        int rc = scales_given
+                     ? scale_fastdiv_launch(d_scale32, H, d_signs ? (int)LQ_F32 : dtype, fastdiv, d_scale16, clear, s)
+                     : head_scales_launch(d_x, dtype, n_chunks, n_heads, bph, head_dim, d_signs, d_chunk_bits,
+                                          reinterpret_cast<double*>(base + w.sums), d_sigma2, d_scale32, d_scale16, fastdiv,
+                                          clear, s);
+        if (rc != LQ_OK) return rc;
+        rc = d_signs ? lq_chunk_quantize_rht(d_x, dtype, n_chunks, n_heads, bph, head_dim, d_signs, d_scale32, sym,
+                                             d_coset_bits, d_blk_n1, d_hist, d_status, d_dither_seed, s)
+                     : lq_chunk_quantize(d_x, dtype, n_chunks, n_heads, bph, d_scale32, fastdiv, sym, d_coset_bits,
+                                         d_blk_n1, d_hist, d_status, d_deq, dtype, d_dither_seed, s);
+        if (rc != LQ_OK) return rc;
+        rc = tables_launch(d_hist, n_chunks, d_tables, d_status, skip_overflowed, reads ? slot.host : nullptr, s);
+        if (rc != LQ_OK) return rc;
+        if (reads && !h_words && hipEventRecord(slot.event, s) != hipSuccess) return LQ_ERR_LAUNCH;
+        rc = encode_launch(sym, d_blk_n1, n_chunks, V, d_tables, base + w.enc, d_blk_off, d_blk_state, d_stream_nbits,
+                           d_stream_state, d_stream_woff, d_chunk_words, d_chunk_base, counter,
+                           h_words ? slot.host + 1 : nullptr, s);
+        if (rc != LQ_OK) return rc;
+        if (h_words && hipEventRecord(slot.event, s) != hipSuccess) return LQ_ERR_LAUNCH;
+        if (d_words)
+            rc = lq_chunk_pack(n_chunks, V, d_tables, base + w.enc, d_blk_off, d_stream_nbits, d_stream_woff, d_chunk_base,
+                               d_words, s);
+        if (rc != LQ_OK || !reads) return rc;
+        // the launches behind the event go on while the caller reads on
+        if (hipEventSynchronize(slot.event) != hipSuccess) return LQ_ERR_LAUNCH;
+        if (h_status) *h_status = slot.host[0];
+        if (h_words) *h_words = slot.host[1];
+        return LQ_OK;
+    };
+    const int rc = run();
+    if (reads) {
+        if (rc != LQ_OK) (void)hipStreamSynchronize(s);   // no launch may still write the slot
+        read_pool().give(slot);
+    }
+    return rc;
+}
+
+int lq_encode_chunks_pack(int64_t n_chunks, int64_t n_heads, int64_t bph, const lq_table* d_tables, const void* d_work,
+                          const uint32_t* d_blk_off, const int64_t* d_stream_nbits, const int64_t* d_stream_woff,
+                          const int64_t* d_chunk_base, uint32_t* d_words, hipStream_t s) {
+    if (n_chunks <= 0 || n_heads <= 0 || bph <= 0 || !d_work || !d_words) return LQ_ERR_ARG;
+    const WriteWork w = write_layout(n_chunks, n_heads, bph);
+    return lq_chunk_pack(n_chunks, n_heads * bph, d_tables, static_cast<const char*>(d_work) + w.enc, d_blk_off,
+                         d_stream_nbits, d_stream_woff, d_chunk_base, d_words, s);
+}
+
 int lq_chunk_tables(const uint32_t* d_hist, int64_t n_chunks, lq_table* d_tables, int32_t* d_status, hipStream_t s) {
-    if (n_chunks <= 0) return LQ_ERR_ARG;
-    const int64_t ns = n_chunks * LQ_STREAMS;
-    hipLaunchKernelGGL(k_chunk_tables_wave, dim3((unsigned)((ns + kTabWaves - 1) / kTabWaves)), dim3(64 * kTabWaves), 0,
-                       s, d_hist, ns, d_tables, d_status);
-    return launch_status();
+    return tables_launch(d_hist, n_chunks, d_tables, d_status, 0, nullptr, s);
 }
 
 int64_t lq_chunk_encode_workspace(int64_t n_chunks, int64_t n_vectors) {
@@ -2014,7 +2230,7 @@ int lq_chunk_encode(const int8_t* d_sym, const uint32_t* d_blk_n1, int64_t n_chu
                     int64_t* d_stream_nbits, int32_t* d_stream_state, int64_t* d_stream_woff, int64_t* d_chunk_words,
                     hipStream_t s) {
     return encode_launch(d_sym, d_blk_n1, n_chunks, n_vectors, d_tables, d_work, d_blk_off, d_blk_state, d_stream_nbits,
-                         d_stream_state, d_stream_woff, d_chunk_words, s);
+                         d_stream_state, d_stream_woff, d_chunk_words, nullptr, nullptr, nullptr, s);
 }
 
 int lq_chunk_encode_wide(const int16_t* d_sym, const uint32_t* d_blk_n1, int64_t n_chunks, int64_t n_vectors,
@@ -2022,7 +2238,7 @@ int lq_chunk_encode_wide(const int16_t* d_sym, const uint32_t* d_blk_n1, int64_t
                          int64_t* d_stream_nbits, int32_t* d_stream_state, int64_t* d_stream_woff, int64_t* d_chunk_words,
                          hipStream_t s) {
     return encode_launch(d_sym, d_blk_n1, n_chunks, n_vectors, d_tables, d_work, d_blk_off, d_blk_state, d_stream_nbits,
-                         d_stream_state, d_stream_woff, d_chunk_words, s);
+                         d_stream_state, d_stream_woff, d_chunk_words, nullptr, nullptr, nullptr, s);
 }
 
 int lq_chunk_tables_wide(const uint32_t* d_hist, const int32_t* d_minmax, int64_t n_chunks, lq_table* d_tables,

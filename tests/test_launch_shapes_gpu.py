@@ -182,3 +182,73 @@ def test_stream_decoder_truncated_gpu():
                     x = (x << 1) | (int(words[q >> 5]) >> (q & 31) & 1)
                 pos += max(k, 0)
         assert np.array_equal(got, np.array(want)), (nb, st, n)
+
+
+@pytest.mark.parametrize("C,T", [(1, 40), (3, 1100), (70, 64), (2, 16400)])
+@pytest.mark.parametrize("wide", ["auto", False])
+@pytest.mark.parametrize("arena", ["own", "bound", "given"])
+def test_write_call_sizes_gpu(C, T, wide, arena):
+    """The write's one native call: chunk bases and total (one workgroup and
+    the tiled scan of long streams, more chunks than a wave's lanes), in an
+    arena of its exact size, at the bound, and the caller's."""
+    from latticequant_amd import codec
+    x = _x(C, 8, T, 128, C * T)
+    given = torch.full((codec.words_bound(C, 8 * T * 16),), -7, dtype=torch.int32, device="cuda")
+    kw = {"own": {}, "bound": {"exact_size": False}, "given": {"words_out": given}}[arena]
+    enc, _ = codec.encode_batch(x, 4, wide=wide, **kw)
+    cw = enc.chunk_words.cpu()
+    assert torch.equal(enc.chunk_base.cpu(), torch.cumsum(cw, 0) - cw)
+    total = int(cw.sum())
+    if arena == "own":
+        assert enc.words.numel() == total + 2
+    if arena == "given":
+        assert enc.words.data_ptr() == given.data_ptr() and bool((given[total:] == -7).all())
+    c = C - 1
+    ch = O.compress_chunk(x[c].cpu().numpy(), 4, scales_f32=enc.scale32.view(C, -1)[c].cpu().numpy())
+    base = int(enc.chunk_base[c])
+    assert np.array_equal(enc.words[base:base + int(cw[c])].cpu().numpy().view(np.uint32), ch.bitstream)
+    given_scales, _ = codec.encode_batch(x, 4, scale32=enc.scale32, wide=wide)
+    assert torch.equal(given_scales.words[:total], enc.words[:total])
+    assert torch.equal(given_scales.scale16, enc.scale16)
+
+
+def test_write_call_overflow_leaves_arena_gpu():
+    """One chunk of three outside int8: the batch is coded once, on int16
+    symbols; words past its bitstreams are not touched."""
+    from latticequant_amd import codec
+    x = _x(3, 2, 600, 128, 3)
+    x[1, 0, 0, :, 0] *= 400.0
+    bound = codec.words_bound(3, 2 * 600 * 16)
+    given = torch.full((bound,), -7, dtype=torch.int32, device="cuda")
+    enc, _ = codec.encode_batch(x, 5, words_out=given)
+    assert enc.extra["wide"]
+    ref, _ = codec.encode_batch(x, 5, wide=True)
+    total = int(ref.chunk_words.sum())
+    assert torch.equal(enc.chunk_words, ref.chunk_words)
+    assert torch.equal(given[:total], ref.words[:total]) and bool((given[total:] == -7).all())
+    assert torch.equal(codec.decode_batch(enc), codec.decode_batch(ref))
+
+
+def test_write_call_threads_gpu():
+    """Calls from several threads on their own streams, each with its read-back."""
+    import threading
+    from latticequant_amd import codec
+    xs = [_x(2, 4, 300 + 7 * i, 128, i) for i in range(6)]
+    want = [codec.encode_batch(x, 4)[0] for x in xs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(8):
+                e, _ = codec.encode_batch(xs[i], 4)
+                s.synchronize()
+                if not (torch.equal(e.words[:-2], want[i].words[:-2]) and torch.equal(e.chunk_base, want[i].chunk_base)):
+                    bad.append(i)
+        s.synchronize()
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad

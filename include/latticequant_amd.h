@@ -141,6 +141,17 @@ int lq_quantize_deq(const void *d_x, int dtype, int64_t n_chunks, int64_t n_head
                     const int32_t *d_chunk_bits, void *d_work, float *d_sigma2, float *d_scale32,
                     uint16_t *d_scale16, void *d_deq, hipStream_t s);
 
+/* A decode step's update of one layer in one launch: K and V (n_heads * bph
+ * contiguous vectors each, bph <= 1023, 16-byte aligned) get the scales of
+ * lq_head_scales at bits_k / bits_v (K's n_heads, then V's, in d_sigma2,
+ * d_scale32, d_scale16) and their dequantised rows q * scale32 are written in
+ * x's dtype to d_out_k / d_out_v, head h's vectors from h * stride (vectors);
+ * d_rows receives a copy of K's vectors, then V's.
+ * Replaces llm/compressed_kv_cache.py:188-221 and the append of :384-395. */
+int lq_update_small(const void *d_k, const void *d_v, int dtype, int64_t n_heads, int64_t bph, int bits_k, int bits_v,
+                    void *d_rows, float *d_sigma2, float *d_scale32, uint16_t *d_scale16, void *d_out_k,
+                    int64_t stride_k, void *d_out_v, int64_t stride_v, hipStream_t s);
+
 /* Rotated rows: lq_chunk_quantize of w = RHT(x) (as lq_head_scales_rht), the
  * rotation in registers, the scale division rounded as IEEE division, optional dither; no
  * dequantised output.  Same outputs and layouts as lq_chunk_quantize on a

@@ -387,6 +387,28 @@ def quantize_deq(x: torch.Tensor, bits, scratch: QuantizeScratch):
     return scale32, scale16, deq, sigma2
 
 
+UPDATE_MAX_BPH = 1023   # vectors per head of lq_update_small
+
+
+def update_small(k: torch.Tensor, v: torch.Tensor, bits_k: int, bits_v: int, out_k: torch.Tensor, out_v: torch.Tensor):
+    """K and V of one layer's small update (contiguous (B, H, T, hd), 16-byte
+    aligned, T * hd / 8 <= UPDATE_MAX_BPH) quantized in one launch
+    (lq_update_small): the dequantised rows go to out_k / out_v ((B, H, T, hd)
+    views of buffers whose heads are equally spaced).  Returns (rows: a copy of
+    both, (2, B, H, T, hd); scale32, scale16, sigma2 of K's heads, then V's)."""
+    B, H, T, hd = k.shape
+    n = 2 * B * H
+    rows = torch.empty((2, B, H, T, hd), dtype=k.dtype, device=k.device)
+    sc = torch.empty(3 * n, dtype=torch.float32, device=k.device)   # as quantize_deq
+    at = sc.data_ptr()
+    L.check(L.lib().lq_update_small(k.data_ptr(), v.data_ptr(), L.dtype_code(k.dtype), B * H, T * hd // 8, bits_k, bits_v,
+                                    rows.data_ptr(), at, at + 4 * n, at + 8 * n, out_k.data_ptr(),
+                                    out_k.stride(1) // 8, out_v.data_ptr(), out_v.stride(1) // 8,
+                                    L.stream_ptr(k.device)), "lq_update_small")
+    sigma2, scale32, s16 = sc.split(n)
+    return rows, scale32, s16.view(torch.float16)[:n], sigma2
+
+
 def quantize_points(t: torch.Tensor, bits, scale32: Optional[torch.Tensor] = None):
     """Lattice points of one (B, H, T, hd) tensor as _compress_tensor computes
     them (x / scale[head] -> E8).  Returns (q (B*H*T*hd/8, 8) fp32, scale32, scale16)."""

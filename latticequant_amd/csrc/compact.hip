@@ -173,7 +173,8 @@ __global__ __launch_bounds__(256) void k_compact_sumsq(const void* __restrict__ 
     const int64_t wg = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, n_wg = (int64_t)gridDim.x * gridDim.y;
     for (int64_t i = wg * 256 + threadIdx.x; i < n_clear; i += n_wg * 256) clear[i] = 0ull;
     if (wg == 0 && threadIdx.x == 0) *extra = 0;
-    head_sumsq_part<false>(x, dtype, bph, parts, blockIdx.x, blockIdx.y, work, red, nullptr, 1, 1.0f);
+    const double sum = head_sumsq_part<false>(x, dtype, bph, parts, blockIdx.x, blockIdx.y, red, nullptr, 1, 1.0f);
+    if (threadIdx.x == 0) work[(int64_t)blockIdx.x * parts + blockIdx.y] = sum;
 }
 
 // One tile of kTile blocks per workgroup; ranks from the tile offset plus

@@ -102,7 +102,9 @@ __global__ void k_head_sumsq(const void* __restrict__ x, int dtype, int64_t vec_
     __shared__ double red[256];
     clear_words(clear, ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x,
                 (int64_t)gridDim.x * gridDim.y * blockDim.x);
-    head_sumsq_part<ROT, LPR>(x, dtype, vec_per_head, parts, blockIdx.x, blockIdx.y, work, red, signs, lpr, rdiv);
+    const double sum = head_sumsq_part<ROT, LPR>(x, dtype, vec_per_head, parts, blockIdx.x, blockIdx.y, red, signs, lpr,
+                                                 rdiv);
+    if (threadIdx.x == 0) work[(int64_t)blockIdx.x * parts + blockIdx.y] = sum;
 }
 
 __device__ void fastdiv_check(float s, int32_t* word) {
@@ -147,6 +149,55 @@ __global__ void k_scale_fastdiv(const float* __restrict__ scale32, int dtype, in
         fastdiv_check(scale32[h], fastdiv + h);
     } else if (threadIdx.x == 0) {
         fastdiv[h] = 0;
+    }
+}
+
+// ---------------------------------------------------------- small updates --
+
+// A decode step's update of one layer, K and V in one launch, one workgroup per
+// head: the head's scale (the sums and formula of lq_head_scales with one part
+// per head), the dequantised rows q * scale32 written where attention reads
+// them, and a copy of the rows for the entropy coder.  A few vectors per head:
+// launches bound it, six of them (stack, sums, finalisation, quantizer, two
+// appends: about 20 us of kernels) before.  The rows are divided with IEEE
+// division: for so few of them the check behind the fast division costs more.
+constexpr int64_t kUpdateMaxBph = 1023;   // head_parts gives one part below 1024 vectors per head
+
+__global__ __launch_bounds__(256) void k_update_small(const void* __restrict__ k, const void* __restrict__ v, int dtype,
+                                                      int64_t n_heads, int64_t bph, int bits_k, int bits_v,
+                                                      void* __restrict__ rows, float* __restrict__ sigma2,
+                                                      float* __restrict__ scale32, uint16_t* __restrict__ scale16,
+                                                      void* __restrict__ out_k, int64_t stride_k,
+                                                      void* __restrict__ out_v, int64_t stride_v) {
+    __shared__ double red[256];
+    __shared__ float sc;
+    const int64_t h = blockIdx.x;
+    const bool is_v = h >= n_heads;
+    const int64_t hh = is_v ? h - n_heads : h;
+    const void* const x = is_v ? v : k;
+    const double sum = head_sumsq_part<false>(x, dtype, bph, 1, hh, 0, red, nullptr, 1, 1.0f);
+    if (threadIdx.x == 0) {
+        float s2;
+        const float s = head_scale(sum, bph * 8, is_v ? bits_v : bits_k, &s2);
+        sigma2[h] = s2;
+        scale32[h] = s;
+        scale16[h] = f2h(s);
+        sc = s;
+    }
+    __syncthreads();
+    const float s = sc;
+    void* const out = is_v ? out_v : out_k;
+    const int64_t o0 = hh * (is_v ? stride_v : stride_k);
+    for (int64_t i = threadIdx.x; i < bph; i += 256) {
+        float xv[8], t[8], q[8];
+        load8(x, dtype, hh * bph + i, xv);
+        store8(rows, dtype, h * bph + i, xv);   // exact: the values are dtype's
+#pragma unroll
+        for (int j = 0; j < 8; j++) t[j] = xv[j] / s;
+        const float off = e8_nearest_fast(t, q) ? 0.5f : 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) q[j] = (q[j] + off) * s;
+        store8(out, dtype, o0 + i, q);
     }
 }
 
@@ -700,6 +751,21 @@ int lq_quantize_deq(const void* d_x, int dtype, int64_t n_chunks, int64_t n_head
     if (rc != LQ_OK) return rc;
     return lq_chunk_quantize(d_x, dtype, n_chunks, n_heads, bph, d_scale32, fastdiv, sym, coset, n1, hist, status,
                              d_deq, dtype, nullptr, s);
+}
+
+int lq_update_small(const void* d_k, const void* d_v, int dtype, int64_t n_heads, int64_t bph, int bits_k, int bits_v,
+                    void* d_rows, float* d_sigma2, float* d_scale32, uint16_t* d_scale16, void* d_out_k,
+                    int64_t stride_k, void* d_out_v, int64_t stride_v, hipStream_t s) {
+    if (!d_k || !d_v || !d_rows || !d_sigma2 || !d_scale32 || !d_scale16 || !d_out_k || !d_out_v || n_heads <= 0 ||
+        bph <= 0 || bph > kUpdateMaxBph || stride_k < bph || stride_v < bph || dtype < 0 || dtype > 2)
+        return LQ_ERR_ARG;
+    const uintptr_t at = reinterpret_cast<uintptr_t>(d_k) | reinterpret_cast<uintptr_t>(d_v) |
+                         reinterpret_cast<uintptr_t>(d_rows) | reinterpret_cast<uintptr_t>(d_out_k) |
+                         reinterpret_cast<uintptr_t>(d_out_v);
+    if (at & 15) return LQ_ERR_ARG;
+    hipLaunchKernelGGL(k_update_small, dim3((unsigned)(2 * n_heads)), dim3(256), 0, s, d_k, d_v, dtype, n_heads, bph, bits_k,
+                       bits_v, d_rows, d_sigma2, d_scale32, d_scale16, d_out_k, stride_k, d_out_v, stride_v);
+    return launch_status();
 }
 
 // Rotated rows (head_dim a power of two in [8, 128], bph a multiple of

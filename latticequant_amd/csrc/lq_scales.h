@@ -39,10 +39,11 @@ __device__ __forceinline__ float sq_vec16(const u32x4 w, bool f16) {
 // holding w, so the scales equal those of the materialised rotation.
 // One (head h, part p) on a 256-thread workgroup; red: 256 doubles of LDS.
 // LPR > 0: lpr as a compile-time constant (straight-line butterfly stages).
+// Returns the sum in every thread.
 template <bool ROT, int LPR = 0>
-__device__ __forceinline__ void head_sumsq_part(const void* __restrict__ x, int dtype, int64_t vec_per_head,
-                                                int parts, int64_t h, int p, double* __restrict__ work, double* red,
-                                                const float* __restrict__ signs, int lpr, float rdiv) {
+__device__ __forceinline__ double head_sumsq_part(const void* __restrict__ x, int dtype, int64_t vec_per_head,
+                                                  int parts, int64_t h, int p, double* red,
+                                                  const float* __restrict__ signs, int lpr, float rdiv) {
     int64_t per = (vec_per_head + parts - 1) / parts;
     if (ROT) per = (per + lpr - 1) / lpr * lpr;
     int64_t v0 = (int64_t)p * per, v1 = v0 + per < vec_per_head ? v0 + per : vec_per_head;
@@ -105,7 +106,7 @@ __device__ __forceinline__ void head_sumsq_part(const void* __restrict__ x, int 
         if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) work[h * parts + p] = red[0];
+    return red[0];
 }
 
 // w[0] + w[1] + .. + w[parts - 1] in that order (one rounding order for every

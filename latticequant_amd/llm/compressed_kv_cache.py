@@ -294,6 +294,9 @@ def _get_placeholder(device, dtype=torch.bfloat16):
     return _PLACEHOLDER
 
 
+_DIRECT_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+
+
 class _Resident:
     """Growable (B, H, cap, hd) buffer of decompressed tokens; view() is [:, :, :T]."""
 
@@ -302,7 +305,8 @@ class _Resident:
         self.buf = torch.empty((B, H, max(2 * T, 16), hd), dtype=like.dtype, device=like.device)
         self.T = 0
 
-    def append(self, t: torch.Tensor):
+    def room(self, t: torch.Tensor) -> torch.Tensor:
+        """The view the next t.shape[2] tokens go to (the buffer grown if needed)."""
         B, H, T, hd = t.shape
         if self.T + T > self.buf.shape[2] or self.buf.shape[0] != B or self.buf.shape[1] != H:
             if self.buf.shape[0] != B or self.buf.shape[1] != H or self.buf.shape[3] != hd:
@@ -311,8 +315,16 @@ class _Resident:
             nb = torch.empty((B, H, cap, hd), dtype=self.buf.dtype, device=self.buf.device)
             nb[:, :, :self.T].copy_(self.buf[:, :, :self.T])
             self.buf = nb
-        self.buf[:, :, self.T:self.T + T].copy_(t)
-        self.T += T
+        return self.buf[:, :, self.T:self.T + T]
+
+    def append(self, t: torch.Tensor):
+        self.room(t).copy_(t)
+        self.T += t.shape[2]
+
+    def holds(self, t: torch.Tensor) -> bool:
+        """Whether t's rows can be written into the buffer as they are."""
+        b, s = self.buf.shape, t.shape
+        return b[0] == s[0] and b[1] == s[1] and b[3] == s[3] and self.buf.dtype == t.dtype and self.buf.device == t.device
 
     def view(self) -> torch.Tensor:
         return self.buf[:, :, :self.T]
@@ -369,12 +381,7 @@ class CompressedKVCache(DynamicCache):
         pend = None
         if not self.eval_only_no_entropy and n_vectors <= self.DEFER_MAX_VECTORS:
             scale32, scale16, deq, sigma2 = codec.quantize_deq(x, bits, self._qscratch)
-            key = (tuple(x.shape[1:]), x.dtype, x.device)
-            grp = self._groups.get(key)
-            if grp is None or grp.full(self.DEFER_CHUNKS):
-                if grp is not None:
-                    self._flush_group(grp)
-                grp = self._groups[key] = _DeferredGroup()
+            grp = self._open_group((tuple(x.shape[1:]), x.dtype, x.device))
             i0 = grp.add(x, bits, scale32, sigma2)
             per = scale16.view(len(tensors), -1)
             out = []
@@ -405,6 +412,48 @@ class CompressedKVCache(DynamicCache):
         if pend is not None:
             self._pending.append((pend, chunks))
         return out
+
+    def _update_direct(self, k: torch.Tensor, v: torch.Tensor, layer_idx: int, bk: int, bv: int):
+        """_compress_many([k, v]) of a small update and its append in one launch
+        (codec.update_small), the dequantised rows written straight into the
+        layer's buffers.  Returns the two chunks, or None where the call is not
+        of that form: entropy coding off, different element types or devices, a
+        head of 1024 vectors or more, an update too large to be deferred, rows
+        that do not start on 16 bytes or buffers of another form."""
+        B, H, T, hd = k.shape
+        bph, nh = T * hd // 8, B * H
+        if (self.eval_only_no_entropy or hd % 8 or bph > codec.UPDATE_MAX_BPH or bph * nh == 0
+                or bph * nh > self.DEFER_MAX_VECTORS or k.dtype != v.dtype or k.device != v.device or not k.is_cuda
+                or k.dtype not in _DIRECT_DTYPES):
+            return None
+        have = layer_idx < len(self._resident_k) and self._resident_k[layer_idx] is not None
+        rk = self._resident_k[layer_idx] if have else _Resident(k)
+        rv = self._resident_v[layer_idx] if have else _Resident(v)
+        if not rk.holds(k) or not rv.holds(v):
+            return None
+        kc, vc = k.contiguous(), v.contiguous()
+        if (kc.data_ptr() | vc.data_ptr()) & 15:
+            return None
+        rows, scale32, scale16, sigma2 = codec.update_small(kc, vc, bk, bv, rk.room(kc), rv.room(vc))
+        rk.T += T
+        rv.T += T
+        grp = self._open_group((tuple(k.shape), k.dtype, k.device))
+        i0 = grp.add(rows, bk if bk == bv else [bk, bv], scale32, sigma2)
+        per = scale16.view(2, -1)
+        chunks = [OptimizedChunk(None, i0 + i, per[i], k.shape, nh * bph, nh, bph, b, k.dtype, pending=grp)
+                  for i, b in enumerate((bk, bv))]
+        grp.chunks.extend(chunks)
+        self.total_vectors += 2 * nh * bph
+        return chunks[0], chunks[1], rk, rv
+
+    def _open_group(self, key) -> "_DeferredGroup":
+        """The open group of small updates of one (shape, dtype, device)."""
+        grp = self._groups.get(key)
+        if grp is None or grp.full(self.DEFER_CHUNKS):
+            if grp is not None:
+                self._flush_group(grp)
+            grp = self._groups[key] = _DeferredGroup()
+        return grp
 
     # small (untracked) pending batches are settled together once this many
     # are pending, or once they keep this many device bytes alive
@@ -482,7 +531,12 @@ class CompressedKVCache(DynamicCache):
             self._settle_ready()
         self._last_layer = layer_idx
         bk, bv = self._layer_bits(layer_idx)
+        direct = None
         if key_states.shape == value_states.shape:
+            direct = self._update_direct(key_states, value_states, layer_idx, bk, bv)
+        if direct is not None:
+            comp_k, comp_v, rk, rv = direct
+        elif key_states.shape == value_states.shape:
             (comp_k, k_new), (comp_v, v_new) = self._compress_many([key_states, value_states],
                                                                    bk if bk == bv else [bk, bv])
         else:
@@ -511,11 +565,14 @@ class CompressedKVCache(DynamicCache):
             self._comp_values[layer_idx] = CompressedKVLayer()
         self._comp_keys[layer_idx].append_chunk(comp_k)
         self._comp_values[layer_idx].append_chunk(comp_v)
-        if self._resident_k[layer_idx] is None:
-            self._resident_k[layer_idx] = _Resident(k_new)
-            self._resident_v[layer_idx] = _Resident(v_new)
-        self._resident_k[layer_idx].append(k_new)
-        self._resident_v[layer_idx].append(v_new)
+        if direct is not None:
+            self._resident_k[layer_idx], self._resident_v[layer_idx] = rk, rv
+        else:
+            if self._resident_k[layer_idx] is None:
+                self._resident_k[layer_idx] = _Resident(k_new)
+                self._resident_v[layer_idx] = _Resident(v_new)
+            self._resident_k[layer_idx].append(k_new)
+            self._resident_v[layer_idx].append(v_new)
         k_full = self._resident_k[layer_idx].view()
         v_full = self._resident_v[layer_idx].view()
         self.key_cache[layer_idx] = k_full

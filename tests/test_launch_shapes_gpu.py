@@ -252,3 +252,51 @@ def test_write_call_threads_gpu():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,hd,steps", [
+    (1, 8, 128, [1, 1, 1, 5, 1, 1, 16, 1]),      # decode steps, buffers growing
+    (2, 3, 64, [127, 1, 128, 1]),                # 1016 vectors per head, then 1024: the general path between
+    (1, 1, 8, [1, 2, 1000, 1023, 1024, 1]),      # one vector per token, up to the limit and past it
+    (3, 2, 24, [7, 1, 340]),                     # head_dim not a power of two
+])
+def test_direct_updates_gpu(B, H, hd, steps, dtype, monkeypatch):
+    """update()'s one-launch form against the general one (quantize, then
+    append): rows, scales, sigma^2 and bitstreams, with K and V at their own
+    rates, from contiguous, transposed and misaligned tensors, zero heads."""
+    from latticequant_amd.allocation.eval_alloc import VariableRateKVCache
+    g = torch.Generator().manual_seed(hd)
+    kv = []
+    for i, T in enumerate(steps):
+        t = torch.randn(2, B, H, T, hd, generator=g) * 3.0
+        t[:, 0, 0] *= 0.0 if i == 1 else 1.0
+        t[1, :, -1] *= 1e-4
+        t = t.to(dtype).cuda()
+        k, v = t[0], t[1]
+        if i % 3 == 1:      # as attention layers hand them over: (B, T, H, hd) transposed
+            k, v = (a.transpose(1, 2).contiguous().transpose(1, 2) for a in (k, v))
+        if i % 3 == 2:      # rows that start 2 or 4 bytes past a 16-byte boundary
+            k = torch.cat([k.new_zeros(1), k.reshape(-1)])[1:].view(k.shape)
+        kv.append((k, v))
+
+    def fill(direct):
+        if not direct:
+            monkeypatch.setattr(VariableRateKVCache, "_update_direct", lambda *a: None)
+        c = VariableRateKVCache([{"K": 3, "V": 5}, {"K": 4, "V": 4}], eval_only_no_entropy=False)
+        outs = []
+        for k, v in kv:
+            for layer in range(2):
+                outs.append([t.clone() for t in c.update(k, v, layer)])
+        return c, outs
+
+    a, oa = fill(True)
+    b, ob = fill(False)
+    for (ka, va), (kb, vb) in zip(oa, ob):
+        assert torch.equal(ka, kb) and torch.equal(va, vb)
+    assert a.total_vectors == b.total_vectors and a.compressed_bytes() == b.compressed_bytes()
+    for la, lb in zip(a._layers(), b._layers()):
+        for ca, cb in zip(la.chunks, lb.chunks):
+            assert torch.equal(ca.gpu_bitstream, cb.gpu_bitstream) and torch.equal(ca.coset_packed, cb.coset_packed)
+            assert torch.equal(ca.scales, cb.scales) and torch.equal(ca.encoded.sigma2, cb.encoded.sigma2)
+            assert torch.equal(a._decompress_chunk(ca), b._decompress_chunk(cb))

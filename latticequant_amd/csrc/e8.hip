@@ -585,7 +585,8 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
 // [min, min + 1023] of each stream (a stream whose max exceeds the window has
 // an alphabet beyond L and is flagged by the table stage).  Workgroup: 16
 // blocks x 16 streams of one chunk, one lane per (block, stream) column, read
-// 16 symbols (32 bytes) at a time with the next chunk's loads in flight.
+// 16 symbols (32 bytes) at a time with four chunks' loads in flight (4096
+// blocks: 37.3 us with one chunk ahead under a condition, TBD so).
 // Counts accumulate in LDS as 16-bit halves, two bins per word (a bin counts
 // at most 16 x 512 symbols of a workgroup), and are added to hist once.
 constexpr int kHBlocks = 16;
@@ -611,17 +612,24 @@ __global__ __launch_bounds__(256) void k_chunk_hist_wide(const int16_t* __restri
         const int16_t* col = sym + (chunk * nblk + g) * (int64_t)kSymStride + sym_region(c, n0) + 16 * idx;
         uint32_t* hs = sh + st * (LQ_L / 2);
         const int nk = (n + 15) >> 4;   // column chunks (the last one may be partial)
-        Chunk16<int16_t> cur = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)}, nxt = cur;
-        if (nk > 0) cur = gload_chunk(col);
-        for (int k = 0; k < nk; k++) {
-            if (k + 1 < nk) nxt = gload_chunk(col + 128 * (int64_t)(k + 1));
-            const int m = n - 16 * k < 16 ? n - 16 * k : 16;
+        // kDeep chunks in flight, reloaded in place once counted; the loads are
+        // unconditional (past the last chunk: the last again), see for_each_rev
+        constexpr int kDeep = 4;
+        auto at = [&](int k) { return gload_chunk(col + 128 * (k < nk ? k : (nk > 0 ? nk - 1 : 0))); };
+        Chunk16<int16_t> buf[kDeep];
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int v = cur.get(i) - lo;
-                if (i < m && (unsigned)v < (unsigned)LQ_L) atomicAdd(hs + (v >> 1), 1u << ((v & 1) * 16));
+        for (int j = 0; j < kDeep; j++) buf[j] = at(j);
+        for (int k0 = 0; __any(k0 < nk); k0 += kDeep) {
+#pragma unroll
+            for (int j = 0; j < kDeep; j++) {
+                const int m = n - 16 * (k0 + j);
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int v = buf[j].get(i) - lo;
+                    if (i < m && (unsigned)v < (unsigned)LQ_L) atomicAdd(hs + (v >> 1), 1u << ((v & 1) * 16));
+                }
+                buf[j] = at(k0 + j + kDeep);
             }
-            cur = nxt;
         }
     }
     __syncthreads();

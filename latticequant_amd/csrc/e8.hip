@@ -586,7 +586,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
 // an alphabet beyond L and is flagged by the table stage).  Workgroup: 16
 // blocks x 16 streams of one chunk, one lane per (block, stream) column, read
 // 16 symbols (32 bytes) at a time with four chunks' loads in flight (4096
-// blocks: 37.3 us with one chunk ahead under a condition, TBD so).
+// blocks: 37.3 us with one chunk ahead under a condition, 30.3 so).
 // Counts accumulate in LDS as 16-bit halves, two bins per word (a bin counts
 // at most 16 x 512 symbols of a workgroup), and are added to hist once.
 constexpr int kHBlocks = 16;

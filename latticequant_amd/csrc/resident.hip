@@ -378,15 +378,11 @@ struct TileRaw {
     uint2 vb;               // their low bytes
     uint4 vs;               // fp16 scales of those 8 tokens
     uint4 meta;             // lanes 0..3: block metadata of K block 0, 1, V block 0, 1
+    uint2 mask;             // lanes 0..15: exception masks, groups 0..3 of K block 0, 1, V block 0, 1
 };
 
-// a block's exception header and base from the tile's meta registers
-// (i = 0, 1: K blocks, 2, 3: V blocks); wave-uniform
-__device__ __forceinline__ uint64_t meta_hdr(const TileRaw& d, int i) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.meta.x, i);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.meta.y, i);
-    return (uint64_t)lo | ((uint64_t)hi << 32);
-}
+// a block's first exception entry, from the tile's meta registers (i = 0, 1: K
+// blocks, 2, 3: V blocks); wave-uniform
 __device__ __forceinline__ uint32_t meta_base(const TileRaw& d, int i) {
     return (uint32_t)__builtin_amdgcn_readlane((int)d.meta.z, i);
 }
@@ -421,6 +417,9 @@ __device__ __forceinline__ void tile_load(const AttnArgs& A, int64_t kvh, int64_
         const int i = lane & 3;
         const uint32_t* mp = ((i & 2) ? A.v.meta : A.k.meta) + rb0 * 4;
         d.meta = *reinterpret_cast<const uint4*>(mp + (i & 1) * dblk * 4);
+        const int j = lane & 15;
+        const uint64_t* xp = ((j & 8) ? A.v.mask : A.k.mask) + rb0 * 4;
+        d.mask = *reinterpret_cast<const uint2*>(xp + ((j >> 2) & 1) * dblk * 4 + (j & 3));
     }
     const int n = lane & 15, k8 = lane >> 4;
     // records of vector n of tokens 8 k8 .. 8 k8 + 7: block k8 / 2 of the tile
@@ -432,51 +431,45 @@ __device__ __forceinline__ void tile_load(const AttnArgs& A, int64_t kvh, int64_
     d.vs = *reinterpret_cast<const uint4*>(A.v.scale + hb * kRB + tb0 + (uint32_t)((k8 >> 1) * dblk * 16 + 8 * (k8 & 1)));
 }
 
-// exception k of a block (0 <= k < count): slot | group << 6 from the header,
-// or, past the header's seven entries, from the block's masks; -1 past the end
-__device__ __forceinline__ int exc_code(const lq_resident& r, int64_t rb, uint64_t hdr, int k) {
-    if (k < 7) return (int)((hdr >> (8 * (k + 1))) & 0xffu);
-    int before = 0;
-    for (int c = 0; c < 4; c++) {
-        unsigned long long m = r.mask[rb * 4 + c];
-        const int pc = __popcll(m);
-        if (k < before + pc) {
-            for (int q = before; q < k; q++) m &= m - 1ull;
-            return (__ffsll((long long)m) - 1) | (c << 6);
-        }
-        before += pc;
-    }
-    return -1;
-}
+// Exceptions (vectors outside the 5-bit range, whose records are zero) are
+// patched from the exception list, all lanes of a block at once: a block's
+// entries lie in (group, slot) order from its base, so an entry's index is the
+// base plus the set bits of the block's masks before it, and each group of
+// entries is one load instruction.  With outlier channels several vectors of
+// every token are exceptions; taking them one after the other, each with its
+// own memory latency, made the step 168 us at 32768 tokens with 5.5 % of the
+// vectors (C2's channels: four of 128, x10), 25.9 us now; 22.9 us without any.
 
 // Scores of block x: s += q . k over the four record groups, each group's K
-// operand decoded (and, rarely, patched with exception entries) just before
-// its MFMA, so that only one group's pairs are live at a time.
-__device__ __forceinline__ void tile_k(const AttnArgs& A, const TileRaw& d, int64_t rb, int x, int lane,
-                                       const h8_t qa[4], f4_t& s) {
-    const uint64_t hdr = meta_hdr(d, x);
-    const int n = (int)(hdr & 0xffu);
+// operand decoded (and patched with exception entries) just before its MFMA,
+// so that only one group's pairs are live at a time.
+__device__ __forceinline__ void tile_k(const AttnArgs& A, const TileRaw& d, int x, int lane, const h8_t qa[4], f4_t& s) {
+    const int n = (int)((uint32_t)__builtin_amdgcn_readlane((int)d.meta.x, x) & 0xffu);
     const uint32_t mk = d.ks[x] * 0x00010001u;   // (s, s) of the lane's token
+    uint4 ex[4];
+    bool mine[4] = {false, false, false, false};
+    if (n) {   // wave-uniform
+        int64_t base = meta_base(d, x);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {   // the lane's slot of group c is bit `lane` of the group's mask
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)d.mask.x, 4 * x + c);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)d.mask.y, 4 * x + c);
+            const int64_t idx = base + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            mine[c] = (((lane & 32) ? hi : lo) >> (lane & 31)) & 1u && idx < A.k.exc_cap;
+            if (mine[c]) ex[c] = reinterpret_cast<const uint4*>(A.k.exc)[idx];
+            base += __builtin_popcount(lo) + __builtin_popcount(hi);
+        }
+    }
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         uint32_t p[4];
         rec_pairs(d.ka[x][c], d.kb[x][c], p);
 #pragma unroll
         for (int i = 0; i < 4; i++) p[i] = unbias(p[i]);
-        if (n) {   // rare: exception entries of group c replace records (uniform loop)
-            const int64_t base = meta_base(d, x);
-            const int cnt = n < 255 ? n : 4 * 64;
-            for (int e = 0; e < cnt; e++) {
-                const int code = exc_code(A.k, rb, hdr, e);
-                if (code < 0) break;
-                const int64_t idx = base + e;
-                if ((code >> 6) == c && (code & 63) == lane && idx < A.k.exc_cap) {
-                    int v[8];
-                    exc_load(A.k.exc, idx, v);
+        if (n && mine[c]) {
+            const uint32_t w[4] = {ex[c].x, ex[c].y, ex[c].z, ex[c].w};
 #pragma unroll
-                    for (int i = 0; i < 4; i++) p[i] = pair_from_i16(v[2 * i], v[2 * i + 1]);
-                }
-            }
+            for (int i = 0; i < 4; i++) p[i] = pair_from_i16((int)(int16_t)(w[i] & 0xffffu), (int)(int16_t)(w[i] >> 16));
         }
         mul_pairs<4>(p, mk);
         s = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[c], as_h8(p[0], p[1], p[2], p[3]), s, 0, 0, 0);
@@ -486,8 +479,7 @@ __device__ __forceinline__ void tile_k(const AttnArgs& A, const TileRaw& d, int6
 // V of the lane's 8 tokens (vector lane % 16), two tokens at a time:
 // vp[k][i] = fp16 pair (dimension 8 n + i of token 2 k, of token 2 k + 1),
 // dequantised -- the operand halves of P V's MFMA i as they are.
-__device__ __forceinline__ void tile_v(const AttnArgs& A, const TileRaw& d, int64_t rb0, int lane,
-                                       uint32_t vp[4][8]) {
+__device__ __forceinline__ void tile_v(const AttnArgs& A, const TileRaw& d, int lane, uint32_t vp[4][8]) {
     const int n = lane & 15, k8 = lane >> 4, xb = k8 >> 1;
     const uint32_t aw[8] = {d.va0.x, d.va0.y, d.va0.z, d.va0.w, d.va1.x, d.va1.y, d.va1.z, d.va1.w};
 #pragma unroll
@@ -497,34 +489,48 @@ __device__ __forceinline__ void tile_v(const AttnArgs& A, const TileRaw& d, int6
 #pragma unroll
         for (int i = 0; i < 8; i++) vp[k][i] = unbias(vp[k][i]);
     }
-    const uint64_t h0 = meta_hdr(d, 2), h1 = meta_hdr(d, 3);
-    if ((h0 | h1) & 0xffull) {   // rare: exception entries replace records (uniform loops)
-#pragma unroll 1
-        for (int x = 0; x < 2; x++) {
-            const uint64_t hdr = x ? h1 : h0;
-            const int64_t base = x ? meta_base(d, 3) : meta_base(d, 2);
-            const int cnt0 = (int)(hdr & 0xffu);
-            const int cnt = cnt0 < 255 ? cnt0 : 4 * 64;
-            for (int e = 0; e < cnt; e++) {
-                const int code = exc_code(A.v, rb0 + x, hdr, e);
-                if (code < 0) break;
-                const int sl = code & 63, g = code >> 6;
-                const int64_t idx = base + e;
-                // the lane holding (slot sl, group g) of block x, and its token q
-                const bool mine = xb == x && n == 4 * g + (sl >> 4) && (k8 & 1) == ((sl & 15) >> 3);
-                if (mine && idx < A.v.exc_cap) {
-                    int v[8];
-                    exc_load(A.v.exc, idx, v);
-                    const int q = sl & 7;
+    const uint32_t c0 = (uint32_t)__builtin_amdgcn_readlane((int)d.meta.x, 2) & 0xffu;
+    const uint32_t c1 = (uint32_t)__builtin_amdgcn_readlane((int)d.meta.x, 3) & 0xffu;
+    if (c0 | c1) {   // wave-uniform
+        // the lane's tokens are 8 consecutive slots, one byte of the mask of
+        // block xb's group n / 4; entries before that group's in lane 8 + 4 xb + n / 4
+        const int pc = __builtin_popcount(d.mask.x) + __builtin_popcount(d.mask.y);
+        int before = 0;
 #pragma unroll
-                    for (int k = 0; k < 4; k++)
+        for (int o = 1; o < 4; o++) {
+            const int u = __shfl(pc, (lane & ~3) | ((lane - o) & 3), 64);
+            before += (lane & 3) >= o ? u : 0;
+        }
+        const int src = 8 + 4 * xb + (n >> 2);
+        const uint32_t lo = (uint32_t)__shfl((int)d.mask.x, src, 64), hi = (uint32_t)__shfl((int)d.mask.y, src, 64);
+        const int s0 = 16 * (n & 3) + 8 * (k8 & 1);   // bit of the lane's first token
+        const uint64_t m = ((uint64_t)hi << 32) | lo;
+        const int64_t base = (int64_t)(xb ? meta_base(d, 3) : meta_base(d, 2)) + __shfl(before, src, 64) +
+                             __builtin_popcountll(m & ((1ull << s0) - 1ull));
+        const uint32_t own = (uint32_t)(m >> s0) & 0xffu;
 #pragma unroll
-                        for (int i = 0; i < 8; i++) {
-                            h2_t h = __builtin_bit_cast(h2_t, vp[k][i]);
-                            if (q == 2 * k) h[0] = (_Float16)((float)v[i] * 0.5f);
-                            if (q == 2 * k + 1) h[1] = (_Float16)((float)v[i] * 0.5f);
-                            vp[k][i] = __builtin_bit_cast(uint32_t, h);
-                        }
+        for (int q0 = 0; q0 < 8; q0 += 4) {
+            uint4 ex[4];
+            bool mine[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int q = q0 + j;
+                const int64_t idx = base + __builtin_popcount(own & ((1u << q) - 1u));
+                mine[j] = ((own >> q) & 1u) && idx < A.v.exc_cap;
+                if (mine[j]) ex[j] = reinterpret_cast<const uint4*>(A.v.exc)[idx];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (!__any(mine[j])) continue;
+                if (mine[j]) {
+                    const uint32_t w[4] = {ex[j].x, ex[j].y, ex[j].z, ex[j].w};
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const int c = (int)(int16_t)((i & 1) ? w[i >> 1] >> 16 : w[i >> 1] & 0xffffu);
+                        h2_t h = __builtin_bit_cast(h2_t, vp[(q0 + j) >> 1][i]);
+                        h[j & 1] = (_Float16)((float)c * 0.5f);
+                        vp[(q0 + j) >> 1][i] = __builtin_bit_cast(uint32_t, h);
+                    }
                 }
             }
         }
@@ -599,9 +605,9 @@ __device__ __forceinline__ void tile_softmax_pv(int G, const f4_t s[2], const bo
     wave_lds_sync();
 }
 
-// Decode of one prefix tile from its registers (rb0: resident block of the
-// tile's first token): the scores s of its two blocks and the V pairs.
-__device__ __forceinline__ void prefix_decode(const AttnArgs& A, const TileRaw& d, int64_t rb0, int64_t t0, int64_t T,
+// Decode of one prefix tile from its registers: the scores s of its two blocks
+// and the V pairs.
+__device__ __forceinline__ void prefix_decode(const AttnArgs& A, const TileRaw& d, int64_t t0, int64_t T,
                                               int lane, const h8_t qa[4], f4_t s[2], bool valid[2],
                                               uint32_t vp[4][8]) {
 #pragma unroll
@@ -609,9 +615,9 @@ __device__ __forceinline__ void prefix_decode(const AttnArgs& A, const TileRaw& 
         s[x] = f4_t{0.f, 0.f, 0.f, 0.f};
         valid[x] = t0 + 16 * x + (lane & 15) < T;
         if (t0 + 16 * x < T)   // wave-uniform
-            tile_k(A, d, rb0 + x, x, lane, qa, s[x]);
+            tile_k(A, d, x, lane, qa, s[x]);
     }
-    tile_v(A, d, rb0, lane, vp);
+    tile_v(A, d, lane, vp);
 }
 
 // The tail tiles this wave owns: tail tile tt goes to the kv head's wave
@@ -664,7 +670,6 @@ __device__ __forceinline__ void prefix_tiles(const AttnArgs& A, int64_t kvh, int
         if (A.t_tail > 0) tail_owned<HPL>(A, kvh, gw, W, A.t_tail, lane, qa, pt, m_run, l_run, o);
         return;
     }
-    const int64_t hb = kvh * A.k.cap_blocks;
     TileRaw d;
     tile_load(A, kvh, g * kTile, T, lane, d);
     if (A.t_tail > 0) tail_owned<HPL>(A, kvh, gw, W, A.t_tail, lane, qa, pt, m_run, l_run, o);
@@ -677,7 +682,7 @@ __device__ __forceinline__ void prefix_tiles(const AttnArgs& A, int64_t kvh, int
         f4_t s[2];
         bool valid[2];
         uint32_t vp[4][8];
-        prefix_decode(A, d, hb + ta / kRB, ta, T, lane, qa, s, valid, vp);
+        prefix_decode(A, d, ta, T, lane, qa, s, valid, vp);
         // Every use of this tile's registers is scheduled before the reload, and
         // the reload is unconditional (past the prefix it re-reads this tile,
         // from cache), so the next tile's loads land in place and nothing

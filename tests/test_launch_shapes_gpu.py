@@ -300,3 +300,50 @@ def test_direct_updates_gpu(B, H, hd, steps, dtype, monkeypatch):
             assert torch.equal(ca.gpu_bitstream, cb.gpu_bitstream) and torch.equal(ca.coset_packed, cb.coset_packed)
             assert torch.equal(ca.scales, cb.scales) and torch.equal(ca.encoded.sigma2, cb.encoded.sigma2)
             assert torch.equal(a._decompress_chunk(ca), b._decompress_chunk(cb))
+
+
+@pytest.mark.parametrize("T,chans,factor", [
+    (16, 1, 400.0),      # one block, one vector of every token outside the records' range
+    (48, 128, 400.0),    # every vector is an exception (256 of a block: the count saturates)
+    (2064, 3, 40.0),     # several per token, a half tile at the end
+    (4096, 40, 12.0),    # about one vector in three
+])
+@pytest.mark.parametrize("which", ["k", "v", "both"])
+def test_attention_exceptions_gpu(T, chans, factor, which):
+    """Attention over prefixes with many exception vectors, in K, in V and in
+    both, against float64 attention over the rows the dequantiser writes for
+    the same prefix (it reads every exception on its own).  The step rounds
+    each weight of P V to fp16 (2^-11 of it) and its output (2^-11), so it lies
+    within 2^-10 of sum_t p_t |v_t|; a fifth of that for the fp32 scores."""
+    from latticequant_amd import codec
+    from latticequant_amd.llm import resident
+    B, H, group, tail = 2, 2, 4, 5
+    g = torch.Generator().manual_seed(T + chans)
+    kv = torch.randn(2, B, H, T, 128, generator=g)
+    pick = torch.randperm(128, generator=g)[:chans]
+    for i in range(2):
+        if which in ("both", "kv"[i]):
+            kv[i][..., pick] *= factor
+    if which != "v":
+        kv[0] *= 0.05     # keep the scores of outlier channels in range of a soft maximum
+    kv = kv.half().cuda()
+    q = torch.randn(B, H * group, 1, 128, generator=g).half().cuda()
+    tl = torch.randn(2, B, H, tail, 128, generator=g).half().cuda()
+    res = []
+    for i in range(2):
+        # coordinates up to 900: outlier channels far outside [-16, 15], and below
+        # 1024, up to which fp16 holds every half-integer (the kernel's operands
+        # are fp16; larger coordinates are rounded before the scale)
+        s32 = torch.full((B * H,), float(kv[i].abs().max()) / 900.0, device="cuda")
+        r = resident.ResidentKV(B * H, T)
+        r.append(kv[i], s32, s32.half())
+        res.append(r)
+    assert int(res[0].n_exc) + int(res[1].n_exc) > 0
+    out = resident.resident_decode_attention(res[0], res[1], q, tl[0], tl[1])
+    k, v = (torch.cat([r.dequant(torch.float32).view(B, H, T, 128).half(), tl[i]], 2).double()
+            for i, r in enumerate(res))
+    qq = q.double().view(B, H, group, 128)
+    p = torch.matmul(qq, k.transpose(-1, -2).contiguous()) / 128 ** 0.5
+    w = p.softmax(-1)
+    err = (out.double().view(B, H, group, 128) - torch.matmul(w, v)).abs().amax(-1) / torch.matmul(w, v.abs()).amax(-1)
+    assert float(err.max()) < 1.2 * 2.0 ** -10

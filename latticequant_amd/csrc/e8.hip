@@ -290,11 +290,16 @@ __device__ __forceinline__ void stage_minmax(const uint4& w, int row16, int n0, 
 // by the scale as IEEE division rounds (div_exact where the row and the scale
 // lie in its range); no dequantised output, at least 5 waves per SIMD.
 // LDT >= 0: the input dtype as a compile-time constant (the lean launches),
-// so no dtype test is kept live across the block loop.  LPR > 0: the rotation's
+// so no dtype test is kept live across the block loop.
+// VALU issue bounds the lean launches (131072 blocks of fp16: about 300
+// operations per vector and lane; 581 us with both D8 roundings' flips
+// resolved and no load ahead, 558 us with only the chosen one's, 513 us with
+// the next block's rows in flight; the bytes alone take 326 us).  6 waves per
+// SIMD is what their 75 to 77 vector registers allow; forcing 7 spills.  LPR > 0: the rotation's
 // lanes per row as a compile-time constant, so the butterfly stages are
 // straight-line code (no per-stage branch and register copies).
 template <typename SymT, bool DITHER, bool LEAN = false, bool ROT = false, int LDT = -1, int LPR = 0>
-__global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_quantize(
+__global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 6 : 1)) void k_chunk_quantize(
     const void* __restrict__ x, int dtype, int64_t n_heads, int64_t bph, int64_t nblk,
     const float* __restrict__ scale32, const int32_t* __restrict__ fastdiv, SymT* __restrict__ sym,
     uint8_t* __restrict__ coset_bits, uint32_t* __restrict__ blk_n1, uint32_t* __restrict__ hist,
@@ -302,6 +307,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
     const int64_t* __restrict__ dseed, const float* __restrict__ signs, int lpr, float rdiv, int bpw) {
     constexpr bool kWide = sizeof(SymT) == 2;
     constexpr int kSymMin = kWide ? -32768 : -128, kSymMax = kWide ? 32767 : 127;
+    constexpr bool kBiased = LEAN || ROT;   // no dequantised output: the points are only needed as integers
     __shared__ uint32_t shist[kWide ? 1 : LQ_STREAMS * kHRow];
     __shared__ int smin[LQ_STREAMS], smax[LQ_STREAMS];
     __shared__ __align__(16) SymT stage[kSymStride];
@@ -328,10 +334,22 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
     // (stage_minmax: the staged rows a thread copies all hold one coordinate)
     int tmin[2] = {INT_MAX, INT_MAX}, tmax[2] = {INT_MIN, INT_MIN};
 
+    // the lean 16-bit launches load a block's rows while the one before is
+    // staged and copied out (unconditionally: after the last block its own
+    // rows, from the cache, past the chunk's end the last row again)
+    constexpr bool kAhead = LEAN && !ROT && (LDT == LQ_F16 || LDT == LQ_BF16);
+    uint4 ahead[2];
+    auto fetch = [&](int64_t blk) {   // a block of the chunk: uniform base, 32-bit lane offsets
+        const uint4* const row = reinterpret_cast<const uint4*>(x) + chunk * V + blk * kBlk;
+        const int last = (int)((V - blk * kBlk) < kBlk ? (V - blk * kBlk) : kBlk) - 1;
+#pragma unroll
+        for (int r = 0; r < 2; r++) ahead[r] = row[(uint32_t)min(r * kQThreads + tid, last)];
+    };
+    const int64_t bend = b0 + bpw < nblk ? b0 + bpw : nblk;
+    if constexpr (kAhead) fetch(b0);
+
     int flag = 0;
-    for (int bi = 0; bi < bpw; bi++) {
-        const int64_t blk = b0 + bi;
-        if (blk >= nblk) break;
+    for (int64_t blk = b0; blk < bend; blk++) {
         const int64_t vbase = blk * kBlk;
         const int valid = (int)((V - vbase) < kBlk ? (V - vbase) : kBlk);
         // head of the block's first vector and its offset in that head (uniform);
@@ -357,7 +375,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
                 rs0 = __int_as_float(w0); rs1 = __int_as_float(w1);   // RN(1 / s) where fast
             }
         }
-        int32_t sy[2][8];
+        int32_t sy[2][8];   // kE8Bias + coordinate, wrapping
         int cs[2];
         unsigned long long bal[2];
         // pass 1: quantize two vectors per thread
@@ -392,7 +410,8 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
                     hq = h;
                 }
                 float xv[8], t[8], ic[8], dd[8];
-                load8(x, LDT >= 0 ? LDT : dtype, chunk * V + v, xv);
+                if constexpr (kAhead) unpack8(ahead[r], LDT, xv);
+                else load8(x, LDT >= 0 ? LDT : dtype, chunk * V + v, xv);
                 if constexpr (ROT) {
                     // rows start at multiples of lpr vectors and blocks at
                     // multiples of 512, so the lane's place in its row is tid % lpr;
@@ -432,14 +451,14 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
                     float4* slot = reinterpret_cast<float4*>(tslot + 8 * tid);
                     slot[0] = make_float4(t[0], t[1], t[2], t[3]);
                     slot[1] = make_float4(t[4], t[5], t[6], t[7]);
-                    c = e8_nearest_fast(t, ic, [&](float tt[8]) {
+                    c = e8_nearest_fast<kBiased>(t, ic, [&](float tt[8]) {
                         asm volatile("" ::: "memory");   // read the slot back: t is not kept live for this
                         const float4 a = slot[0], b = slot[1];
                         tt[0] = a.x; tt[1] = a.y; tt[2] = a.z; tt[3] = a.w;
                         tt[4] = b.x; tt[5] = b.y; tt[6] = b.z; tt[7] = b.w;
                     }, &tm);
                 } else {               // the rare exact path recomputes t from x
-                    c = e8_nearest_fast(t, ic, [&](float tt[8]) {
+                    c = e8_nearest_fast<kBiased>(t, ic, [&](float tt[8]) {
                         float xx[8];
                         load8(x, LDT >= 0 ? LDT : dtype, chunk * V + v, xx);
 #pragma unroll
@@ -454,26 +473,29 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
                 }
                 cs[r] = c;
 #pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const int32_t iv = (int32_t)ic[i];
-                    sy[r][i] = i < 7 ? iv : (iv >> 1);
-                }
+                for (int i = 0; i < 8; i++)
+                    sy[r][i] = kBiased ? __float_as_int(ic[i]) : (int32_t)(kE8Bias + (uint32_t)(int32_t)ic[i]);
                 // max |t_i| < kSymMax - 1 puts every coordinate in
                 // [-kSymMax, kSymMax] (e8_nearest_fast), so the symbols are in
                 // range; only vectors with a larger (or infinite) |t_i| are
                 // checked.  Out-of-range symbols are flagged and clamped
                 // (histogram indices stay in range).
                 if (!(tm < (float)(kSymMax - 1))) {
-                    int32_t lo = INT_MAX, hi = INT_MIN;
+                    int32_t sv[8], lo = INT_MAX, hi = INT_MIN;
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
-                        lo = min(lo, sy[r][i]);
-                        hi = max(hi, sy[r][i]);
+                        const int32_t iv = (int32_t)((uint32_t)sy[r][i] - kE8Bias);
+                        sv[i] = i < 7 ? iv : iv >> 1;
+                        lo = min(lo, sv[i]);
+                        hi = max(hi, sv[i]);
                     }
                     if (lo < kSymMin || hi > kSymMax) {
                         flag = 1;
 #pragma unroll
-                        for (int i = 0; i < 8; i++) sy[r][i] = min(max(sy[r][i], kSymMin), kSymMax);
+                        for (int i = 0; i < 8; i++) {
+                            const int32_t cl = min(max(sv[i], kSymMin), kSymMax);
+                            sy[r][i] = (int32_t)kE8Bias + (i < 7 ? cl : 2 * cl);
+                        }
                     }
                 }
                 if (!LEAN && !ROT && deq) {
@@ -489,6 +511,7 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
             bal[r] = __ballot(cs[r]);
             if (lane == 0) masks[r * 4 + wave] = bal[r];
         }
+        if constexpr (kAhead) fetch(blk + 1 < bend ? blk + 1 : blk);
         __syncthreads();
         // coset-1 counts of the block's 8 ballot words: the words are the same
         // for every lane, so they are made wave-uniform and counted on the
@@ -526,13 +549,9 @@ __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 7 : 1)) void k_chunk_q
                 const int c = cs[r];
                 const int rk = c ? rank1 : rank0;
                 SymT* sp = stage + sym_pos(c, 0, rk, n0);   // column i adds 16 * i
-                if constexpr (!kWide) {
+                // the low bits of the biased integers (kE8Bias has none there)
 #pragma unroll
-                    for (int i = 0; i < 8; i++) sp[16 * i] = (SymT)sy[r][i];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; i++) sp[16 * i] = (SymT)sy[r][i];
-                }
+                for (int i = 0; i < 8; i++) sp[16 * i] = (SymT)(i < 7 ? sy[r][i] : sy[r][i] >> 1);
             }
         }
         __syncthreads();

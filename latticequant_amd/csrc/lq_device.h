@@ -84,27 +84,31 @@ __device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even, 
 }
 
 // Load one 8-dim vector (index v) of an fp16 / bf16 / fp32 array as fp32.
+// The eight 16-bit values (fp16 or bf16) of one 16-byte row.
+__device__ __forceinline__ void unpack8(const uint4& r, int dtype, float x[8]) {
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+    if (dtype == LQ_F16) {   // dtype is uniform: one branch, not a select per element
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x[2 * i] = h2f((uint16_t)(w[i] & 0xffffu));
+            x[2 * i + 1] = h2f((uint16_t)(w[i] >> 16));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x[2 * i] = __uint_as_float(w[i] << 16);
+            x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+        }
+    }
+}
+
 __device__ __forceinline__ void load8(const void* base, int dtype, int64_t v, float x[8]) {
     if (dtype == LQ_F32) {
         const float4* p = reinterpret_cast<const float4*>(base) + 2 * v;
         float4 a = p[0], b = p[1];
         x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
     } else {
-        uint4 r = reinterpret_cast<const uint4*>(base)[v];
-        uint32_t w[4] = {r.x, r.y, r.z, r.w};
-        if (dtype == LQ_F16) {   // dtype is uniform: one branch, not a select per element
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                x[2 * i] = h2f((uint16_t)(w[i] & 0xffffu));
-                x[2 * i + 1] = h2f((uint16_t)(w[i] >> 16));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                x[2 * i] = __uint_as_float(w[i] << 16);
-                x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-            }
-        }
+        unpack8(reinterpret_cast<const uint4*>(base)[v], dtype, x);
     }
 }
 
@@ -198,79 +202,51 @@ __host__ __device__ __forceinline__ int e8_nearest(const float x[8], float ic[8]
 }
 
 // The same nearest E8 point as e8_nearest, with less arithmetic on the common
-// path.  Both D8 roundings are taken as in d8_round, but their flips are not
-// applied until the coset is known (one flip instead of two).  The coset
-// choice d1 <= d2 is first decided from an estimate of d1 - d2 with a proven
-// error bound; only when the estimate lies within that bound of zero are the
-// two distances summed in the reference's order from the same halves.
+// path: what the reference needs two complete D8 roundings and two distance
+// sums for is decided from the roundings' remainders, and only the chosen
+// rounding's flip is looked for.  The kernels that call this are bound by VALU
+// issue, so the count of instructions is their time (the int8 quantizer at
+// 131072 blocks: see k_chunk_quantize).
 //
 // With e1 = x - r1 and e2 = y - r2 (y = RN(x - 1/2); both differences exact),
 //   d1 = sum e1^2 + odd1 (1 - 2 |e1_j|),  d2 = sum e2^2 + odd2 (1 - 2 |e2_k|)
 // (j, k the flipped coordinates).  |e2_i| = 1/2 - |e1_i| + s_i with |s_i| <= U,
 // U the ulp of max(1, max |x_i|) (the rounding of y), so
 // e1_i^2 - e2_i^2 = |e1_i| - 1/4 + O(1.01 U), and with f_i = RN(1 - 2 |e1_i|)
-// (the flip costs d8_half computes anyway)
-//   d1 - d2 ~ est = 2 - (sum f_i) / 2 + odd1 f1_j - odd2 f2_k.
-// The error of est against the exact d1 - d2 (the s_i, the rounding of the
-// reference's differences x - c, of the f_i and of the fp32 evaluation, <= 1.9e-6)
-// plus the reference's own rounding of its sums (<= 9 * 2^-24 relative on
-// d <= 4) stays below 1e-5 + 32 U; beyond that margin the sign of est is the
-// sign of the reference's fp32 d1 - d2.  max |x_i| >= 2^21 (or inf / NaN
-// through est) takes the exact path.
+// (the flip costs of d8_half) and m1, m2 the smallest tie-broken flip costs
+// RN(f_i + tiebreak_i) of each half
+//   d1 - d2 ~ est = 2 - (sum f_i) / 2 + odd1 m1 - odd2 m2.
+// The error of est against the exact d1 - d2 (the s_i, the tie-break terms in
+// m1 and m2 with their rounding, <= 1.6e-6, the rounding of the reference's
+// differences x - c, of the f_i and of the fp32 evaluation, <= 1.9e-6) plus
+// the reference's own rounding of its sums (<= 9 * 2^-24 relative on d <= 4)
+// stays below 1e-5 + 32 U; beyond that margin the sign of est is the sign of
+// the reference's fp32 d1 - d2.  Within it, and for max |x_i| >= 2^20 (or inf /
+// NaN through est), e8_nearest is taken.  Below 2^20 every sum of rounded
+// coordinates is an exact integer below 2^24, whose parity is s - 2 rint(s / 2)
+// as -1, 0 or 1.
 struct D8Half {
-    float r[8], e[8];
-    bool sel[8];   // first-index argmin of RN(RN(1 - 2|e_i|) + tiebreak_i)
-    float es;      // e at that index
+    float best;    // min RN(RN(1 - 2|e_i|) + tiebreak_i)
     float fsum;    // sum of RN(1 - 2|e_i|) (left to right), when asked for
-    bool odd;      // the fp32 coordinate sum is odd
+    float odd;     // +-1 when the coordinate sum is odd, else 0
 };
 
 template <bool FSUM>
 __host__ __device__ __forceinline__ void d8_half(const float x[8], D8Half& h) {
+    float adj[8], s = 0.f, fs = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        h.r[i] = rintf(x[i]);
-        h.e[i] = x[i] - h.r[i];
-    }
-    float s = h.r[0];
-#pragma unroll
-    for (int i = 1; i < 8; i++) s += h.r[i];
-    h.odd = fabsf(s) < 16777216.0f && (((int32_t)s) & 1);
-    float best = 0.f, es = h.e[0], fs = 0.f;
-    bool upd[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float fc = __builtin_fmaf(-2.0f, fabsf(h.e[i]), 1.0f);
+        const float r = rintf(x[i]);
+        const float fc = __builtin_fmaf(-2.0f, fabsf(x[i] - r), 1.0f);
+        s = i == 0 ? r : s + r;
         if (FSUM) fs = i == 0 ? fc : fs + fc;
-        const float adj = i == 0 ? fc : fc + tiebreak(i);
-        upd[i] = i == 0 || adj < best;
-        best = upd[i] ? adj : best;
-        es = upd[i] ? h.e[i] : es;
+        adj[i] = i == 0 ? fc : fc + tiebreak(i);   // tiebreak(0) = 0 and fc is never -0
     }
-    bool later = false;
-#pragma unroll
-    for (int i = 7; i >= 0; i--) {
-        h.sel[i] = upd[i] && !later;
-        later = later || upd[i];
-    }
-    h.es = es;
+    h.odd = __builtin_fmaf(-2.0f, rintf(s * 0.5f), s);
+    // in threes: three-operand minima on the device
+    h.best = fminf(fminf(fminf(fminf(adj[0], adj[1]), adj[2]), fminf(fminf(adj[3], adj[4]), adj[5])),
+                   fminf(adj[6], adj[7]));
     h.fsum = fs;
-}
-
-// Reference-order coset choice (core/e8_quantizer.py:79-83) given the halves.
-__host__ __device__ __forceinline__ bool e8_choose_exact(const float x[8], const D8Half& a, const D8Half& b,
-                                                         float fa, float fb) {
-    float d1 = 0.f, d2 = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float c1 = a.r[i] + (a.sel[i] ? fa : 0.f);
-        const float c2 = (b.r[i] + (b.sel[i] ? fb : 0.f)) + 0.5f;
-        const float u = x[i] - c1, v = x[i] - c2;
-        const float u2 = u * u, v2 = v * v;
-        d1 = (i == 0) ? u2 : d1 + u2;
-        d2 = (i == 0) ? v2 : d2 + v2;
-    }
-    return d1 <= d2;
 }
 
 // reload(float x[8]) writes x again for the rare exact path, so that x need
@@ -279,7 +255,13 @@ __host__ __device__ __forceinline__ bool e8_choose_exact(const float x[8], const
 // integer T, every returned coordinate lies in [-(T + 1), T + 1]: rint(x_i)
 // lies in [-T, T], rint(x_i - 1/2) in [-T, T - 1], and a flip adds +-1.
 // Callers can skip the range checks of their symbols then.
-template <typename Reload>
+//
+// BIASED: ic[i] receives the bits kE8Bias + (int32_t)ic_i (wrapping) instead,
+// kE8Bias those of 1.5 * 2^23: the flip is added to that number, so the integer
+// stands in the low bits without a conversion.
+constexpr uint32_t kE8Bias = 0x4b400000u;
+
+template <bool BIASED = false, typename Reload>
 __host__ __device__ __forceinline__ int e8_nearest_fast(const float x[8], float ic[8], Reload&& reload,
                                                         float* tmax = nullptr) {
     D8Half a, b;
@@ -289,28 +271,49 @@ __host__ __device__ __forceinline__ int e8_nearest_fast(const float x[8], float 
     for (int i = 0; i < 8; i++) y[i] = x[i] - 0.5f;
     d8_half<false>(y, b);
     float est = __builtin_fmaf(a.fsum, -0.5f, 2.0f);
-    if (a.odd) est += __builtin_fmaf(-2.0f, fabsf(a.es), 1.0f);
-    if (b.odd) est -= __builtin_fmaf(-2.0f, fabsf(b.es), 1.0f);
-    float t = fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))),
-                    fmaxf(fmaxf(fabsf(x[4]), fabsf(x[5])), fmaxf(fabsf(x[6]), fabsf(x[7]))));
-    t = fmaxf(t, 1.0f);
+    est = __builtin_fmaf(fabsf(a.odd), a.best, est);
+    est = __builtin_fmaf(-fabsf(b.odd), b.best, est);
+    const float t = fmaxf(fmaxf(fmaxf(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fabsf(x[2])),
+                                      fmaxf(fmaxf(fabsf(x[3]), fabsf(x[4])), fabsf(x[5]))),
+                                fmaxf(fabsf(x[6]), fabsf(x[7]))), 1.0f);
     const float p2 = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) & 0x7f800000u);   // 2^floor(log2 t)
     const float margin = __builtin_fmaf(32.0f * 0x1p-23f, p2, 1e-5f);   // 1e-5 + 32 ulp(t)
-    // each half's flip as a float step (0 when its sum is even)
-    const float fa = a.odd ? (a.es < 0.f ? -1.f : 1.f) : 0.f;
-    const float fb = b.odd ? (b.es < 0.f ? -1.f : 1.f) : 0.f;
-    bool use1 = est < 0.f;
-    if (!(t < 2097152.0f) || !(fabsf(est) > margin)) {
-        float xr[8];
-        reload(xr);
-        use1 = e8_choose_exact(xr, a, b, fa, fb);
-    }
     if (tmax) *tmax = t;
+    bool use1 = est < 0.f;
+    // the chosen half: its flip goes to the first coordinate of the smallest
+    // cost (no coordinate when its sum is even: every cost is >= 0)
+    const float odd = use1 ? a.odd : b.odd;
+    float best = use1 ? a.best : b.best;
+    best = odd != 0.f ? best : -1.f;
+    // its coordinates and costs are taken from x again (x - 0 is x): keeping
+    // both halves' instead (24 selects for these 39 operations) held 91 to 102
+    // vector registers in the quantizers and was slower at every occupancy
+    const float shift = use1 ? 0.f : 0.5f;
+    float r[8], es = 0.f;
+    bool sel[8], seen = false;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float ca = a.r[i] + (a.sel[i] ? fa : 0.f);
-        const float cb = b.r[i] + (b.sel[i] ? fb : 0.f);
-        ic[i] = use1 ? ca : cb;
+        const float xs = x[i] - shift;
+        r[i] = rintf(xs);
+        const float e = xs - r[i];
+        const float fc = __builtin_fmaf(-2.0f, fabsf(e), 1.0f);
+        const bool eq = (i == 0 ? fc : fc + tiebreak(i)) == best;
+        sel[i] = eq && !seen;
+        seen = seen || eq;
+        es = sel[i] ? e : es;
+    }
+    constexpr float kZero = BIASED ? 12582912.0f : 0.f;   // 1.5 * 2^23
+    const float step = kZero + __builtin_copysignf(1.0f, es);   // es is never -0
+#pragma unroll
+    for (int i = 0; i < 8; i++) ic[i] = r[i] + (sel[i] ? step : kZero);
+    if (!(t < 1048576.0f) || !(fabsf(est) > margin)) {
+        float xr[8];
+        reload(xr);
+        use1 = e8_nearest(xr, ic) == 0;
+        if (BIASED) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) ic[i] = __builtin_bit_cast(float, kE8Bias + (uint32_t)(int32_t)ic[i]);
+        }
     }
     return use1 ? 0 : 1;
 }

@@ -347,3 +347,64 @@ def test_attention_exceptions_gpu(T, chans, factor, which):
     w = p.softmax(-1)
     err = (out.double().view(B, H, group, 128) - torch.matmul(w, v)).abs().amax(-1) / torch.matmul(w, v.abs()).amax(-1)
     assert float(err.max()) < 1.2 * 2.0 ** -10
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("H,bph", [(1, 512), (1, 1025), (3, 515), (2, 20 * 512 + 7)])
+def test_quantizer_integer_output_gpu(dtype, wide, H, bph):
+    """Launches without a dequantised output keep the lattice points as biased
+    integers and load a block ahead; those with one keep floats and load none.
+    Both give the same symbols, bitmaps, counts, histograms or ranges, and
+    status, up to coordinates beyond every symbol range, infinities and NaN,
+    and at ragged ends."""
+    from latticequant_amd import _lib as L
+    C, V, nblk = 2, H * bph, (H * bph + 511) // 512
+    g = torch.Generator().manual_seed(bph)
+    x = torch.randn(C, V, 8, generator=g) * 2.0 ** torch.randint(-3, 5, (C, V, 1), generator=g)
+    x[:, ::3] = torch.round(x[:, ::3] * 2) / 2                     # grid points: ties
+    x[0, 7::61] = torch.randn(x[0, 7::61].shape, generator=g) * 30000    # chunk 0 overflows, chunk 1 does not
+    x[0, 11::97, 3] = float("inf")
+    x[0, 13::89, 5] = float("-inf")
+    x[0, 17::101, 0] = float("nan")
+    if dtype != torch.float16:
+        x[0, 19::103] = torch.randn(x[0, 19::103].shape, generator=g) * 1e7
+    x = x.to(dtype).cuda().contiguous()
+    scale = torch.full((C * H,), 0.75, device="cuda")
+    code, lib, s = L.dtype_code(dtype), L.lib(), L.stream_ptr(x.device)
+    fd = torch.empty(C * H, dtype=torch.int32, device="cuda")
+    L.check(lib.lq_scale_fastdiv(scale.data_ptr(), C * H, code, fd.data_ptr(), s), "lq_scale_fastdiv")
+
+    def run(out):
+        sym = torch.zeros(C * nblk * L.LQ_SYM_STRIDE * (2 if wide else 1), dtype=torch.int8, device="cuda")
+        cb = torch.zeros(C * nblk * 64, dtype=torch.uint8, device="cuda")
+        n1 = torch.zeros(C * nblk, dtype=torch.int32, device="cuda")
+        st = torch.zeros(C, dtype=torch.int32, device="cuda")
+        if wide:
+            tab = torch.tensor([2 ** 31 - 1, -2 ** 31], dtype=torch.int32).repeat(C * 16).cuda()
+        else:
+            tab = torch.zeros(C * 16 * 256, dtype=torch.int32, device="cuda")
+        f = lib.lq_chunk_quantize_wide if wide else lib.lq_chunk_quantize
+        L.check(f(x.data_ptr(), code, C, H, bph, scale.data_ptr(), fd.data_ptr(), sym.data_ptr(), cb.data_ptr(),
+                  n1.data_ptr(), tab.data_ptr(), st.data_ptr(), L.ptr(out), code, None, s), "lq_chunk_quantize")
+        return sym, cb, n1, tab, st
+
+    lean, full = run(None), run(torch.empty_like(x))
+    # rows of a group's unused places keep what an earlier block staged there,
+    # so the staging is compared through the counts' ranges: symbols by column
+    for a, b in zip(lean[1:], full[1:]):
+        assert torch.equal(a, b)
+    assert lean[4].cpu().tolist() == [lean[4][0].item(), 0] and lean[4][0].item() != 0
+    w = torch.int16 if wide else torch.int8
+    a, b = (t.view(w).view(C * nblk, -1).cpu() for t in (lean[0], full[0]))
+    n1 = lean[2].cpu()
+    for k in range(C * nblk):
+        valid = min(512, V - (k % nblk) * 512)
+        one = int(n1[k])
+        base = 0
+        for n in (valid - one, one):
+            for q in range(0, n, 16):
+                m = min(16, n - q)
+                ga, gb = (t[k, base:base + 128].view(8, 16)[:, :m] for t in (a, b))
+                assert torch.equal(ga, gb), (k, q)
+                base += 128

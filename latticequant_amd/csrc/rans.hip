@@ -1835,12 +1835,42 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
 // renormalisation needs no more than those bits; it fills a CU's LDS, so it is
 // taken for up to two streams per CU, and the one-symbol table (many
 // workgroups per CU) beyond.  One lane per stream with the tables in global
-// memory, bit by bit, took 30771 us for 16 streams of 32768 symbols; this takes
-// 1436 us.
+// memory, bit by bit, took 30771 us for 16 streams of 32768 symbols,
+// the chain alone 1434 us.
 // The chain's tables hold for states in [L, 2L) and tables whose steps stay
 // there; anything else, and the stream's last bits, take plain_step.
+//
+// Long streams are first decoded in parallel.  A state holds ten bits, of which
+// each step replaces some by stream bits, so decoders that start at different
+// (bit, state) places of one stream mostly end in the same chain after some
+// hundred symbols (measured over rounded normals of 2 to 8 bits per symbol:
+// median 200 to 850, the last of 2000 starts 300 to 7000).  A tile of the stream
+// is cut into kSyncLanes segments of equal bits; a lane decodes its segment from
+// a guessed place, then again from the place where the lane before it ended,
+// until no lane's start changes: every start is then the end of the segment
+// before, from the tile's known first place on, so the chain is the serial one,
+// whatever the guesses were.  Lane j's start is right after j rounds at the
+// latest; lanes whose start did not change rest.  Streams that do not fall into
+// step (kSyncRounds, and half the lanes by round kSyncLook: four equally likely
+// symbols, for one, keep odd and even bits apart) keep the segments that are
+// proven and go on serially.  The steps are those of the longest way into step
+// instead of the whole stream's: 16 streams of 32768 symbols of 4 to 5 bits
+// 1434 -> 239 us, of 12000 symbols 549 -> 249 us, of 200000 8589 -> 1091 us.
 constexpr int kAhead = 5;
 constexpr int kWordRing = 256;   // stream words in LDS
+constexpr int kSyncLanes = 256;
+constexpr int kSyncRounds = 128;
+constexpr int kSyncLook = 16;
+// Taken where the way into step is short against the stream: from 8192 symbols
+// on (4200 symbols of 4 bits: 218 us serially, 332 so), more with fewer bits per
+// symbol, as the way grows with about the inverse square of these (streams of 2
+// to 3 bits: 16384 symbols 657 us serially, 714 so, 32768 symbols 1260 and 630).
+// Not for more streams than the two-symbol table is taken for, whose waves share
+// the SIMDs (600 streams of 8192 symbols: 589 us serially, 706 so).
+constexpr int kSyncMin = 8192;
+__device__ __forceinline__ bool sync_pays(int64_t n, int64_t nb) {
+    return n >= kSyncMin && nb >= kSyncMin && (double)nb * (double)nb >= 1.5e5 * (double)n;
+}
 
 template <bool PAIR>
 __global__ __launch_bounds__(256) void k_decode_streams(
@@ -1854,14 +1884,21 @@ __global__ __launch_bounds__(256) void k_decode_streams(
     // two[slot << kAhead | next bits]: k1 | (64 - kAhead - k2) << 6 | next slot << 22, the
     // pair's first shift and second read; k1 = 0 and the first symbol's own k and slot
     // where it needs more than kAhead bits
+    // (before that table is built: a tile's words)
+    constexpr int kTileWords = 8191;
+    constexpr int64_t kTileBits = (kTileWords - 1) * 32;   // a step reads a word and the one behind it
+    static_assert(kTileBits + 10 < 1 << 18, "segment ends pack a bit position and a slot into 28 bits");
     __shared__ uint32_t two[PAIR ? kL << kAhead : 1];
     __shared__ uint32_t ring[kWordRing];
+    __shared__ int32_t alph[PAIR ? kL : 1];   // the symbols' values
+    __shared__ uint32_t s_end[PAIR ? kSyncLanes : 1];
+    __shared__ int s_sum[kSyncLanes / 64], s_first;
     __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63;
     const int t = blockIdx.x;
     const uint32_t* wb = reinterpret_cast<const uint32_t*>(bits);
-    const int64_t boff = bit_off[t];
-    const int64_t nb = nbits[t];
+    int64_t boff = bit_off[t];
+    int64_t nb = nbits[t];
     const int n = ndec[t];
     const int tb = tid_[t];
     const int32_t* LU = lookup + (int64_t)tb * kL;
@@ -1886,23 +1923,112 @@ __global__ __launch_bounds__(256) void k_decode_streams(
         }
     }
     __syncthreads();
+    int i = 0;   // symbols done
+    const bool chain = !s_bad && nb > 0;
     if constexpr (PAIR) {
-        for (int i = tid; i < kL << kAhead; i += 256) {
-            uint32_t e = one[i >> kAhead], ks = 0u;
-            const uint32_t k1 = e & 63u;
-            if (k1 <= (uint32_t)kAhead) {
-                ks = k1;
-                e = one[(e >> 16) + ((uint32_t)(i & ((1 << kAhead) - 1)) >> (kAhead - k1))];
+        if (chain && sync_pays(n, nb)) {   // (before the barrier behind the tile's words)
+            for (int j = tid; j < kL && j < max_sym; j += kSyncLanes) alph[j] = A[j];
+        }
+        while (chain && sync_pays(n - i, nb)) {   // uniform
+            // equal tiles of the bits that the symbols may take
+            const int64_t left = nb < 10 * (int64_t)(n - i) ? nb : 10 * (int64_t)(n - i);
+            const int64_t tiles = (left + kTileBits - 64) / (kTileBits - 63);
+            const int p0 = (int)(boff & 31);
+            // a step starts below `end`: within the tile, with its 10 bits there
+            const int64_t lastp = p0 + nb - 9;
+            const int64_t tend = p0 + (left + tiles - 1) / tiles;
+            const int end = (int)(tend < lastp ? tend : lastp);
+            const int seg = (end - p0 + kSyncLanes - 1) / kSyncLanes, cap = 4 * seg + 64;
+            const int64_t first = boff >> 5, lastw = (boff + nb - 1) >> 5;
+            for (int w = tid; w < (end >> 5) + 2; w += kSyncLanes)   // at most kTileWords
+                two[w] = wb[first + w < lastw ? first + w : lastw];
+            __syncthreads();
+            const int e0 = p0 + (tid + 1) * seg, stop = e0 < end ? e0 : end;
+            // a segment: the steps from (p, sl) that start before `stop` (at most cap:
+            // steps may read no bits); sym: the symbol index of each
+            auto walk = [&](int p, uint32_t sl, int* count, auto sym) -> uint32_t {
+                int c = 0;
+                auto step = [&](int j) {
+                    const uint32_t e = one[sl], k = e & 63u, *w = two + (p >> 5);
+                    const uint32_t v = __builtin_bitreverse32(__builtin_amdgcn_alignbit(w[1], w[0], (uint32_t)p));
+                    sl = (e >> 16) + (v >> 1 >> (31u - k));
+                    p += (int)k;
+                    sym(c + j, (e >> 6) & 1023u);
+                };
+                // four at a time without a test between them while they must start below
+                for (; p <= stop - 31 && c < cap; c += 4) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) step(j);
+                }
+                for (; p < stop && c < cap; c++) step(0);
+                *count = c;
+                return (uint32_t)p << 10 | sl;
+            };
+            uint32_t from = (uint32_t)(p0 + tid * seg < end ? p0 + tid * seg : end) << 10;
+            if (tid == 0) from |= x - (uint32_t)kL;
+            bool changed = true;
+            int count = 0, rounds = 0;
+            uint32_t to = 0;
+            for (;;) {
+                if (changed) to = walk((int)(from >> 10), from & 1023u, &count, [](int, uint32_t) {});
+                s_end[tid] = to;
+                if (tid == 0) s_first = kSyncLanes;
+                __syncthreads();
+                const uint32_t f = tid ? s_end[tid - 1] : from;
+                changed = f != from;
+                rounds++;
+                const bool look = rounds == kSyncLook;   // (the count takes longer than the test)
+                const int apart = look ? __syncthreads_count(changed ? 1 : 0) : __syncthreads_or(changed ? 1 : 0);
+                if (!apart || rounds == kSyncRounds || (look && apart > kSyncLanes / 2)) break;
+                from = f;
             }
-            two[i] = ks | ((uint32_t)(64 - kAhead) - (e & 63u)) << 6 | (e >> 16) << 22;
+            // the lanes before the first whose start would change: their segments are the chain's
+            if (changed) atomicMin(&s_first, tid);
+            __syncthreads();
+            const int good = s_first;   // at least `rounds` of them
+            const bool mine = tid < good;
+            const uint32_t sum = wave_incl_scan(mine ? (uint32_t)count : 0u);
+            if (lane == 63) s_sum[tid >> 6] = (int)sum;
+            __syncthreads();
+            int before = 0, total = 0;
+            for (int w = 0; w < kSyncLanes / 64; w++) {
+                if (w < (tid >> 6)) before += s_sum[w];
+                total += s_sum[w];
+            }
+            if (mine && count > 0) {
+                const int at = before + (int)sum - count, room = n - i - at;
+                int64_t* q = o + i + at;
+                int c2;
+                walk((int)(from >> 10), from & 1023u, &c2, [&](int c, uint32_t si) {
+                    if (c < room) q[c] = alph[si];
+                });
+            }
+            const uint32_t done = s_end[good - 1];
+            const int read = (int)(done >> 10) - p0;
+            i = total < n - i ? i + total : n;
+            boff += read;
+            nb -= read;
+            x = (uint32_t)kL + (done & 1023u);
+            __syncthreads();   // the tile and s_end are written again
+            if (good < kSyncLanes) break;
+        }
+        if (n - i >= 128) {   // uniform
+            for (int j = tid; j < kL << kAhead; j += 256) {
+                uint32_t e = one[j >> kAhead], ks = 0u;
+                const uint32_t k1 = e & 63u;
+                if (k1 <= (uint32_t)kAhead) {
+                    ks = k1;
+                    e = one[(e >> 16) + ((uint32_t)(j & ((1 << kAhead) - 1)) >> (kAhead - k1))];
+                }
+                two[j] = ks | ((uint32_t)(64 - kAhead) - (e & 63u)) << 6 | (e >> 16) << 22;
+            }
         }
         __syncthreads();
     }
     if (tid >= 64) return;   // the first wave decodes
 
-    int i = 0;         // symbols done
     int64_t pos = 0;   // bits read
-    if (!s_bad && nb > 0) {
+    if (chain && nb > 0 && i < n) {
         // Words from the one holding the stream's first bit (past the stream's
         // last: its last) reach the chain through a ring in LDS, topped up with
         // 64 of them per batch (load at its start, store at its end), and, within

@@ -157,6 +157,41 @@ def test_stream_coder_lengths_gpu(spread):
         assert np.array_equal(got, parts[i % 19][0])
 
 
+# the parallel decode: from 8192 symbols on (more with few bits per symbol), in
+# tiles of about 262000 bits; streams of four equally likely symbols move by two
+# bits per step, so starts on an odd bit never fall into step and the proven
+# segments go on serially; fewer symbols than the stream holds, and fewer bits
+# than the symbols take; beyond two streams per CU all goes serially
+@pytest.mark.parametrize("many", [False, True])
+def test_stream_decoder_parallel_gpu(many):
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(11)
+    parts = [_stream(rng, n, sp) for n, sp in [(8191, 3.0), (8192, 3.0), (30000, 0.6), (8203, 30.0), (33000, 9.0),
+                                               (70001, 4.0), (150000, 0.7), (131072, 12.0), (90000, 1.0)]]
+    four = [np.repeat(np.arange(4), n // 4) for n in (16384, 40004, 262144)]
+    for f in four:
+        rng.shuffle(f)
+        parts.append((f.astype(np.int64), np.full(4, len(f) // 4, np.int64), [0, 1, 2, 3]))
+    tabs = gpu_ans.build_rans_tables([p[1] for p in parts], [p[2] for p in parts])
+    assert all((t.freqs == 256).all() for t in tabs[-3:])
+    enc = gpu_ans.rans_encode_many([p[0] for p in parts], tabs)
+    streams, want = [], []
+    for (w, st, nb), p, t in zip(enc, parts, tabs):
+        for n in (len(p[0]), len(p[0]) - 1, 8192, 8400):
+            n = min(n, len(p[0]))
+            streams.append(gpu_ans.RANSStream(w, nb, st, n, t))
+            want.append(p[0][:n])
+        # the symbols whose bits are all there: a step takes at most 10
+        cut = nb * 2 // 3
+        streams.append(gpu_ans.RANSStream(w, cut, st, cut // 10, t))
+        want.append(p[0][:cut // 10])
+    if many:   # small streams fill the launch
+        streams += [streams[0]] * 520
+        want += [want[0]] * 520
+    for i, (got, ref) in enumerate(zip(gpu_ans.gpu_rans_decode(streams), want)):
+        assert np.array_equal(got, ref), (i, len(ref))
+
+
 def test_stream_decoder_truncated_gpu():
     """A stream with fewer bits than its symbols need is decoded to its length
     with the reference's rule (a step reads min(needed, bits left)), from any

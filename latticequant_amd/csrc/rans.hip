@@ -868,7 +868,10 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
         *reinterpret_cast<uint4*>(scr + (kCapW - 4 - (int)flushed)) = make_uint4(q[768], q[512], q[256], q[0]);
         flushed += 4u;
     };
-    // fewer than 4 words wait before a chunk and it completes at most 5: 8 fit the ring
+    // At most 127 bits wait before a chunk and its first 13 symbols add at most
+    // 130, so only the last emit can meet 8 complete words, with the one it
+    // fills the ring's ninth: four of them leave first (10 bits in nearly every
+    // symbol: alphabets near L).
     for_each_rev<4>(col.p, col.n, entries, [&](uint32_t e, int b, bool in) {
         uint32_t k;
         const uint32_t xin = x;
@@ -878,6 +881,7 @@ __global__ __launch_bounds__(256) void k_chunk_encode(const SymT* __restrict__ s
         alo = __builtin_amdgcn_alignbit(ahi, alo, k);
         ahi = __builtin_amdgcn_alignbit(xin, ahi, k);
         ks += k;
+        if (b == 0 && (total >> 5) >= flushed + (uint32_t)kEncRing) store4();
         if (b % 3 == 0) emit();
     }, [&]() {
         while ((total >> 5) >= flushed + 4u) store4();

@@ -157,6 +157,23 @@ def test_stream_coder_lengths_gpu(spread):
         assert np.array_equal(got, parts[i % 19][0])
 
 
+# alphabets of nearly L symbols, all about equally likely: nearly every symbol
+# takes 10 bits, the most a 16-symbol chunk can add to the encoder's ring of words
+@pytest.mark.parametrize("T", [256, 1031])
+def test_wide_encoder_ten_bits_per_symbol_gpu(T):
+    from latticequant_amd import codec
+    g = torch.Generator().manual_seed(T)
+    x = ((torch.rand(1, 2, T, 128, generator=g) - 0.5) * 990).to(torch.float16)
+    x[..., 7::8] *= 2   # the last coordinate's symbol is half of it
+    scale = torch.ones(2)
+    enc, _ = codec.encode_batch(x.cuda()[None], 4, scale32=scale, wide=True, escape=False)
+    ch = O.compress_chunk(x.numpy(), 4, scales_f32=scale.numpy())
+    base, nw = int(enc.chunk_base[0]), int(enc.chunk_words[0])
+    assert int(enc.stream_nbits.min()) > 9.5 * 0.4 * T * 2 * 16   # both cosets of every coordinate
+    assert np.array_equal(enc.words[base:base + nw].cpu().numpy().view(np.uint32), ch.bitstream)
+    assert np.array_equal(codec.decode_batch(enc)[0].cpu().numpy(), O.decompress_chunk(ch))
+
+
 # the parallel decode: from 8192 symbols on (more with few bits per symbol), in
 # tiles of about 262000 bits; streams of four equally likely symbols move by two
 # bits per step, so starts on an odd bit never fall into step and the proven

@@ -1378,7 +1378,7 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
         const uint32_t* __restrict__ blk_off, const int64_t* __restrict__ stream_nbits,
         const uint16_t* __restrict__ blk_state, const uint8_t* __restrict__ coset_bits,
         const lq_table* __restrict__ tables, const uint16_t* __restrict__ scale16,
-        int64_t n_chunks, int64_t n_heads, int64_t bph, int64_t nblk, int64_t tpw, int wpc, void* __restrict__ out,
+        int64_t n_chunks, int64_t n_heads, int64_t bph, int64_t nblk, int64_t span, int64_t tpw, int wpc, void* __restrict__ out,
         const int64_t* __restrict__ dseed, const float* __restrict__ signs, int lpr, float rdiv,
         const int32_t* __restrict__ esc_k, const int64_t* __restrict__ fine_off, const uint32_t* __restrict__ fine) {
     __shared__ uint32_t lut[LQ_STREAMS * kL];                               // 64 KB
@@ -1388,13 +1388,11 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
     const int tid = threadIdx.x;
     const float rrcp = ROT ? 1.0f / rdiv : 1.0f;   // the rotation's RN(1 / sqrt(head_dim))
     const int64_t V = n_heads * bph;
-    const int64_t per_chunk = (nblk + 3) / 4;   // tasks
-    const int64_t total = n_chunks * per_chunk;
-    // wpc > 0: wpc workgroups to a chunk, tpw tasks each; else tpw tasks each
-    // of the whole batch's
+    // the workgroup's tasks (decode_split): chunk c has numbers c * span .., its
+    // (nblk + 3) / 4 tasks first
     const int64_t wc = wpc > 0 ? (int64_t)blockIdx.x / wpc : 0;
-    const int64_t first = wc * per_chunk + ((int64_t)blockIdx.x - wc * wpc) * tpw;
-    const int64_t lim = wpc > 0 ? (wc + 1) * per_chunk : total;
+    const int64_t first = wc * span + ((int64_t)blockIdx.x - wc * wpc) * tpw;
+    const int64_t lim = wpc > 0 ? (wc + 1) * span : n_chunks * span;
     const int64_t last = first + tpw < lim ? first + tpw : lim;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     // The workgroup walks tasks first .. last - 1, chunk by chunk; wave w builds
@@ -1402,8 +1400,9 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
     // chunk's tasks w, w + 16, ..  Each wave stages its own 4 blocks' bitmaps
     // and moves to its next task without waiting for the other waves.
     for (int64_t t0 = first; t0 < last;) {
-    const int64_t chunk = t0 / per_chunk;
-    const int64_t tend = (chunk + 1) * per_chunk < last ? (chunk + 1) * per_chunk : last;
+    const int64_t chunk = t0 / span;
+    const int64_t tend = (chunk + 1) * span < last ? (chunk + 1) * span : last;
+    const int64_t tasks_end = chunk * span + (nblk + 3) / 4 < tend ? chunk * span + (nblk + 3) / 4 : tend;
     const bool lut_biased = chunk_biased(tables + chunk * LQ_STREAMS, lane);   // the LUTs' symbol fields
     if (t0 != first) __syncthreads();   // every wave is done with the previous chunk's LUTs
     {
@@ -1412,8 +1411,8 @@ __global__ __launch_bounds__(kDecThreads) void k_chunk_decode(
                  lut + wave * kL, lane);
     }
     __syncthreads();
-    for (int64_t task4 = t0 + wave; task4 < tend; task4 += kDecThreads / 64) {
-    const int64_t gbase = (task4 - chunk * per_chunk) * 4 - wave * 4;   // block b of the workgroup: gbase + b
+    for (int64_t task4 = t0 + wave; task4 < tasks_end; task4 += kDecThreads / 64) {
+    const int64_t gbase = (task4 - chunk * span) * 4 - wave * 4;   // block b of the workgroup: gbase + b
     __builtin_amdgcn_wave_barrier();
     for (int i = lane; i < 4 * (kBlk / 32 + 1); i += 64) {
         const int bl = wave * 4 + i / (kBlk / 32 + 1), w = i % (kBlk / 32 + 1);
@@ -2424,19 +2423,9 @@ static int chunk_decode_launch(const uint32_t* d_words, const int64_t* d_chunk_b
     // blocks) each has a SIMD to itself.  With 64 blocks per workgroup whatever
     // the size, and the LUTs from a launch of their own, 512 blocks (a chunk of
     // 2048 tokens) took 65.2 us, 8192 blocks 72.3 and 131072 blocks 525; now
-    // 39.4, 49.0 and 493.  Either every chunk is cut into equal
-    // parts (no workgroup crosses a chunk boundary), or the whole batch is cut
-    // into one part per CU, and a workgroup that crosses a boundary waits for
-    // its slowest wave there and builds the next chunk's LUTs, about what a
-    // round of 16 tasks costs: the equal parts unless they are 16 tasks longer.
-    const int64_t per_chunk = (nblk + 3) / 4, tasks = n_chunks * per_chunk;
-    const int64_t cus = device_cus();
-    const int64_t parts = n_chunks < cus ? cus / n_chunks : 1;
-    const int64_t tpw_c = (per_chunk + parts - 1) / parts, tpw_b = (tasks + cus - 1) / cus;
-    const bool by_chunk = tpw_c <= tpw_b + 16;
-    const int64_t tpw = by_chunk ? tpw_c : tpw_b;
-    const int wpc = by_chunk ? (int)((per_chunk + tpw - 1) / tpw) : 0;
-    const dim3 grid((unsigned)(by_chunk ? n_chunks * wpc : (tasks + tpw - 1) / tpw));
+    // 39.4, 49.0 and 493.
+    const DecodeSplit cut = decode_split(n_chunks, (nblk + 3) / 4, device_cus());
+    const dim3 grid((unsigned)cut.grid);
     const bool aligned = bph % kBlk == 0;
     const int lpr = d_signs ? head_dim / 8 : 1;
     const float div = d_signs ? (float)sqrt((double)head_dim) : 1.0f;
@@ -2445,7 +2434,7 @@ static int chunk_decode_launch(const uint32_t* d_words, const int64_t* d_chunk_b
 #define LQ_DECODE_E(DT, AL, DI, RO, ES)                                                                           \
     hipLaunchKernelGGL((k_chunk_decode<DT, AL, DI, RO, ES>), grid, dim3(kDecThreads), 0, s, d_words, d_chunk_base,      \
                        d_stream_woff, d_blk_off, d_stream_nbits, d_blk_state, d_coset_bits, d_tables, d_scale16,       \
-                       n_chunks, n_heads, bph, nblk, tpw, wpc, d_out, d_dither_seed, d_signs, lpr, div,         \
+                       n_chunks, n_heads, bph, nblk, cut.span, cut.tpw, cut.wpc, d_out, d_dither_seed, d_signs, lpr, div, \
                        d_esc_k, d_fine_off, d_fine)
 #define LQ_DECODE(DT, AL, DI, RO)                                                                                 \
     do {                                                                                                          \

@@ -27,6 +27,7 @@ def _x(C, H, T, hd, seed, dtype=torch.float16):
     (100, 8, 260, 128),    # 17 tasks per chunk, two parts
     (7, 8, 2100, 128),     # 132 tasks per chunk over 36 parts
     (129, 2, 1024, 128),   # one part of 16 tasks per chunk
+    (300, 1, 2080, 128),   # 17 tasks per chunk, more chunks than CUs: runs of whole rounds over chunk boundaries
 ])
 def test_decode_parts_gpu(C, H, T, hd):
     """Every chunk decoded in the batch equals the chunk decoded alone, and the

@@ -921,6 +921,41 @@ __device__ __forceinline__ void chunk_bases(const int64_t* chunk_words, int64_t 
     if (total && lane == 0) *total = carry;
 }
 
+// chunk_bases of many chunks, by one workgroup of its own.
+__global__ __launch_bounds__(1024) void k_chunk_bases(const int64_t* __restrict__ chunk_words, int64_t n_chunks,
+                                                      int64_t* __restrict__ chunk_base, int64_t* __restrict__ total) {
+    __shared__ int64_t wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int64_t carry = 0;
+    for (int64_t c0 = 0; c0 < n_chunks; c0 += 1024) {
+        const int64_t c = c0 + tid, v = c < n_chunks ? chunk_words[c] : 0;
+        int64_t incl = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t u = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += u;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        int64_t below = carry;
+#pragma unroll
+        for (int w = 0; w < 16; w++) {
+            const int64_t sum = wsum[w];
+            below += w < wave ? sum : 0;
+            carry += sum;
+        }
+        if (c < n_chunks) chunk_base[c] = below + incl - v;
+        __syncthreads();   // wsum is written again
+    }
+    if (total && tid == 0) *total = carry;
+}
+
+// Chunks up to which the scan's last workgroup makes the bases.  Every chunk pays
+// for it with a release and acquire of the L2 (the scan of 300 chunks 19.1 us
+// with them, 10.7 without, of 1000 chunks 46.3 and 19.5), a launch of its own
+// costs about 5 us whatever the batch.
+constexpr int64_t kBasesInScan = 64;
+
 // chunk_base (nullable; counter is then a cleared word): the workgroup that
 // finishes last also writes the chunks' bases.
 __global__ __launch_bounds__(1024) void k_chunk_scan_offsets(const uint32_t* __restrict__ blk_bits,
@@ -2183,9 +2218,12 @@ int encode_launch(const SymT* d_sym, const uint32_t* d_blk_n1, int64_t n_chunks,
         hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(256), 0, s, d_stream_nbits, d_tables, n_chunks, d_stream_woff,
                            d_chunk_words, d_chunk_base, h_total);
     } else {
+        const bool bases = d_chunk_base && n_chunks <= kBasesInScan;
         hipLaunchKernelGGL(k_chunk_scan_offsets, dim3((unsigned)n_chunks), dim3(64 * LQ_STREAMS), 0, s, bits,
                            d_blk_state, d_tables, nblk, d_blk_off, d_stream_nbits, d_stream_state, d_stream_woff,
-                           d_chunk_words, d_chunk_base, d_counter, h_total);
+                           d_chunk_words, bases ? d_chunk_base : nullptr, d_counter, h_total);
+        if (d_chunk_base && !bases)
+            hipLaunchKernelGGL(k_chunk_bases, dim3(1), dim3(1024), 0, s, d_chunk_words, n_chunks, d_chunk_base, h_total);
     }
     return launch_status();
 }

@@ -265,6 +265,76 @@ def test_write_call_sizes_gpu(C, T, wide, arena):
     assert torch.equal(given_scales.scale16, enc.scale16)
 
 
+def _us(f, n=20):
+    """Median time of f's work on the GPU, in microseconds."""
+    ts = []
+    for i in range(n + 3):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        ts.append(a.elapsed_time(b) * 1e3)
+    return sorted(ts[3:])[n // 2]
+
+
+# chunk bases by the scan's last workgroup (up to 64 chunks) and by a launch of
+# their own, 1024 chunks at a time
+@pytest.mark.parametrize("C", [64, 65, 1024, 1025, 2500])
+def test_write_call_bases_gpu(C):
+    from latticequant_amd import codec
+    x = _x(C, 1, 5, 8, C)
+    enc, _ = codec.encode_batch(x, 4)
+    cw = enc.chunk_words.cpu()
+    assert torch.equal(enc.chunk_base.cpu(), torch.cumsum(cw, 0) - cw)
+    assert enc.words.numel() == int(cw.sum()) + 2
+    one, _ = codec.encode_batch(x[C - 1:], 4)
+    assert torch.equal(enc.words[int(enc.chunk_base[-1]):-2], one.words[:-2])
+
+
+def test_write_call_many_chunks_time_gpu():
+    """The one call does what its launches made one by one do, whose chunk
+    bases come from torch.cumsum: with 16384 chunks of one block the GPU may not
+    take longer by more than a fifth (with a release and an acquire of the L2
+    per chunk it took a third longer; 4 % without)."""
+    from latticequant_amd import codec, _lib as L
+    C, V = 16384, 128
+    x = _x(C, 1, 8, 128, 1)
+    lib, s = L.lib(), L.stream_ptr(x.device)
+    arena = torch.zeros(codec.words_bound(C, V), dtype=torch.int32, device="cuda")
+    e, _ = codec.encode_batch(x, 4, words_out=arena, wide=False)
+    want = arena.clone()
+
+    def dev(n, dt):
+        return torch.empty(int(n), dtype=dt, device="cuda")
+
+    sym, work = dev(C * L.LQ_SYM_STRIDE, torch.int8), dev(lib.lq_chunk_encode_workspace(C, V), torch.uint8)
+    fd, sums, cw = dev(C, torch.int32), dev(4096 + C, torch.float64), torch.zeros(C + 1, dtype=torch.int64, device="cuda")
+
+    def launches():
+        e.hist.zero_(), e.status.zero_()
+        L.check(lib.lq_head_scales(x.data_ptr(), L.LQ_F16, C, 1, V, e.bits.data_ptr(), sums.data_ptr(), e.sigma2.data_ptr(),
+                                   e.scale32.data_ptr(), e.scale16.data_ptr(), fd.data_ptr(), s), "scales")
+        L.check(lib.lq_chunk_quantize(x.data_ptr(), L.LQ_F16, C, 1, V, e.scale32.data_ptr(), fd.data_ptr(), sym.data_ptr(),
+                                      e.coset_bits.data_ptr(), e.blk_n1.data_ptr(), e.hist.data_ptr(), e.status.data_ptr(),
+                                      None, L.LQ_F16, None, s), "quantize")
+        L.check(lib.lq_chunk_tables(e.hist.data_ptr(), C, e.tables.data_ptr(), e.status.data_ptr(), s), "tables")
+        L.check(lib.lq_chunk_encode(sym.data_ptr(), e.blk_n1.data_ptr(), C, V, e.tables.data_ptr(), work.data_ptr(),
+                                    e.blk_off.data_ptr(), e.blk_state.data_ptr(), e.stream_nbits.data_ptr(),
+                                    e.stream_state.data_ptr(), e.stream_woff.data_ptr(), cw[1:].data_ptr(), s), "encode")
+        base = torch.cumsum(cw[:C], 0)
+        L.check(lib.lq_chunk_pack(C, V, e.tables.data_ptr(), work.data_ptr(), e.blk_off.data_ptr(),
+                                  e.stream_nbits.data_ptr(), e.stream_woff.data_ptr(), base.data_ptr(), arena.data_ptr(),
+                                  s), "pack")
+
+    arena.zero_()
+    one = _us(lambda: codec.encode_batch(x, 4, words_out=arena, wide=False))
+    arena.zero_()
+    apart = _us(launches)
+    assert torch.equal(arena, want)
+    assert one < 1.2 * apart, (one, apart)
+
+
 def test_write_call_overflow_leaves_arena_gpu():
     """One chunk of three outside int8: the batch is coded once, on int16
     symbols; words past its bitstreams are not touched."""

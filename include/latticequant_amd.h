@@ -364,8 +364,8 @@ int lq_build_tables(const int64_t *d_counts, const int64_t *d_count_off, const i
                     int32_t n_tables, int32_t *d_freqs, int32_t *d_cum, int32_t *d_lookup, int32_t *d_status,
                     hipStream_t s);
 
-/* rANS encode of n_streams streams of symbol indices (one workgroup each; the
- * tables are lq_build_tables': frequencies in [1, L] summing to L).
+/* rANS encode of n_streams streams of symbol indices (the tables are
+ * lq_build_tables': frequencies in [1, L] summing to L).
  * Stream t: d_idx + d_sym_off[t], length d_n[t], table freqs/cum at
  * d_tab_off[t].  Words go to d_words + d_word_off[t] (capacity
  * 10*n/32 + 2 words each); state and n_bits per stream.

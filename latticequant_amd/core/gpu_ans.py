@@ -105,7 +105,7 @@ def _contiguous(alphabet) -> bool:
 
 
 def _encode_many(symbol_lists, tables, dev):
-    """Encode several streams in one launch (one workgroup per stream)."""
+    """Encode several streams in one launch."""
     lib = L_.lib()
     s = L_.stream_ptr(dev)
     n_s = len(symbol_lists)

@@ -1717,57 +1717,125 @@ __global__ __launch_bounds__(256) void k_build_tables(const int64_t* __restrict_
 
 // ------------------------------------------------------ generic streams --
 
-// Encode of arbitrary streams, one workgroup per stream.  The stream is cut
-// into segments of kSegSyms symbols, one lane each; a lane finds the exact
-// state entering its segment as the chunk encoder does (an interval of states,
-// run over a growing window of the symbols behind the segment until it is one
-// state or the window reaches the stream's end, where the state is L), encodes
-// the segment into its LDS column, and the segments' bits are joined by a scan
-// of their counts.  Encoding runs from the stream's end, so a segment's place
-// is known from the end: the joined bits are right-aligned in the stream's
-// scratch words, and a last pass shifts them to the reference's layout (n_words
-// + 1 words, last zero).  Streams longer than kSegLanes segments take that
-// many at a time, from the end.  One lane per stream, symbol by symbol, took
-// 9278 us for 16 streams of 32768 symbols; this takes 52 us.
+// Encode of arbitrary streams.  A stream is cut into segments of kSegSyms
+// symbols, one lane each; a lane finds the exact state entering its segment as
+// the chunk encoder does (an interval of states, run over a growing window of
+// the symbols behind the segment until it is one state or the window reaches the
+// stream's end, where the state is L), encodes the segment into its LDS column,
+// and the segments' bits are joined by a scan of their counts.
+//
+// Workgroup b takes streams b, b + gridDim, ..  Streams of up to 64, 256, 1024
+// and 4096 symbols are taken together by as many groups of 1, 4, 16 and 64 lanes
+// as there are, each group writing its stream's words in place; longer ones by the
+// whole workgroup, one after the other (encode_long).  One lane per stream,
+// symbol by symbol, took 9278 us for 16 streams of 32768 symbols, 52 us so; one
+// workgroup per stream whatever its length took 7614 us for 32768 streams of 10
+// symbols, 125 for 512 of 10 and 578 for 2048 of 1000; a lane per stream 8, 8 and
+// 269; so 10, 8 and 27 us.
 // The tables are build_rans_table's (frequencies in [1, L], summing to L).
 constexpr int kSegSyms = 64;
 constexpr int kSegWords = 10 * kSegSyms / 32;   // at most 10 bits per symbol
 constexpr int kSegLanes = 1024;
+constexpr int kGroupSyms = 64 * kSegSyms;       // longest stream of a group of lanes
 
-__global__ __launch_bounds__(kSegLanes) void k_encode_streams(
-        const int32_t* __restrict__ idx, const int64_t* __restrict__ sym_off, const int64_t* __restrict__ nsym,
-        const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum, const int64_t* __restrict__ tab_off,
-        uint32_t* __restrict__ scratch, uint32_t* __restrict__ words, const int64_t* __restrict__ word_off,
-        int64_t* __restrict__ state_out, int64_t* __restrict__ nbits_out) {
-    __shared__ uint32_t seg[kSegWords][kSegLanes];   // 80 KB: a lane's bits, right-aligned in its column
-    __shared__ uint32_t wsum[kSegLanes / 64];
+// f(entry, in) for symbols j1 - 1 .. j0, U at a time with their loads together
+// (U of 8 where every lane has its own stream, i.e. its own 64-bit addresses)
+template <int U, typename F>
+__device__ __forceinline__ void seg_rev(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t j0, int64_t j1,
+                                        F&& f) {
+    for (int64_t j = j1; j > j0; j -= U) {
+        uint32_t e[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t p = j - 1 - u > j0 ? j - 1 - u : j0;
+            e[u] = (uint32_t)id[p];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) e[u] = encx_of(enc_pack((uint32_t)freqs[e[u]], (uint32_t)cum[e[u]]));
+#pragma unroll
+        for (int u = 0; u < U; u++) f(e[u], j - 1 - u >= j0);
+    }
+}
+
+// Segment [b, e) of a stream of n symbols into the lane's column, right-aligned
+// in the column's first *capw words; the count of its bits.  *xout: the state
+// it leaves.
+template <int U>
+__device__ __forceinline__ uint32_t seg_encode(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t b,
+                                               int64_t e, int64_t n, uint32_t (*seg)[kSegLanes], int tid, int* capw,
+                                               uint32_t* xout) {
+    uint32_t x = kL, total = 0;
+    for (int64_t window = 16; e < n; window *= 4) {
+        const int64_t top = e + window < n ? e + window : n;
+        uint32_t lo = kL, hi = top == n ? (uint32_t)kL : 2u * kL - 1u;
+        seg_rev<U>(id, freqs, cum, e, top, [&](uint32_t en, bool in) {
+            uint32_t l2 = lo, h2 = hi;
+            hull_step(l2, h2, en);
+            lo = in ? l2 : lo;
+            hi = in ? h2 : hi;
+        });
+        x = lo;
+        if (lo == hi) break;   // always so once the window ends at n
+    }
+    *capw = (int)((10 * (e - b) + 31) / 32);
+    int wpos = *capw - 1;
+    uint64_t acc = 0;
+    uint32_t nacc = 0;
+    seg_rev<U>(id, freqs, cum, b, e, [&](uint32_t en, bool in) {
+        uint32_t k;
+        const uint32_t xin = x, xn = encx_step(xin, en, &k);
+        if (in) {
+            acc = (acc << k) | (((uint64_t)__builtin_bitreverse32(xin) << k) >> 32);
+            nacc += k;
+            total += k;
+            x = xn;
+            if (nacc >= 32) {
+                nacc -= 32;
+                seg[wpos][tid] = (uint32_t)(acc >> nacc);
+                wpos = wpos > 0 ? wpos - 1 : 0;   // never below 0 with tables of the kind above
+            }
+        }
+    });
+    if (nacc) seg[wpos][tid] = (uint32_t)(acc << (32 - nacc));
+    *xout = x;
+    return total < 32u * (uint32_t)*capw ? total : 32u * (uint32_t)*capw;
+}
+
+// The total bits of a lane's column (right-aligned in capw words) to bits D ..
+// D + total - 1 of dst; a word shared with other lanes (SHARED) is merged into
+// its cleared place with an atomic.
+template <bool SHARED>
+__device__ __forceinline__ void seg_copy(const uint32_t (*seg)[kSegLanes], int tid, int capw, uint32_t total, int64_t D,
+                                         uint32_t* dst) {
+    const int sp0 = capw * 32 - (int)total;   // first bit in the column
+    for (int64_t w = D >> 5; total && w <= (D + total - 1) >> 5; w++) {
+        const int64_t lo = w * 32 > D ? w * 32 : D, hi = w * 32 + 32 < D + total ? w * 32 + 32 : D + total;
+        const int sp = sp0 + (int)(lo - D), take = (int)(hi - lo), wi = sp >> 5, sh = sp & 31;
+        uint64_t v = seg[wi][tid];
+        if (sh + take > 32) v |= (uint64_t)seg[wi + 1][tid] << 32;
+        const uint32_t bits = (uint32_t)(v >> sh);
+        if (take == 32) dst[w] = bits;
+        else if (SHARED) atomicOr(dst + w, (bits & ((1u << take) - 1u)) << (int)(lo - w * 32));
+        else dst[w] = bits & ((1u << take) - 1u);   // D = 0: the last word's low bits
+    }
+}
+
+// Stores of this wave have reached the L2, where the atomics of its CU work.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// A stream by the whole workgroup.  Encoding runs from the stream's end, so a
+// segment's place is known from the end: the joined bits are right-aligned in the
+// stream's scratch words, and a last pass shifts them to the reference's layout
+// (n_words + 1 words, last zero).  Streams longer than kSegLanes segments take
+// that many at a time, from the end.
+__device__ __forceinline__ void encode_long(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t n,
+                                            uint32_t* scr, uint32_t* out, int64_t* state_out, int64_t* nbits_out,
+                                            uint32_t (*seg)[kSegLanes], uint32_t* wsum) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t t = blockIdx.x;
-    const int64_t n = nsym[t];
-    const int32_t* id = idx + sym_off[t];
-    const int32_t* F = freqs + tab_off[t];
-    const int32_t* C = cum + tab_off[t];
     const int64_t cap = (10 * n + 31) / 32 + 2;
-    uint32_t* scr = scratch + word_off[t];
-    uint32_t* out = words + word_off[t];
     for (int64_t w = tid; w < cap; w += kSegLanes) scr[w] = 0u;
     const int64_t nseg = (n + kSegSyms - 1) / kSegSyms;
     int64_t done = 0;   // bits of the segments behind the current ones
-    // f(entry, in) for symbols j1 - 1 .. j0, 16 at a time with their loads together
-    auto rev = [&](int64_t j0, int64_t j1, auto&& f) {
-        for (int64_t j = j1; j > j0; j -= 16) {
-            uint32_t e[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const int64_t p = j - 1 - u > j0 ? j - 1 - u : j0;
-                e[u] = (uint32_t)id[p];
-            }
-#pragma unroll
-            for (int u = 0; u < 16; u++) e[u] = encx_of(enc_pack((uint32_t)F[e[u]], (uint32_t)C[e[u]]));
-#pragma unroll
-            for (int u = 0; u < 16; u++) f(e[u], j - 1 - u >= j0);
-        }
-    };
     for (int64_t s1 = nseg; s1 > 0; s1 -= kSegLanes) {
         const int64_t s0 = s1 > kSegLanes ? s1 - kSegLanes : 0;
         const int64_t g = s0 + tid;
@@ -1775,48 +1843,14 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
         int capw = 0;
         if (g < s1) {
             const int64_t b = g * kSegSyms, e = b + kSegSyms < n ? b + kSegSyms : n;
-            uint32_t x = kL;
-            for (int64_t window = 16; e < n; window *= 4) {
-                const int64_t top = e + window < n ? e + window : n;
-                uint32_t lo = kL, hi = top == n ? (uint32_t)kL : 2u * kL - 1u;
-                rev(e, top, [&](uint32_t en, bool in) {
-                    uint32_t l2 = lo, h2 = hi;
-                    hull_step(l2, h2, en);
-                    lo = in ? l2 : lo;
-                    hi = in ? h2 : hi;
-                });
-                x = lo;
-                if (lo == hi) break;   // always so once the window ends at n
-            }
-            capw = (int)((10 * (e - b) + 31) / 32);
-            int wpos = capw - 1;
-            uint64_t acc = 0;
-            uint32_t nacc = 0;
-            rev(b, e, [&](uint32_t en, bool in) {
-                uint32_t k;
-                const uint32_t xin = x, xn = encx_step(xin, en, &k);
-                if (in) {
-                    acc = (acc << k) | (((uint64_t)__builtin_bitreverse32(xin) << k) >> 32);
-                    nacc += k;
-                    total += k;
-                    x = xn;
-                    if (nacc >= 32) {
-                        nacc -= 32;
-                        seg[wpos][tid] = (uint32_t)(acc >> nacc);
-                        wpos = wpos > 0 ? wpos - 1 : 0;   // never below 0 with tables of the kind above
-                    }
-                }
-            });
-            if (nacc) seg[wpos][tid] = (uint32_t)(acc << (32 - nacc));
-            total = total < 32u * (uint32_t)capw ? total : 32u * (uint32_t)capw;
-            if (g == 0) state_out[t] = x;
+            uint32_t x;
+            total = seg_encode<16>(id, freqs, cum, b, e, n, seg, tid, &capw, &x);
+            if (g == 0) *state_out = x;
         }
         // bits of the segments behind mine in this tile
         const uint32_t incl = wave_incl_scan(total);
-        // the cleared words reach the L2, where the atomics below work; wsum of
-        // the previous tile is read
-        if (s1 == nseg) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __syncthreads();
+        stores_done();     // the cleared words
+        __syncthreads();   // and wsum of the tile before is read
         if (lane == 63) wsum[wave] = incl;
         __syncthreads();
         uint32_t upto = 0, tile = 0;
@@ -1827,22 +1861,10 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
             tile += v;
         }
         const int64_t behind = done + (int64_t)(tile - (upto + incl));
-        // my bits go to bits D .. D + total - 1 of the scratch words; words shared
-        // with other segments are merged with atomics
-        const int64_t D = cap * 32 - behind - total;
-        const int sp0 = capw * 32 - (int)total;   // first bit in my column
-        for (int64_t w = D >> 5; total && w <= (D + total - 1) >> 5; w++) {
-            const int64_t lo = w * 32 > D ? w * 32 : D, hi = w * 32 + 32 < D + total ? w * 32 + 32 : D + total;
-            const int sp = sp0 + (int)(lo - D), take = (int)(hi - lo), wi = sp >> 5, sh = sp & 31;
-            uint64_t v = seg[wi][tid];
-            if (sh + take > 32) v |= (uint64_t)seg[wi + 1][tid] << 32;
-            const uint32_t bits = (uint32_t)(v >> sh);
-            if (take == 32) scr[w] = bits;
-            else atomicOr(scr + w, (bits & ((1u << take) - 1u)) << (int)(lo - w * 32));
-        }
+        seg_copy<true>(seg, tid, capw, total, cap * 32 - behind - total, scr);
         done += tile;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    stores_done();
     __syncthreads();
     const int64_t nw = (done + 31) / 32, base = cap * 32 - done;   // scratch bit of the stream's first
     for (int64_t w = tid; w < nw; w += kSegLanes) {
@@ -1855,8 +1877,70 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
     }
     if (tid == 0) {
         out[nw] = 0u;
-        nbits_out[t] = done;
-        if (n == 0) state_out[t] = kL;
+        *nbits_out = done;
+    }
+}
+
+__global__ __launch_bounds__(kSegLanes) void k_encode_streams(
+        const int32_t* __restrict__ idx, const int64_t* __restrict__ sym_off, const int64_t* __restrict__ nsym,
+        const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum, const int64_t* __restrict__ tab_off,
+        int64_t n_streams, uint32_t* __restrict__ scratch, uint32_t* __restrict__ words,
+        const int64_t* __restrict__ word_off, int64_t* __restrict__ state_out, int64_t* __restrict__ nbits_out) {
+    __shared__ uint32_t seg[kSegWords][kSegLanes];   // 80 KB: a lane's bits, right-aligned in its column
+    __shared__ uint32_t wsum[kSegLanes / 64];
+    __shared__ int s_n[kSegLanes];   // lengths of the next streams, longer ones as kGroupSyms + 1
+    const int tid = threadIdx.x;
+    const int64_t stride = gridDim.x;
+    for (int64_t r0 = blockIdx.x; r0 < n_streams; r0 += stride * kSegLanes) {
+        const int64_t left = (n_streams - r0 + stride - 1) / stride;
+        const int cnt = (int)(left < kSegLanes ? left : kSegLanes);
+        const int64_t len = tid < cnt ? nsym[r0 + tid * stride] : 0;
+        s_n[tid] = (int)(len < kGroupSyms + 1 ? len : kGroupSyms + 1);
+        const bool longer = __syncthreads_or(len > kSegSyms ? 1 : 0) != 0;
+        const bool any_long = longer && __syncthreads_or(len > kGroupSyms ? 1 : 0) != 0;
+        for (int lw = 0; lw <= (longer ? 6 : 0); lw += 2) {   // groups of 1 << lw lanes
+            const int W = 1 << lw, gl = tid & (W - 1);
+            for (int i0 = 0; i0 < cnt; i0 += kSegLanes >> lw) {
+                const int i = i0 + (tid >> lw);
+                const int n = i < cnt ? s_n[i] : -1;
+                const bool act = n <= W * kSegSyms && n > (lw ? W / 4 * kSegSyms : -1);
+                if (!__any(act)) continue;
+                const int64_t t = act ? r0 + i * stride : 0;
+                uint32_t* const out = words + word_off[t];
+                uint32_t total = 0, x = kL;
+                int capw = 0;
+                const int b = gl * kSegSyms, e = b + kSegSyms < n ? b + kSegSyms : n;
+                if (act && b < n)
+                    total = seg_encode<8>(idx + sym_off[t], freqs + tab_off[t], cum + tab_off[t], b, e, n, seg, tid, &capw, &x);
+                uint32_t incl = total;   // scan over the group; every lane of the wave is here
+                for (int o = 1; o < W; o <<= 1) {
+                    const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 64);
+                    incl += gl >= o ? u : 0u;
+                }
+                const uint32_t bits = (uint32_t)__shfl((int)incl, tid | (W - 1), 64);
+                const uint32_t nw = (bits + 31u) / 32u;
+                if (lw == 0) {
+                    if (act) out[nw] = 0u;
+                    seg_copy<false>(seg, tid, capw, total, 0, out);
+                } else {
+                    if (act)
+                        for (uint32_t w = gl; w <= nw; w += W) out[w] = 0u;
+                    stores_done();
+                    seg_copy<true>(seg, tid, capw, total, incl - total, out);
+                }
+                if (act && gl == 0) {
+                    state_out[t] = x;
+                    nbits_out[t] = bits;
+                }
+            }
+        }
+        for (int i = 0; any_long && i < cnt; i++) {   // uniform
+            if (s_n[i] <= kGroupSyms) continue;
+            const int64_t t = r0 + i * stride;
+            encode_long(idx + sym_off[t], freqs + tab_off[t], cum + tab_off[t], nsym[t], scratch + word_off[t],
+                        words + word_off[t], state_out + t, nbits_out + t, seg, wsum);
+        }
+        __syncthreads();   // s_n is written again
     }
 }
 
@@ -2554,8 +2638,10 @@ int lq_rans_encode_streams(const int32_t* d_idx, const int64_t* d_sym_off, const
                            uint32_t* d_words, const int64_t* d_word_off, int64_t* d_state, int64_t* d_nbits,
                            hipStream_t s) {
     if (n_streams <= 0) return LQ_ERR_ARG;
-    hipLaunchKernelGGL(k_encode_streams, dim3((unsigned)n_streams), dim3(kSegLanes), 0, s, d_idx, d_sym_off, d_n, d_freqs,
-                       d_cum, d_tab_off, d_scratch, d_words, d_word_off, d_state, d_nbits);
+    const int64_t cus = device_cus();   // one workgroup per CU (its LDS)
+    hipLaunchKernelGGL(k_encode_streams, dim3((unsigned)(n_streams < cus ? n_streams : cus)), dim3(kSegLanes), 0, s, d_idx,
+                       d_sym_off, d_n, d_freqs, d_cum, d_tab_off, (int64_t)n_streams, d_scratch, d_words, d_word_off, d_state,
+                       d_nbits);
     return launch_status();
 }
 

@@ -158,6 +158,71 @@ def test_stream_coder_lengths_gpu(spread):
         assert np.array_equal(got, parts[i % 19][0])
 
 
+# streams of every group width (64, 256, 1024, 4096 symbols and one past each)
+# side by side in one launch: fewer streams than CUs, several per workgroup, more
+# than a workgroup's lanes
+@pytest.mark.parametrize("m", [40, 700, 40 + 256 * 1024])
+def test_stream_encoder_groups_gpu(m):
+    from latticequant_amd import _lib as L
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(m)
+    lens = [0, 1, 10, 63, 64, 65, 200, 255, 256, 257, 700, 1023, 1024, 1025, 3000, 4095, 4096, 4097, 5000]
+    if m > 4096:
+        lens = [n for n in lens if n <= 65] + [257]
+    kinds = [_stream(rng, n, sp) for sp in (0.0, 0.4, 3.0, 100.0) for n in lens]
+    tabs = gpu_ans.build_rans_tables([k[1] for k in kinds], [k[2] for k in kinds])
+    want = [O.rans_encode(s, O.build_rans_table(c, a)) for s, c, a in kinds]
+    order = rng.integers(0, len(kinds), m)
+    order[:min(m, len(kinds))] = np.arange(min(m, len(kinds)))
+    n = np.array([len(kinds[k][0]) for k in order], np.int64)
+    cap = (10 * n + 31) // 32 + 2
+    sym_off, word_off = (np.concatenate([[0], np.cumsum(v)[:-1]]) for v in (n, cap))
+    tsz = np.array([t.n_symbols + 1 for t in tabs])
+    toff = np.concatenate([[0], np.cumsum(tsz)[:-1]])
+
+    def dev(a, dt):
+        return torch.from_numpy(np.ascontiguousarray(a)).to(dt).cuda()
+
+    idx = dev(np.concatenate([kinds[k][0] - kinds[k][2][0] for k in order]), torch.int32)
+    so, ln, to, wo = (dev(a, torch.int64) for a in (sym_off, n, toff[order], word_off))
+    fr = dev(np.concatenate([np.append(t.freqs, 0) for t in tabs]), torch.int32)
+    cu = dev(np.concatenate([t.cumfreqs for t in tabs]), torch.int32)
+    scr, words = (torch.full((int(cap.sum()) + 8,), -9, dtype=torch.int32, device="cuda") for _ in range(2))
+    st, nb = (torch.full((m,), -1, dtype=torch.int64, device="cuda") for _ in range(2))
+    L.check(L.lib().lq_rans_encode_streams(idx.data_ptr(), so.data_ptr(), ln.data_ptr(), fr.data_ptr(), cu.data_ptr(),
+                                           to.data_ptr(), m, scr.data_ptr(), words.data_ptr(), wo.data_ptr(),
+                                           st.data_ptr(), nb.data_ptr(), L.stream_ptr(idx.device)), "encode")
+    words, st, nb = words.cpu().numpy().view(np.uint32), st.cpu().numpy(), nb.cpu().numpy()
+    assert np.array_equal(st, np.array([int(want[k][1]) for k in order]))
+    assert np.array_equal(nb, np.array([int(want[k][2]) for k in order]))
+    for i in list(range(min(m, 700))) + list(rng.integers(0, m, 3000)):
+        w = want[order[i]][0]
+        assert np.array_equal(words[word_off[i]:word_off[i] + len(w)], w), (i, n[i])
+    assert (words[int(cap.sum()):] == 0xfffffff7).all()
+
+
+def test_stream_encoder_many_short_time_gpu():
+    """8192 streams of 10 symbols take about the time of 16 (one lane each);
+    with a workgroup each they took 160 times as long."""
+    from latticequant_amd import _lib as L
+    from latticequant_amd.core import gpu_ans
+    tab = gpu_ans.build_rans_tables([np.array([3, 4, 1])], [[0, 1, 2]])[0]
+    us = []
+    for m in (16, 8192):
+        def dev(a, dt):
+            return torch.from_numpy(np.ascontiguousarray(a)).to(dt).cuda()
+
+        idx, so = dev(np.arange(10 * m) % 3, torch.int32), dev(np.arange(m) * 10, torch.int64)
+        ln, to, wo = dev(np.full(m, 10), torch.int64), dev(np.zeros(m), torch.int64), dev(np.arange(m) * 6, torch.int64)
+        fr, cu = dev(np.append(tab.freqs, 0), torch.int32), dev(tab.cumfreqs, torch.int32)
+        scr, words = (torch.zeros(6 * m, dtype=torch.int32, device="cuda") for _ in range(2))
+        st, nb = (torch.zeros(m, dtype=torch.int64, device="cuda") for _ in range(2))
+        us.append(_us(lambda: L.check(L.lib().lq_rans_encode_streams(
+            idx.data_ptr(), so.data_ptr(), ln.data_ptr(), fr.data_ptr(), cu.data_ptr(), to.data_ptr(), m, scr.data_ptr(),
+            words.data_ptr(), wo.data_ptr(), st.data_ptr(), nb.data_ptr(), L.stream_ptr(idx.device)), "encode")))
+    assert us[1] < 10 * us[0], us
+
+
 # alphabets of nearly L symbols, all about equally likely: nearly every symbol
 # takes 10 bits, the most a 16-symbol chunk can add to the encoder's ring of words
 @pytest.mark.parametrize("T", [256, 1031])

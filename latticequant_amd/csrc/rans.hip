@@ -1741,14 +1741,13 @@ constexpr int kGroupSyms = 64 * kSegSyms;       // longest stream of a group of 
 // f(entry, in) for symbols j1 - 1 .. j0, U at a time with their loads together
 // (U of 8 where every lane has its own stream, i.e. its own 64-bit addresses)
 template <int U, typename F>
-__device__ __forceinline__ void seg_rev(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t j0, int64_t j1,
-                                        F&& f) {
-    for (int64_t j = j1; j > j0; j -= U) {
+__device__ __forceinline__ void seg_rev(const int32_t* id, const int32_t* freqs, const int32_t* cum, int j0, int j1, F&& f) {
+    for (int j = j1; j > j0; j -= U) {
         uint32_t e[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int64_t p = j - 1 - u > j0 ? j - 1 - u : j0;
-            e[u] = (uint32_t)id[p];
+            const int p = j - 1 - u > j0 ? j - 1 - u : j0;
+            e[u] = (uint32_t)id[(uint32_t)p];
         }
 #pragma unroll
         for (int u = 0; u < U; u++) e[u] = encx_of(enc_pack((uint32_t)freqs[e[u]], (uint32_t)cum[e[u]]));
@@ -1757,27 +1756,35 @@ __device__ __forceinline__ void seg_rev(const int32_t* id, const int32_t* freqs,
     }
 }
 
-// Segment [b, e) of a stream of n symbols into the lane's column, right-aligned
-// in the column's first *capw words; the count of its bits.  *xout: the state
-// it leaves.
+// The state entering the segment that ends at e, from the symbols behind it up to
+// `end`, where the state is xend: an interval of states over windows of 16, 64, ..
+// `limit` symbols; 0 if that leaves more than one.
 template <int U>
-__device__ __forceinline__ uint32_t seg_encode(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t b,
-                                               int64_t e, int64_t n, uint32_t (*seg)[kSegLanes], int tid, int* capw,
-                                               uint32_t* xout) {
-    uint32_t x = kL, total = 0;
-    for (int64_t window = 16; e < n; window *= 4) {
-        const int64_t top = e + window < n ? e + window : n;
-        uint32_t lo = kL, hi = top == n ? (uint32_t)kL : 2u * kL - 1u;
-        seg_rev<U>(id, freqs, cum, e, top, [&](uint32_t en, bool in) {
+__device__ __forceinline__ uint32_t seg_state(const int32_t* id, const int32_t* freqs, const int32_t* cum, int e, int end,
+                                              uint32_t xend, int limit) {
+    if (e >= end) return xend;
+    for (int window = 16; window <= limit; window *= 4) {
+        const bool whole = e + window >= end;
+        uint32_t lo = whole ? xend : (uint32_t)kL, hi = whole ? xend : 2u * kL - 1u;
+        seg_rev<U>(id, freqs, cum, e, whole ? end : e + window, [&](uint32_t en, bool in) {
             uint32_t l2 = lo, h2 = hi;
             hull_step(l2, h2, en);
             lo = in ? l2 : lo;
             hi = in ? h2 : hi;
         });
-        x = lo;
-        if (lo == hi) break;   // always so once the window ends at n
+        if (lo == hi) return lo;   // always so once the window reaches the end
     }
-    *capw = (int)((10 * (e - b) + 31) / 32);
+    return 0;
+}
+
+// Segment [b, e) of a stream, entered in state *xio, into the lane's column,
+// right-aligned in the column's first *capw words; the count of its bits.  *xio:
+// the state it leaves.
+template <int U>
+__device__ __forceinline__ uint32_t seg_encode(const int32_t* id, const int32_t* freqs, const int32_t* cum, int b, int e,
+                                               uint32_t (*seg)[kSegLanes], int tid, int* capw, uint32_t* xio) {
+    uint32_t x = *xio, total = 0;
+    *capw = (10 * (e - b) + 31) / 32;
     int wpos = *capw - 1;
     uint64_t acc = 0;
     uint32_t nacc = 0;
@@ -1797,7 +1804,7 @@ __device__ __forceinline__ uint32_t seg_encode(const int32_t* id, const int32_t*
         }
     });
     if (nacc) seg[wpos][tid] = (uint32_t)(acc << (32 - nacc));
-    *xout = x;
+    *xio = x;
     return total < 32u * (uint32_t)*capw ? total : 32u * (uint32_t)*capw;
 }
 
@@ -1827,10 +1834,62 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // segment's place is known from the end: the joined bits are right-aligned in the
 // stream's scratch words, and a last pass shifts them to the reference's layout
 // (n_words + 1 words, last zero).  Streams longer than kSegLanes segments take
-// that many at a time, from the end.
+// that many at a time (a tile), from the end; a tile's last state is the state the
+// tile behind it left.
+//
+// Long runs of one symbol of nearly all of L move the states round without ever
+// bringing them together, so a window there only ends at the tile's end.  Lanes
+// left without a state after kSegWindow symbols get it from the first wave, which
+// walks the segments behind them one after the other from a known state, the
+// entries of a segment loaded by its lanes: with windows to the stream's end a run
+// of 262144 symbols took 271 ms, of 32768 7.5 (one lane per stream 51 and 6.4); so
+// 16.2 and 1.9.
+constexpr int kSegWindow = 4096;
+struct LongLds {
+    uint32_t wsum[kSegLanes / 64];
+    uint32_t state[kSegLanes];               // entering states, 0: not known yet
+    uint64_t missing[kSegLanes / 64];        // the lanes without one, per wave
+    uint32_t tile_end;                       // the state the tile's last segment is entered in
+};
+
+// id: the tile's n symbols
+__device__ __forceinline__ void walk_missing(const int32_t* id, const int32_t* freqs, const int32_t* cum, int n, LongLds& l) {
+    const int lane = threadIdx.x & 63;
+    auto entry = [&](int i) {   // of symbol `lane` of the tile's segment i
+        const int p = i * kSegSyms + lane;
+        const uint32_t v = (uint32_t)id[(uint32_t)(p < n ? p : n - 1)];
+        return encx_of(enc_pack((uint32_t)freqs[v], (uint32_t)cum[v]));
+    };
+    int have = -1;   // the segment whose entries are here
+    uint32_t en = 0;
+    for (int w = kSegLanes / 64 - 1; w >= 0; w--) {
+        const uint64_t m0 = l.missing[w];
+        uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)m0) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(m0 >> 32)) << 32;
+        while (m) {
+            const int i = 64 * w + 63 - __builtin_clzll(m);   // behind it: segment i + 1, whose state is known
+            m &= ~(1ull << (i & 63));
+            if (have != i + 1) en = entry(i + 1);
+            const uint32_t next = entry(i);   // in flight during the steps
+            have = i;
+            uint32_t x = (uint32_t)__builtin_amdgcn_readfirstlane((int)l.state[i + 1]), k;
+            const int left = n - (i + 1) * kSegSyms;
+            if (left >= kSegSyms) {
+#pragma unroll
+                for (int j = kSegSyms - 1; j >= 0; j--) x = encx_step(x, (uint32_t)__builtin_amdgcn_readlane((int)en, j), &k);
+            } else {
+                for (int j = left - 1; j >= 0; j--) x = encx_step(x, (uint32_t)__builtin_amdgcn_readlane((int)en, j), &k);
+            }
+            if (lane == 0) l.state[i] = x;
+            WaveGroup::sync();
+            en = next;
+        }
+    }
+}
+
 __device__ __forceinline__ void encode_long(const int32_t* id, const int32_t* freqs, const int32_t* cum, int64_t n,
                                             uint32_t* scr, uint32_t* out, int64_t* state_out, int64_t* nbits_out,
-                                            uint32_t (*seg)[kSegLanes], uint32_t* wsum) {
+                                            uint32_t (*seg)[kSegLanes], LongLds& l) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t cap = (10 * n + 31) / 32 + 2;
     for (int64_t w = tid; w < cap; w += kSegLanes) scr[w] = 0u;
@@ -1838,25 +1897,34 @@ __device__ __forceinline__ void encode_long(const int32_t* id, const int32_t* fr
     int64_t done = 0;   // bits of the segments behind the current ones
     for (int64_t s1 = nseg; s1 > 0; s1 -= kSegLanes) {
         const int64_t s0 = s1 > kSegLanes ? s1 - kSegLanes : 0;
-        const int64_t g = s0 + tid;
-        uint32_t total = 0;
+        const int32_t* const tile_id = id + s0 * kSegSyms;
+        const int tn = (int)((s1 * kSegSyms < n ? s1 * kSegSyms : n) - s0 * kSegSyms);   // the tile's symbols
+        const int b = tid * kSegSyms, e = b + kSegSyms < tn ? b + kSegSyms : tn;
+        uint32_t total = 0, x = kL;
         int capw = 0;
-        if (g < s1) {
-            const int64_t b = g * kSegSyms, e = b + kSegSyms < n ? b + kSegSyms : n;
-            uint32_t x;
-            total = seg_encode<16>(id, freqs, cum, b, e, n, seg, tid, &capw, &x);
-            if (g == 0) *state_out = x;
+        if (b < tn) x = seg_state<16>(tile_id, freqs, cum, e, tn, s1 == nseg ? (uint32_t)kL : l.tile_end, kSegWindow);
+        const uint64_t missing = __ballot(x == 0);
+        l.state[tid] = x;
+        if (lane == 0) l.missing[wave] = missing;
+        if (__syncthreads_or(missing != 0 ? 1 : 0)) {
+            if (wave == 0) walk_missing(tile_id, freqs, cum, tn, l);
+            __syncthreads();
+            x = l.state[tid];
+        }
+        if (b < tn) {
+            total = seg_encode<16>(tile_id, freqs, cum, b, e, seg, tid, &capw, &x);
+            if (tid == 0) *state_out = l.tile_end = x;   // the last tile leaves the stream's
         }
         // bits of the segments behind mine in this tile
         const uint32_t incl = wave_incl_scan(total);
         stores_done();     // the cleared words
         __syncthreads();   // and wsum of the tile before is read
-        if (lane == 63) wsum[wave] = incl;
+        if (lane == 63) l.wsum[wave] = incl;
         __syncthreads();
         uint32_t upto = 0, tile = 0;
 #pragma unroll
         for (int w = 0; w < kSegLanes / 64; w++) {
-            const uint32_t v = wsum[w];
+            const uint32_t v = l.wsum[w];
             upto += w < wave ? v : 0u;
             tile += v;
         }
@@ -1887,7 +1955,7 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
         int64_t n_streams, uint32_t* __restrict__ scratch, uint32_t* __restrict__ words,
         const int64_t* __restrict__ word_off, int64_t* __restrict__ state_out, int64_t* __restrict__ nbits_out) {
     __shared__ uint32_t seg[kSegWords][kSegLanes];   // 80 KB: a lane's bits, right-aligned in its column
-    __shared__ uint32_t wsum[kSegLanes / 64];
+    __shared__ LongLds l;
     __shared__ int s_n[kSegLanes];   // lengths of the next streams, longer ones as kGroupSyms + 1
     const int tid = threadIdx.x;
     const int64_t stride = gridDim.x;
@@ -1910,8 +1978,11 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
                 uint32_t total = 0, x = kL;
                 int capw = 0;
                 const int b = gl * kSegSyms, e = b + kSegSyms < n ? b + kSegSyms : n;
-                if (act && b < n)
-                    total = seg_encode<8>(idx + sym_off[t], freqs + tab_off[t], cum + tab_off[t], b, e, n, seg, tid, &capw, &x);
+                if (act && b < n) {
+                    const int32_t *id = idx + sym_off[t], *F = freqs + tab_off[t], *C = cum + tab_off[t];
+                    x = seg_state<8>(id, F, C, e, n, kL, 4 * kGroupSyms);   // its windows reach the end
+                    total = seg_encode<8>(id, F, C, b, e, seg, tid, &capw, &x);
+                }
                 uint32_t incl = total;   // scan over the group; every lane of the wave is here
                 for (int o = 1; o < W; o <<= 1) {
                     const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 64);
@@ -1938,7 +2009,7 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
             if (s_n[i] <= kGroupSyms) continue;
             const int64_t t = r0 + i * stride;
             encode_long(idx + sym_off[t], freqs + tab_off[t], cum + tab_off[t], nsym[t], scratch + word_off[t],
-                        words + word_off[t], state_out + t, nbits_out + t, seg, wsum);
+                        words + word_off[t], state_out + t, nbits_out + t, seg, l);
         }
         __syncthreads();   // s_n is written again
     }

@@ -204,23 +204,58 @@ def test_stream_encoder_groups_gpu(m):
 def test_stream_encoder_many_short_time_gpu():
     """8192 streams of 10 symbols take about the time of 16 (one lane each);
     with a workgroup each they took 160 times as long."""
+    us = [_encode_us(np.array([3, 4, 1]), np.arange(10) % 3, m)[0] for m in (16, 8192)]
+    assert us[1] < 10 * us[0], us
+
+
+def _encode_us(counts, idx, m):
+    """Time of lq_rans_encode_streams for m copies of one stream, in
+    microseconds, and the (state, bits) of the last."""
     from latticequant_amd import _lib as L
     from latticequant_amd.core import gpu_ans
-    tab = gpu_ans.build_rans_tables([np.array([3, 4, 1])], [[0, 1, 2]])[0]
-    us = []
-    for m in (16, 8192):
-        def dev(a, dt):
-            return torch.from_numpy(np.ascontiguousarray(a)).to(dt).cuda()
+    tab = gpu_ans.build_rans_tables([counts], [list(range(len(counts)))])[0]
+    n, cap = len(idx), (10 * len(idx) + 31) // 32 + 2
 
-        idx, so = dev(np.arange(10 * m) % 3, torch.int32), dev(np.arange(m) * 10, torch.int64)
-        ln, to, wo = dev(np.full(m, 10), torch.int64), dev(np.zeros(m), torch.int64), dev(np.arange(m) * 6, torch.int64)
-        fr, cu = dev(np.append(tab.freqs, 0), torch.int32), dev(tab.cumfreqs, torch.int32)
-        scr, words = (torch.zeros(6 * m, dtype=torch.int32, device="cuda") for _ in range(2))
-        st, nb = (torch.zeros(m, dtype=torch.int64, device="cuda") for _ in range(2))
-        us.append(_us(lambda: L.check(L.lib().lq_rans_encode_streams(
-            idx.data_ptr(), so.data_ptr(), ln.data_ptr(), fr.data_ptr(), cu.data_ptr(), to.data_ptr(), m, scr.data_ptr(),
-            words.data_ptr(), wo.data_ptr(), st.data_ptr(), nb.data_ptr(), L.stream_ptr(idx.device)), "encode")))
-    assert us[1] < 10 * us[0], us
+    def dev(a, dt):
+        return torch.from_numpy(np.ascontiguousarray(a)).to(dt).cuda()
+
+    d_idx, so = dev(np.tile(idx, m), torch.int32), dev(np.arange(m) * n, torch.int64)
+    ln, to, wo = dev(np.full(m, n), torch.int64), dev(np.zeros(m), torch.int64), dev(np.arange(m) * cap, torch.int64)
+    fr, cu = dev(np.append(tab.freqs, 0), torch.int32), dev(tab.cumfreqs, torch.int32)
+    scr, words = (torch.zeros(cap * m, dtype=torch.int32, device="cuda") for _ in range(2))
+    st, nb = (torch.zeros(m, dtype=torch.int64, device="cuda") for _ in range(2))
+    us = _us(lambda: L.check(L.lib().lq_rans_encode_streams(
+        d_idx.data_ptr(), so.data_ptr(), ln.data_ptr(), fr.data_ptr(), cu.data_ptr(), to.data_ptr(), m, scr.data_ptr(),
+        words.data_ptr(), wo.data_ptr(), st.data_ptr(), nb.data_ptr(), L.stream_ptr(d_idx.device)), "encode"), 5)
+    return us, (int(st[-1]), int(nb[-1]))
+
+
+# runs over which states do not come together: one symbol with all of L, one of
+# nearly all of it, runs of such a symbol between others, cut at tile ends
+@pytest.mark.parametrize("n", [4097, 5000, 20000, 65536, 65537, 140000])
+def test_stream_encoder_runs_gpu(n):
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(n)
+    runs = np.zeros(n, np.int64)
+    runs[rng.integers(0, n, 12)] = 1
+    half = np.where((np.arange(n) // (n // 3 + 1)) % 2 == 1, rng.integers(-3, 4, n), 0)
+    syms = [np.zeros(n, np.int64), np.zeros(n, np.int64), runs, half]
+    alphabets = [[0], [-2, -1, 0, 1, 2], [0, 1], list(range(-5, 6))]
+    counts = [np.array([np.count_nonzero(s == a) for a in al]) for s, al in zip(syms, alphabets)]
+    enc = gpu_ans.rans_encode_many(syms, gpu_ans.build_rans_tables(counts, alphabets))
+    for i, (s, c, al, (words, state, nbits)) in enumerate(zip(syms, counts, alphabets, enc)):
+        want = O.rans_encode(s, O.build_rans_table(c, al))
+        assert (state, nbits) == (int(want[1]), int(want[2])), i
+        assert np.array_equal(words, want[0]), i
+
+
+@pytest.mark.parametrize("counts", [[7], [0, 0, 7, 0, 0]])
+def test_stream_encoder_one_symbol_time_gpu(counts):
+    """Four times as many equal symbols take about four times as long (with
+    windows to the stream's end: sixteen times, and more than one lane)."""
+    n = 60000
+    short, long = (_encode_us(np.array(counts), np.full(m, len(counts) // 2), 1)[0] for m in (n, 4 * n))
+    assert long < 7 * short, (short, long)
 
 
 # alphabets of nearly L symbols, all about equally likely: nearly every symbol

@@ -375,7 +375,7 @@ int lq_rans_encode_streams(const int32_t *d_idx, const int64_t *d_sym_off, const
                            int32_t n_streams, uint32_t *d_scratch, uint32_t *d_words, const int64_t *d_word_off,
                            int64_t *d_state, int64_t *d_nbits, hipStream_t s);
 
-/* Decode (one workgroup per stream) with the reference's bit-position guard; writes
+/* Decode with the reference's bit-position guard; writes
  * int64 symbol values.  Replaces _rans_decode_kernel (core/gpu_ans.py:175-235). */
 int lq_rans_decode_streams(const int32_t *d_bits, const int32_t *d_bit_off, const int32_t *d_nbits,
                            const int32_t *d_init, const int32_t *d_ndec, const int32_t *d_lookup,

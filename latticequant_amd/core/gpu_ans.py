@@ -260,7 +260,7 @@ def prepare_gpu_decode(streams: List[RANSStream], device: str = "cuda") -> Prepa
 
 
 def run_gpu_decode_kernel(prep: PreparedGPUDecode):
-    """Decode every stream, one workgroup each (core/gpu_ans.py:345-354)."""
+    """Decode every stream (core/gpu_ans.py:345-354)."""
     dev = prep.d_out.device
     with torch.cuda.device(dev):
         prep.d_out.zero_()

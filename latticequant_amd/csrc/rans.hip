@@ -2015,8 +2015,8 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
     }
 }
 
-// _rans_decode_kernel semantics (core/gpu_ans.py:175-235), one workgroup per
-// stream: renormalisation reads min(needed, n_bits - bit_pos) bits.
+// _rans_decode_kernel semantics (core/gpu_ans.py:175-235), a workgroup per stream
+// or, for short ones, a lane (lq_rans_decode_streams): renormalisation reads min(needed, n_bits - bit_pos) bits.
 //
 // A stream is one serial chain (every step needs the state before it), so the
 // kernel is arranged around that chain's latency: tables in LDS, bits in a
@@ -2031,7 +2031,7 @@ __global__ __launch_bounds__(kSegLanes) void k_encode_streams(
 // memory, bit by bit, took 30771 us for 16 streams of 32768 symbols,
 // the chain alone 1434 us.
 // The chain's tables hold for states in [L, 2L) and tables whose steps stay
-// there; anything else, and the stream's last bits, take plain_step.
+// there; anything else, and the stream's last bits, take plain_steps.
 //
 // Long streams are first decoded in parallel.  A state holds ten bits, of which
 // each step replaces some by stream bits, so decoders that start at different
@@ -2065,50 +2065,83 @@ __device__ __forceinline__ bool sync_pays(int64_t n, int64_t nb) {
     return n >= kSyncMin && nb >= kSyncMin && (double)nb * (double)nb >= 1.5e5 * (double)n;
 }
 
+struct StreamArgs {
+    const uint32_t* words;
+    const int32_t *bit_off, *nbits, *init, *ndec, *lookup, *freqs, *cum, *alphabet, *tid;
+    int32_t max_sym;
+    const int32_t* out_off;
+    int64_t* out;
+
+    __device__ __forceinline__ void tables(int64_t t, const int32_t** lu, const int32_t** f, const int32_t** c,
+                                           const int32_t** al) const {
+        const int64_t tb = tid[t];
+        *lu = lookup + tb * kL;
+        *f = freqs + tb * max_sym;
+        *c = cum + tb * max_sym;
+        *al = alphabet + tb * max_sym;
+    }
+};
+
+// The reference's step, from symbol i and state x with pos of the nb bits read
+__device__ __forceinline__ void plain_steps(int n, int i, uint32_t x, int64_t boff, int64_t nb, int64_t pos,
+                                            const uint32_t* __restrict__ wb, const int32_t* __restrict__ LU,
+                                            const int32_t* __restrict__ F, const int32_t* __restrict__ C,
+                                            const int32_t* __restrict__ A, int64_t* __restrict__ o, bool store) {
+    for (; i < n; i++) {
+        const uint32_t slot = x & (kL - 1);
+        const int si = LU[slot];
+        if (store) o[i] = A[si];
+        x = (uint32_t)F[si] * (x >> 10) + slot - (uint32_t)C[si];
+        if (x < (uint32_t)kL) {
+            int64_t k = (int64_t)__clz((int)x) - 21;
+            if (k > nb - pos) k = nb - pos;
+            for (int64_t q = 0; q < k; q++) {
+                const int64_t ab = boff + pos + q;
+                x = (x << 1) | ((wb[ab >> 5] >> (ab & 31)) & 1u);
+            }
+            pos += k;
+        }
+    }
+}
+
+constexpr int kTileWords = 8191;   // words of a tile of the parallel decode
 template <bool PAIR>
-__global__ __launch_bounds__(256) void k_decode_streams(
-        const int32_t* __restrict__ bits, const int32_t* __restrict__ bit_off, const int32_t* __restrict__ nbits,
-        const int32_t* __restrict__ init, const int32_t* __restrict__ ndec, const int32_t* __restrict__ lookup,
-        const int32_t* __restrict__ freqs, const int32_t* __restrict__ cum, const int32_t* __restrict__ alphabet,
-        const int32_t* __restrict__ tid_, int32_t max_sym, const int32_t* __restrict__ out_off,
-        int64_t* __restrict__ out) {
+struct DecodeLds {
     // one[slot]: k | symbol index << 6 | next slot before the k bits << 16
-    __shared__ uint32_t one[kL];
+    uint32_t one[kL];
     // two[slot << kAhead | next bits]: k1 | (64 - kAhead - k2) << 6 | next slot << 22, the
     // pair's first shift and second read; k1 = 0 and the first symbol's own k and slot
     // where it needs more than kAhead bits
     // (before that table is built: a tile's words)
-    constexpr int kTileWords = 8191;
+    uint32_t two[PAIR ? kL << kAhead : 1];
+    uint32_t ring[kWordRing];
+    int32_t alph[PAIR ? kL : 1];   // the symbols' values
+    uint32_t end[PAIR ? kSyncLanes : 1];
+    int sum[kSyncLanes / 64], first;
+    int bad;
+};
+
+// One stream, by the whole workgroup.
+template <bool PAIR, int NT>
+__device__ __forceinline__ void decode_stream(const uint32_t* __restrict__ wb, int64_t boff, int64_t nb, uint32_t x,
+                                              const int n, const int32_t* __restrict__ LU, const int32_t* __restrict__ F,
+                                              const int32_t* __restrict__ C, const int32_t* __restrict__ A,
+                                              const int max_sym, int64_t* __restrict__ o, DecodeLds<PAIR>& l) {
     constexpr int64_t kTileBits = (kTileWords - 1) * 32;   // a step reads a word and the one behind it
     static_assert(kTileBits + 10 < 1 << 18, "segment ends pack a bit position and a slot into 28 bits");
-    __shared__ uint32_t two[PAIR ? kL << kAhead : 1];
-    __shared__ uint32_t ring[kWordRing];
-    __shared__ int32_t alph[PAIR ? kL : 1];   // the symbols' values
-    __shared__ uint32_t s_end[PAIR ? kSyncLanes : 1];
-    __shared__ int s_sum[kSyncLanes / 64], s_first;
-    __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int t = blockIdx.x;
-    const uint32_t* wb = reinterpret_cast<const uint32_t*>(bits);
-    int64_t boff = bit_off[t];
-    int64_t nb = nbits[t];
-    const int n = ndec[t];
-    const int tb = tid_[t];
-    const int32_t* LU = lookup + (int64_t)tb * kL;
-    const int32_t* F = freqs + (int64_t)tb * max_sym;
-    const int32_t* C = cum + (int64_t)tb * max_sym;
-    const int32_t* A = alphabet + (int64_t)tb * max_sym;
-    int64_t* o = out + out_off[t];
-    if (n <= 0) return;   // uniform
-    uint32_t x = (uint32_t)init[t];
-    if (tid == 0) s_bad = x < (uint32_t)kL || x >= 2u * kL ? 1 : 0;
+    auto& one = l.one;
+    auto& two = l.two;
+    auto& ring = l.ring;
+    auto& alph = l.alph;
+    if (tid == 0) l.bad = x < (uint32_t)kL || x >= 2u * kL ? 1 : 0;
     __syncthreads();
-    for (int slot = tid; slot < kL; slot += 256) {
+    for (int slot = tid; slot < kL; slot += NT) {
         const int si = LU[slot];
         int64_t xp = 0;
         if (si >= 0 && si < max_sym && si < kL) xp = (int64_t)F[si] + slot - C[si];
         if (xp < 1 || xp >= 2 * kL) {
-            s_bad = 1;
+            l.bad = 1;
             one[slot] = 0u;
         } else {
             const uint32_t k = xp >= kL ? 0u : (uint32_t)(__clz((int)xp) - 21);
@@ -2117,7 +2150,7 @@ __global__ __launch_bounds__(256) void k_decode_streams(
     }
     __syncthreads();
     int i = 0;   // symbols done
-    const bool chain = !s_bad && nb > 0;
+    const bool chain = !l.bad && nb > 0;
     if constexpr (PAIR) {
         if (chain && sync_pays(n, nb)) {   // (before the barrier behind the tile's words)
             for (int j = tid; j < kL && j < max_sym; j += kSyncLanes) alph[j] = A[j];
@@ -2164,10 +2197,10 @@ __global__ __launch_bounds__(256) void k_decode_streams(
             uint32_t to = 0;
             for (;;) {
                 if (changed) to = walk((int)(from >> 10), from & 1023u, &count, [](int, uint32_t) {});
-                s_end[tid] = to;
-                if (tid == 0) s_first = kSyncLanes;
+                l.end[tid] = to;
+                if (tid == 0) l.first = kSyncLanes;
                 __syncthreads();
-                const uint32_t f = tid ? s_end[tid - 1] : from;
+                const uint32_t f = tid ? l.end[tid - 1] : from;
                 changed = f != from;
                 rounds++;
                 const bool look = rounds == kSyncLook;   // (the count takes longer than the test)
@@ -2176,17 +2209,17 @@ __global__ __launch_bounds__(256) void k_decode_streams(
                 from = f;
             }
             // the lanes before the first whose start would change: their segments are the chain's
-            if (changed) atomicMin(&s_first, tid);
+            if (changed) atomicMin(&l.first, tid);
             __syncthreads();
-            const int good = s_first;   // at least `rounds` of them
+            const int good = l.first;   // at least `rounds` of them
             const bool mine = tid < good;
             const uint32_t sum = wave_incl_scan(mine ? (uint32_t)count : 0u);
-            if (lane == 63) s_sum[tid >> 6] = (int)sum;
+            if (lane == 63) l.sum[tid >> 6] = (int)sum;
             __syncthreads();
             int before = 0, total = 0;
             for (int w = 0; w < kSyncLanes / 64; w++) {
-                if (w < (tid >> 6)) before += s_sum[w];
-                total += s_sum[w];
+                if (w < (tid >> 6)) before += l.sum[w];
+                total += l.sum[w];
             }
             if (mine && count > 0) {
                 const int at = before + (int)sum - count, room = n - i - at;
@@ -2196,7 +2229,7 @@ __global__ __launch_bounds__(256) void k_decode_streams(
                     if (c < room) q[c] = alph[si];
                 });
             }
-            const uint32_t done = s_end[good - 1];
+            const uint32_t done = l.end[good - 1];
             const int read = (int)(done >> 10) - p0;
             i = total < n - i ? i + total : n;
             boff += read;
@@ -2331,21 +2364,36 @@ __global__ __launch_bounds__(256) void k_decode_streams(
         pos = bits_read();
         x = slot + (uint32_t)kL;
     }
-    // the plain step (all lanes alike)
-    for (; i < n; i++) {
-        const uint32_t slot = x & (kL - 1);
-        const int si = LU[slot];
-        if (lane == 0) o[i] = A[si];
-        x = (uint32_t)F[si] * (x >> 10) + slot - (uint32_t)C[si];
-        if (x < (uint32_t)kL) {
-            int64_t k = (int64_t)__clz((int)x) - 21;
-            if (k > nb - pos) k = nb - pos;
-            for (int64_t q = 0; q < k; q++) {
-                const int64_t ab = boff + pos + q;
-                x = (x << 1) | ((wb[ab >> 5] >> (ab & 31)) & 1u);
-            }
-            pos += k;
+    plain_steps(n, i, x, boff, nb, pos, wb, LU, F, C, A, o, lane == 0);
+}
+
+// Streams of at most lanes_below symbols are taken by a lane each, in the first
+// lane_blocks workgroups: these do nothing else (PAIR: and then, as the others do,
+// a stream of their own).  The others take the rest, one after the other.
+template <bool PAIR, int NT>
+__global__ __launch_bounds__(NT) void k_decode_streams(StreamArgs a, int64_t n_streams, int lanes_below, int lane_blocks) {
+    __shared__ DecodeLds<PAIR> l;
+    if ((int)blockIdx.x < lane_blocks) {
+        // PAIR: one or two streams per workgroup, so that no CU waits for another
+        const int64_t t = PAIR ? blockIdx.x + (int64_t)threadIdx.x * lane_blocks : (int64_t)blockIdx.x * NT + threadIdx.x;
+        if (t < n_streams && a.ndec[t] <= lanes_below) {
+            const int32_t *LU, *F, *C, *A;
+            a.tables(t, &LU, &F, &C, &A);
+            plain_steps(a.ndec[t], 0, (uint32_t)a.init[t], a.bit_off[t], a.nbits[t], 0, a.words, LU, F, C, A,
+                        a.out + a.out_off[t], true);
         }
+        if (!PAIR) return;
+    }
+    const int64_t first = PAIR ? blockIdx.x : (int64_t)blockIdx.x - lane_blocks;
+    const int64_t stride = PAIR ? gridDim.x : (int64_t)gridDim.x - lane_blocks;
+    for (int64_t t = first; t < n_streams; t += stride) {
+        const int n = a.ndec[t];
+        if (n <= lanes_below) continue;   // uniform
+        const int32_t *LU, *F, *C, *A;
+        a.tables(t, &LU, &F, &C, &A);
+        decode_stream<PAIR, NT>(a.words, a.bit_off[t], a.nbits[t], (uint32_t)a.init[t], n, LU, F, C, A, a.max_sym,
+                                a.out + a.out_off[t], l);
+        __syncthreads();   // l is written again
     }
 }
 
@@ -2721,12 +2769,37 @@ int lq_rans_decode_streams(const int32_t* d_bits, const int32_t* d_bit_off, cons
                            const int32_t* d_alphabet, const int32_t* d_tid, int32_t max_sym, const int32_t* d_out_off,
                            int32_t n_streams, int64_t* d_out, hipStream_t s) {
     if (n_streams <= 0 || max_sym <= 0) return LQ_ERR_ARG;
-    if (n_streams <= 2 * device_cus())
-        hipLaunchKernelGGL(k_decode_streams<true>, dim3((unsigned)n_streams), dim3(256), 0, s, d_bits, d_bit_off, d_nbits,
-                           d_init, d_ndec, d_lookup, d_freqs, d_cum, d_alphabet, d_tid, max_sym, d_out_off, d_out);
-    else
-        hipLaunchKernelGGL(k_decode_streams<false>, dim3((unsigned)n_streams), dim3(256), 0, s, d_bits, d_bit_off, d_nbits,
-                           d_init, d_ndec, d_lookup, d_freqs, d_cum, d_alphabet, d_tid, max_sym, d_out_off, d_out);
+    const StreamArgs a = {reinterpret_cast<const uint32_t*>(d_bits), d_bit_off, d_nbits, d_init, d_ndec, d_lookup, d_freqs,
+                          d_cum, d_alphabet, d_tid, max_sym, d_out_off, d_out};
+    const int64_t cus = device_cus();
+    const int64_t n = n_streams;
+    // A lane per stream takes 0.7 us per symbol whatever the number of streams (up
+    // to some 30000); a workgroup per stream 0.08 or less, but about 10 us for its
+    // tables, and the CUs hold a few thousand at most.  us, lane / workgroup:
+    // 16 streams of 10 symbols 10.0 / 12.6, of 24 17.8 / 12.6; 512 of 32
+    // 21.2 / 22.9, of 128 73 / 90 (two at a time per CU), of 256 143 / 109; 2048 of
+    // 10 9.3 / 12.0, of 24 18.8 / 16.6; 4096 of 64 43 / 40, of 128 93 / 47; 8192 of
+    // 128 90 / 95, of 256 169 / 118; 16384 of 256 172 / 227; 32768 of 256 204 / 437.
+    if (n <= 2 * cus) {   // the two-symbol tables fill a CU's LDS
+        hipLaunchKernelGGL((k_decode_streams<true, 256>), dim3((unsigned)n), dim3(256), 0, s, a, n, n <= cus ? 16 : 128,
+                           (int)(n < cus ? n : cus));
+    } else {
+        const int64_t least = n <= 4 * cus ? 8 : 16;
+        const int64_t below = n >= 32768 ? INT_MAX : (n * n >> 18 > least ? n * n >> 18 : least);
+        // four waves build the tables faster while a CU has room for them, one wave
+        // leaves room for more streams (1024 of 64 symbols 20.3 us with four, 27
+        // with one; 2000 of 64 38 and 24.5, of 4000 590 and 338)
+        if (n <= 4 * cus) {
+            const int lane_blocks = (int)((n + 255) / 256);
+            hipLaunchKernelGGL((k_decode_streams<false, 256>), dim3((unsigned)(lane_blocks + n)), dim3(256), 0, s, a, n,
+                               (int)below, lane_blocks);
+        } else {
+            const int lane_blocks = (int)((n + 63) / 64);
+            const int64_t rest = below == INT_MAX ? 0 : (n < 32 * cus ? n : 32 * cus);
+            hipLaunchKernelGGL((k_decode_streams<false, 64>), dim3((unsigned)(lane_blocks + rest)), dim3(64), 0, s, a, n,
+                               (int)below, lane_blocks);
+        }
+    }
     return launch_status();
 }
 

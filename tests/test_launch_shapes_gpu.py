@@ -310,6 +310,49 @@ def test_stream_decoder_parallel_gpu(many):
         assert np.array_equal(got, ref), (i, len(ref))
 
 
+def _decode_case(rng, m, lens):
+    """m streams of lengths drawn from lens (each of them once at least), of a few
+    tables, as (streams, wanted symbols)."""
+    from latticequant_amd.core import gpu_ans
+    parts = [_stream(rng, n, 3.0) for n in lens]
+    tabs = gpu_ans.build_rans_tables([p[1] for p in parts], [p[2] for p in parts])
+    enc = gpu_ans.rans_encode_many([p[0] for p in parts], tabs)
+    one = [gpu_ans.RANSStream(w, nb, st, len(p[0]), t) for (w, st, nb), p, t in zip(enc, parts, tabs)]
+    order = np.concatenate([np.arange(len(lens)), rng.integers(0, len(lens), m - len(lens))])
+    rng.shuffle(order)
+    return [one[i] for i in order], [parts[i][0] for i in order]
+
+
+# around the numbers of streams at which the launch changes (one and two per CU,
+# four per CU, 32768), with streams on both sides of the length below which a lane
+# takes a stream: 16, 128, 8, 16, 64 (4100 streams), every length from 32768 on
+@pytest.mark.parametrize("m", [20, 256, 257, 512, 513, 1024, 1025, 2100, 4100, 32767, 32768])
+def test_stream_decoder_launches_gpu(m):
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(m)
+    lens = [1, 8, 9, 15, 16, 17, 63, 64, 65, 127, 128, 129, 200, 700] if m < 4096 else [1, 7, 16, 64, 65, 90]
+    streams, want = _decode_case(rng, m, lens)
+    got = gpu_ans.gpu_rans_decode(streams)
+    assert np.array_equal(np.concatenate(got), np.concatenate(want))
+
+
+@pytest.mark.parametrize("m,n,times", [(8192, 10, 1.6), (32768, 64, 1.8)])
+def test_stream_decoder_many_short_time_gpu(m, n, times):
+    """Short streams take about the time of 64 of them, however many there are: a
+    lane each (with a workgroup each 2.2 and 5 times as long)."""
+    from latticequant_amd.core import gpu_ans
+    rng = np.random.default_rng(n)
+    us = []
+    for k in (64, m):
+        streams, _ = _decode_case(rng, k, [n])
+        prep = gpu_ans.prepare_gpu_decode(streams)
+        if k == 64 and n > 16:   # 64 streams of this length a lane each: 0.7 us per symbol
+            us.append(0.7 * n)
+            continue
+        us.append(_us(lambda: gpu_ans.run_gpu_decode_kernel(prep)))
+    assert us[1] < times * us[0], us
+
+
 def test_stream_decoder_truncated_gpu():
     """A stream with fewer bits than its symbols need is decoded to its length
     with the reference's rule (a step reads min(needed, bits left)), from any

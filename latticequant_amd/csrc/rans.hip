@@ -2104,6 +2104,11 @@ __device__ __forceinline__ void plain_steps(int n, int i, uint32_t x, int64_t bo
     }
 }
 
+// The two-symbol table takes about 17 us to build and saves 0.04 us per symbol:
+// 140 symbols 36 us without and 50 with it, 400 54 and 62, 600 68 and 64 to 74,
+// 800 81 and 72, 4000 288 and 197.
+constexpr int kPairMin = 600;
+
 constexpr int kTileWords = 8191;   // words of a tile of the parallel decode
 template <bool PAIR>
 struct DecodeLds {
@@ -2150,6 +2155,7 @@ __device__ __forceinline__ void decode_stream(const uint32_t* __restrict__ wb, i
     }
     __syncthreads();
     int i = 0;   // symbols done
+    bool pairs = false;
     const bool chain = !l.bad && nb > 0;
     if constexpr (PAIR) {
         if (chain && sync_pays(n, nb)) {   // (before the barrier behind the tile's words)
@@ -2238,7 +2244,8 @@ __device__ __forceinline__ void decode_stream(const uint32_t* __restrict__ wb, i
             __syncthreads();   // the tile and s_end are written again
             if (good < kSyncLanes) break;
         }
-        if (n - i >= 128) {   // uniform
+        pairs = n - i >= kPairMin;   // uniform
+        if (pairs) {
             for (int j = tid; j < kL << kAhead; j += 256) {
                 uint32_t e = one[j >> kAhead], ks = 0u;
                 const uint32_t k1 = e & 63u;
@@ -2302,7 +2309,7 @@ __device__ __forceinline__ void decode_stream(const uint32_t* __restrict__ wb, i
         if constexpr (PAIR) {
             uint32_t ix = (slot << kAhead) | (uint32_t)(bb.buf >> (64 - kAhead));
             // 64 steps read at most 15 bits and decode at most two symbols each
-            while (n - i >= 128 && nb - bits_read() >= 64 * 15 + 64) {
+            while (pairs && n - i >= 128 && nb - bits_read() >= 64 * 15 + 64) {
                 open();
                 uint32_t trace = 0, e = two[ix];
 #pragma unroll 8
@@ -2777,11 +2784,11 @@ int lq_rans_decode_streams(const int32_t* d_bits, const int32_t* d_bit_off, cons
     // to some 30000); a workgroup per stream 0.08 or less, but about 10 us for its
     // tables, and the CUs hold a few thousand at most.  us, lane / workgroup:
     // 16 streams of 10 symbols 10.0 / 12.6, of 24 17.8 / 12.6; 512 of 32
-    // 21.2 / 22.9, of 128 73 / 90 (two at a time per CU), of 256 143 / 109; 2048 of
+    // 21.2 / 22.9, of 64 40 / 38 (two at a time per CU), of 200 112 / 77; 2048 of
     // 10 9.3 / 12.0, of 24 18.8 / 16.6; 4096 of 64 43 / 40, of 128 93 / 47; 8192 of
     // 128 90 / 95, of 256 169 / 118; 16384 of 256 172 / 227; 32768 of 256 204 / 437.
     if (n <= 2 * cus) {   // the two-symbol tables fill a CU's LDS
-        hipLaunchKernelGGL((k_decode_streams<true, 256>), dim3((unsigned)n), dim3(256), 0, s, a, n, n <= cus ? 16 : 128,
+        hipLaunchKernelGGL((k_decode_streams<true, 256>), dim3((unsigned)n), dim3(256), 0, s, a, n, n <= cus ? 16 : 48,
                            (int)(n < cus ? n : cus));
     } else {
         const int64_t least = n <= 4 * cus ? 8 : 16;

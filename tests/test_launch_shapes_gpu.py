@@ -325,12 +325,12 @@ def _decode_case(rng, m, lens):
 
 # around the numbers of streams at which the launch changes (one and two per CU,
 # four per CU, 32768), with streams on both sides of the length below which a lane
-# takes a stream: 16, 128, 8, 16, 64 (4100 streams), every length from 32768 on
+# takes a stream: 16, 48, 8, 16, 64 (4100 streams), every length from 32768 on
 @pytest.mark.parametrize("m", [20, 256, 257, 512, 513, 1024, 1025, 2100, 4100, 32767, 32768])
 def test_stream_decoder_launches_gpu(m):
     from latticequant_amd.core import gpu_ans
     rng = np.random.default_rng(m)
-    lens = [1, 8, 9, 15, 16, 17, 63, 64, 65, 127, 128, 129, 200, 700] if m < 4096 else [1, 7, 16, 64, 65, 90]
+    lens = [1, 8, 9, 15, 16, 17, 47, 48, 49, 64, 65, 128, 599, 600, 700] if m < 4096 else [1, 7, 16, 64, 65, 90]
     streams, want = _decode_case(rng, m, lens)
     got = gpu_ans.gpu_rans_decode(streams)
     assert np.array_equal(np.concatenate(got), np.concatenate(want))

@@ -595,7 +595,11 @@ def _dither_tensor(dither_seed, C: int, dev) -> Optional[torch.Tensor]:
     ds = [int(dither_seed)] * C if isinstance(dither_seed, int) else [int(v) for v in dither_seed]
     if len(ds) != C:
         raise ValueError("dither_seed must be an int or one seed per chunk")
-    # from pinned memory: a copy from pageable memory waits for the stream's earlier work
+    # from pinned memory: a copy from pageable memory waits for the stream's earlier
+    # work.  A graph would record the copy, not the seeds: its replays would read
+    # whatever the staging memory holds by then
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("dither seeds are copied from the host: not while a graph is captured")
     return torch.tensor(ds, dtype=torch.int64, pin_memory=True).to(dev, non_blocking=True)
 
 

@@ -478,6 +478,37 @@ def test_write_call_many_chunks_time_gpu():
     assert one < 1.2 * apart, (one, apart)
 
 
+def test_write_call_capture_gpu():
+    """Without dither the write into a caller's arena is launches only: a graph of
+    it gives the eager words on every replay, with new input too.  With dither
+    seeds, which come from the host, a capture is refused (a recorded copy would
+    read its staging memory again at every replay)."""
+    from latticequant_amd import codec
+    x = _x(2, 4, 300, 128, 1)
+    arena = torch.zeros(codec.words_bound(2, 4 * 300 * 16), dtype=torch.int32, device="cuda")
+    codec.encode_batch(x, 4, words_out=arena, wide=False)   # (the rates' tensor is made outside the graph)
+    side = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        enc, _ = codec.encode_batch(x, 4, words_out=arena, wide=False)
+    for seed in (1, 2, 3):
+        x.copy_(_x(2, 4, 300, 128, seed))
+        want, _ = codec.encode_batch(x, 4)
+        n = int(want.chunk_words.sum())
+        arena.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(arena[:n], want.words[:n]) and torch.equal(enc.chunk_base, want.chunk_base)
+    refused = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError):
+        with torch.cuda.graph(refused, stream=side):
+            codec.encode_batch(x, 4, words_out=arena, wide=False, dither_seed=[5, 6])
+    torch.cuda.synchronize()
+    again, _ = codec.encode_batch(x, 4)
+    assert torch.equal(again.words[:n], want.words[:n])   # (the slack words have no value)
+
+
 def test_write_call_overflow_leaves_arena_gpu():
     """One chunk of three outside int8: the batch is coded once, on int16
     symbols; words past its bitstreams are not touched."""

@@ -14,13 +14,12 @@
 // the true history.  If the interval has not collapsed the window grows, up to
 // the end of the stream where the state is exactly L.  Results are therefore
 // exact, and identical to a serial encode.
-#include <atomic>
 #include <climits>
-#include <thread>
 
 #include "lq_argsort.h"
 #include "lq_decode.h"
 #include "lq_launch.h"
+#include "lq_readpool.h"
 
 using namespace lq;
 
@@ -2447,64 +2446,6 @@ int tables_launch(const uint32_t* d_hist, int64_t n_chunks, lq_table* d_tables, 
     return launch_status();
 }
 
-// What lq_encode_chunks reads back: two words of pinned host memory that the
-// launches write, and an event after the launch that writes the last one.
-// Slots are taken for one call and given back at its end, to the device they
-// belong to (the event's); up to kReadSlots wait for the next call, the others
-// are freed.
-struct ReadSlot {
-    int64_t* host = nullptr;
-    hipEvent_t event = nullptr;
-    int device = -1;
-};
-
-constexpr int kReadSlots = 16;
-
-struct ReadPool {
-    std::atomic_flag busy = ATOMIC_FLAG_INIT;   // held for a scan of the slots
-    ReadSlot slots[kReadSlots];                 // host null: free place
-
-    void lock() { while (busy.test_and_set(std::memory_order_acquire)) std::this_thread::yield(); }
-    void unlock() { busy.clear(std::memory_order_release); }
-
-    bool take(ReadSlot* out) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return false;
-        ReadSlot s;
-        lock();
-        for (ReadSlot& p : slots)
-            if (p.host && p.device == dev) {
-                s = p;
-                p = ReadSlot();
-                break;
-            }
-        unlock();
-        if (!s.host) {
-            s.device = dev;
-            if (hipHostMalloc(reinterpret_cast<void**>(&s.host), 2 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess)
-                return false;
-            if (hipEventCreateWithFlags(&s.event, hipEventDisableTiming) != hipSuccess) {
-                (void)hipHostFree(s.host);
-                return false;
-            }
-        }
-        *out = s;
-        return true;
-    }
-    void give(const ReadSlot& s) {
-        lock();
-        for (ReadSlot& p : slots)
-            if (!p.host) {
-                p = s;
-                unlock();
-                return;
-            }
-        unlock();
-        (void)hipEventDestroy(s.event);
-        (void)hipHostFree(s.host);
-    }
-};
-
 ReadPool& read_pool() {
     static ReadPool p;   // trivially destroyed: the HIP runtime may be gone by then
     return p;
@@ -2560,7 +2501,7 @@ int lq_encode_chunks(const void* d_x, int dtype, int64_t n_chunks, int64_t n_hea
     clear.counter = counter;
     const bool reads = h_status || h_words;
     ReadSlot slot;
-    if (reads && !read_pool().take(&slot)) return LQ_ERR_LAUNCH;
+    if (reads && !read_pool().take(s, &slot)) return LQ_ERR_LAUNCH;
     auto run = [&]() -> int {
         int rc = scales_given
                      ? scale_fastdiv_launch(d_scale32, H, d_signs ? (int)LQ_F32 : dtype, fastdiv, d_scale16, clear, s)

@@ -263,7 +263,9 @@ int lq_chunk_pack(int64_t n_chunks, int64_t n_vectors, const lq_table *d_tables,
  * d_chunk_words first.  h_status, h_words (nullable, host memory): the call
  * returns once the OR of the chunks' status bits, and the sum of d_chunk_words,
  * are there (it waits for the table, or the offset, launch; those behind it run
- * on).  Without them it does not wait.  Replaces llm/compressed_kv_cache.py:188-263. */
+ * on).  Without them it does not wait.  For the wide path after an overflow,
+ * d_work begins with the fast-division words (lq_scale_fastdiv, one int32 per
+ * head) and ends with lq_chunk_encode_workspace bytes that it may use.  Replaces llm/compressed_kv_cache.py:188-263. */
 int64_t lq_encode_chunks_workspace(int64_t n_chunks, int64_t n_heads, int64_t bph);
 int lq_encode_chunks(const void *d_x, int dtype, int64_t n_chunks, int64_t n_heads, int64_t bph, int head_dim,
                      const float *d_signs, const int64_t *d_dither_seed, const int32_t *d_chunk_bits, int scales_given,

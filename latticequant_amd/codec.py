@@ -574,19 +574,28 @@ def encode_batch(x: torch.Tensor, bits, scale32: Optional[torch.Tensor] = None, 
             w = rotate_rows(x, rht_signs, inverse=False)
             return encode_batch(w, bits, scale32, deq_out, exact_size, words_out, wide, dither_seed,
                                 escape=escape)
+    attempt = None
     if wide is not True:
-        enc, deq = _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, wide == "auto", dither_seed, rht_signs)
-        if enc.words is not None:
+        enc, deq, attempt = _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, wide == "auto", dither_seed,
+                                         rht_signs)
+        if enc is not None:
             return enc, deq
         # a chunk's symbols left int8: the int16 path, with the same scales (it
         # reads the materialised rotation)
         if rht_signs is not None:
-            w = rotate_rows(x, rht_signs, inverse=False)
-            return encode_batch(w, bits, enc.scale32, deq_out, exact_size, words_out, wide, dither_seed, escape=escape)
-        scales = (enc.bits, enc.scale32, enc.scale16, enc.sigma2)
-    else:
-        scales = None
-    return _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide, dither_seed, escape)
+            x = rotate_rows(x, rht_signs, inverse=False)
+    return _encode_wide(x, bits, scale32, attempt, deq_out, exact_size, words_out, wide, dither_seed, escape)
+
+
+@dataclass
+class _Int8Attempt:
+    """What an int8 write that overflowed hands on to the int16 path."""
+    bits: torch.Tensor
+    scale32: torch.Tensor
+    scale16: torch.Tensor
+    sigma2: Optional[torch.Tensor]
+    dither_seed: Optional[torch.Tensor]
+    work: torch.Tensor   # lq_encode_chunks' workspace
 
 
 def _dither_tensor(dither_seed, C: int, dev) -> Optional[torch.Tensor]:
@@ -616,7 +625,8 @@ def _arena(words_out: Optional[torch.Tensor], C: int, V: int, dev) -> torch.Tens
 def _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, auto, dither_seed, rht_signs):
     """encode_batch on int8 symbols: one native call (lq_encode_chunks), which
     also reads back the chunks' status (auto) and total size (for an arena of
-    its own, exact_size); `auto` and a symbol outside int8: words is None."""
+    its own, exact_size).  Returns (batch, deq, None), or, with `auto` and a symbol
+    outside int8, (None, None, _Int8Attempt)."""
     lib = L.lib()
     C, B, H, T, hd = x.shape
     dev = x.device
@@ -658,8 +668,9 @@ def _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, auto, dither_
                                  chunk_words.data_ptr(), chunk_base.data_ptr(), L.ptr(words), 1 if auto else 0,
                                  work.data_ptr(), at if auto else None, at + 8 if sized else None, s),
             "lq_encode_chunks")
-    overflow = auto and bool(host[0] & L.LQ_ST_SYM_OVERFLOW)
-    if sized and not overflow:
+    if auto and host[0] & L.LQ_ST_SYM_OVERFLOW:
+        return None, None, _Int8Attempt(bits_t, scale32, scale16, sigma2, dseed, work)
+    if sized:
         words = _empty(host[1] + 2, torch.int32, dev)   # decoder read-ahead slack
         L.check(lib.lq_encode_chunks_pack(C, nh, bph, tables.data_ptr(), work.data_ptr(), blk_off.data_ptr(),
                                           stream_nbits.data_ptr(), stream_woff.data_ptr(), chunk_base.data_ptr(),
@@ -668,8 +679,8 @@ def _encode_int8(x, bits, scale32, deq_out, exact_size, words_out, auto, dither_
                         scale16=scale16, sigma2=sigma2, coset_bits=coset_bits.view(C, -1), blk_n1=blk_n1.view(C, -1),
                         tables=tables, blk_off=blk_off, blk_state=blk_state, stream_nbits=stream_nbits,
                         stream_state=stream_state, stream_woff=stream_woff, chunk_words=chunk_words,
-                        chunk_base=chunk_base, words=None if overflow else words, status=status, hist=hist,
-                        extra={"wide": False, "dither_seed": dseed, "esc": None}), deq
+                        chunk_base=chunk_base, words=words, status=status, hist=hist,
+                        extra={"wide": False, "dither_seed": dseed, "esc": None}), deq, None
 
 
 def _cut(dtype, dev, sizes):
@@ -681,9 +692,10 @@ def _cut(dtype, dev, sizes):
     return [p if p.numel() == n else p[:n] for p, n in zip(parts, sizes)]
 
 
-def _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide, dither_seed, escape):
-    """encode_batch on int16 symbols.  scales: (bits, scale32, scale16, sigma2)
-    of the int8 attempt, or None."""
+def _encode_wide(x, bits, scale32, attempt: Optional[_Int8Attempt], deq_out, exact_size, words_out, wide, dither_seed,
+                 escape):
+    """encode_batch on int16 symbols.  attempt: the int8 write that overflowed
+    (its scales, fast-division words and encoder workspace are used), or None."""
     lib = L.lib()
     C, B, H, T, hd = x.shape
     dev = x.device
@@ -692,12 +704,14 @@ def _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide,
     nblk = (V + L.LQ_BLK - 1) // L.LQ_BLK
     dt = L.dtype_code(x.dtype)
     s = L.stream_ptr(dev)
-    if scales is None:
+    ws = lib.lq_chunk_encode_workspace(C, V)
+    if attempt is None:
         bits_t, scale32, scale16, sigma2, fastdiv = _head_scales(x, bits, scale32)
-    else:
-        bits_t, scale32, scale16, sigma2 = scales
-        fastdiv = _empty(C * nh, torch.int32, dev)
-        L.check(lib.lq_scale_fastdiv(scale32.data_ptr(), C * nh, dt, fastdiv.data_ptr(), s), "lq_scale_fastdiv")
+        dseed = _dither_tensor(dither_seed, C, dev)
+        work = _empty(ws, torch.uint8, dev)
+    else:   # the workspace's first and last parts
+        bits_t, scale32, scale16, sigma2 = attempt.bits, attempt.scale32, attempt.scale16, attempt.sigma2
+        dseed, fastdiv, work = attempt.dither_seed, attempt.work[:4 * C * nh].view(torch.int32), attempt.work[-ws:]
     # every block's 64 bytes of coset bits are written by the quantizer (bits of
     # vectors past the end are zero), so no fill
     coset_bits = _empty(C * nblk * L.LQ_BLK // 8, torch.uint8, dev)
@@ -707,7 +721,6 @@ def _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide,
     status, cwz, hist = _zero_views(dev, (C, torch.int32), (C + 1, torch.int64), (C * L.LQ_STREAMS * L.LQ_L, torch.int32))
     deq = torch.empty_like(x) if deq_out else None
     tables = _empty(C * L.LQ_STREAMS * L.TABLE_BYTES, torch.uint8, dev)
-    dseed = _dither_tensor(dither_seed, C, dev)
     sym = _empty(C * nblk * L.LQ_SYM_STRIDE, torch.int16, dev)
     minmax = torch.empty(C * L.LQ_STREAMS, 2, dtype=torch.int32, device=dev)
     minmax[:, 0] = 2 ** 31 - 1
@@ -730,8 +743,6 @@ def _encode_wide(x, bits, scale32, scales, deq_out, exact_size, words_out, wide,
                                 "normalisation never terminates there); use more bits or smaller chunks")
         if st & L.LQ_ST_SYM_OVERFLOW:
             raise AlphabetError("a lattice symbol does not fit int16")
-    ws = lib.lq_chunk_encode_workspace(C, V)
-    work = _empty(ws, torch.uint8, dev)
     ntask = C * L.LQ_STREAMS * nblk
     blk_off = _empty(ntask, torch.int32, dev)
     blk_state = _empty(ntask, torch.int16, dev)

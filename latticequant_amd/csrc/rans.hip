@@ -2452,16 +2452,16 @@ ReadPool& read_pool() {
 }
 
 struct WriteWork {   // offsets into lq_encode_chunks' workspace
-    int64_t sums, fastdiv, counter, sym, enc, total;
+    int64_t fastdiv, sums, counter, sym, enc, total;
 };
 
 inline WriteWork write_layout(int64_t n_chunks, int64_t n_heads, int64_t bph) {
     auto al = [](int64_t b) { return (b + 255) / 256 * 256; };
     const int64_t H = n_chunks * n_heads, V = n_heads * bph, nblk = (V + kBlk - 1) / kBlk;
     WriteWork w;
-    w.sums = 0;
-    w.fastdiv = w.sums + al((4096 + H) * 8);
-    w.counter = w.fastdiv + al(H * 4);
+    w.fastdiv = 0;   // first, and enc last: a batch that overflows hands both on
+    w.sums = w.fastdiv + al(H * 4);
+    w.counter = w.sums + al((4096 + H) * 8);
     w.sym = w.counter + 256;
     w.enc = w.sym + al(n_chunks * nblk * kSymStride);
     w.total = w.enc + enc_layout(n_chunks, V).total;
@@ -2526,7 +2526,10 @@ int lq_encode_chunks(const void* d_x, int dtype, int64_t n_chunks, int64_t n_hea
             rc = lq_chunk_pack(n_chunks, V, d_tables, base + w.enc, d_blk_off, d_stream_nbits, d_stream_woff, d_chunk_base,
                                d_words, s);
         if (rc != LQ_OK || !reads) return rc;
-        // the launches behind the event go on while the caller reads on
+        // The launches behind the event go on while the caller reads on.  (Those of
+        // a batch whose streams were left empty run while its caller makes the wide
+        // path's arrays: leaving them out, by a wait before the scan, gave such a
+        // batch 0 to 10 us of 430 and cost every other small write 5 to 8 of 115.)
         if (hipEventSynchronize(slot.event) != hipSuccess) return LQ_ERR_LAUNCH;
         if (h_status) *h_status = slot.host[0];
         if (h_words) *h_words = slot.host[1];

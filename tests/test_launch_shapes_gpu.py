@@ -526,6 +526,36 @@ def test_write_call_overflow_leaves_arena_gpu():
     assert torch.equal(codec.decode_batch(enc), codec.decode_batch(ref))
 
 
+@pytest.mark.parametrize("rotated", [False, True])
+@pytest.mark.parametrize("given", [False, True])
+def test_write_call_overflow_once_gpu(rotated, given, monkeypatch):
+    """A batch that leaves int8 is tried on int8 once, and the int16 path takes over
+    its scales, their fast-division words and sigma^2: the batch is the one
+    wide=True writes."""
+    from latticequant_amd import _lib as L, codec
+    x = _x(2, 4, 300, 128, 9)
+    x[1, 0, 2, 7] *= 2000.0
+    signs = (torch.randint(0, 2, (8, 128), generator=torch.Generator().manual_seed(2)) * 2 - 1).float().cuda()
+    rows = codec.rotate_rows(x, signs, inverse=False) if rotated else x
+    s32, s16, _, s2 = codec.quantize_batch(rows, 5, with_sigma2=True)
+    kw = {"scale32": s32 if given else None, "dither_seed": [3, 4] if rotated else None}
+    want, _ = codec.encode_batch(rows, 5, wide=True, **kw)
+    calls, lib = [], L.lib()
+    for name in ("lq_encode_chunks", "lq_encode_chunks_pack", "lq_scale_fastdiv", "lq_head_scales"):
+        f = getattr(lib, name)
+        monkeypatch.setattr(lib, name, lambda *a, f=f, name=name: calls.append(name) or f(*a))
+
+    got, _ = codec.encode_batch(x, 5, rht_signs=signs if rotated else None, **kw)
+    monkeypatch.undo()
+    assert got.extra["wide"] and calls == ["lq_encode_chunks"]
+    assert torch.equal(got.scale32, s32) and torch.equal(got.scale16, s16)
+    assert got.sigma2 is None if given else torch.equal(got.sigma2, s2)
+    n = int(want.chunk_words.sum())
+    assert torch.equal(got.words[:n], want.words[:n]) and torch.equal(got.chunk_words, want.chunk_words)
+    for f in ("coset_bits", "blk_n1", "blk_off", "blk_state", "stream_nbits", "stream_state", "stream_woff", "chunk_base"):
+        assert torch.equal(getattr(got, f), getattr(want, f)), f
+
+
 def test_write_call_threads_gpu():
     """Calls from several threads on their own streams, each with its read-back."""
     import threading

@@ -557,28 +557,37 @@ def test_write_call_overflow_once_gpu(rotated, given, monkeypatch):
 
 
 def test_write_call_threads_gpu():
-    """Calls from several threads on their own streams, each with its read-back."""
+    """Calls from more threads at once than read-back slots are kept (16), on their
+    own streams, each with its read-back; every call ends and gives its words."""
     import threading
     from latticequant_amd import codec
-    xs = [_x(2, 4, 300 + 7 * i, 128, i) for i in range(6)]
+    n, rounds = 20, 4
+    xs = [_x(2, 4, 300 + 7 * i, 128, i) for i in range(n)]
     want = [codec.encode_batch(x, 4)[0] for x in xs]
     torch.cuda.synchronize()
-    bad = []
+    bad, done = [], []
+    together = threading.Barrier(n, timeout=60)
 
     def work(i):
-        s = torch.cuda.Stream()
-        with torch.cuda.stream(s):
-            for _ in range(8):
-                e, _ = codec.encode_batch(xs[i], 4)
-                s.synchronize()
-                if not (torch.equal(e.words[:-2], want[i].words[:-2]) and torch.equal(e.chunk_base, want[i].chunk_base)):
-                    bad.append(i)
-        s.synchronize()
+        try:
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                for _ in range(rounds):
+                    together.wait()
+                    e, _ = codec.encode_batch(xs[i], 4)
+                    s.synchronize()
+                    if not (torch.equal(e.words[:-2], want[i].words[:-2]) and torch.equal(e.chunk_base, want[i].chunk_base)):
+                        bad.append(i)
+                    done.append(i)
+            s.synchronize()
+        except Exception as e:   # a thread's exception would not fail the test by itself
+            bad.append(e)
+            together.abort()
 
-    ts = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(n)]
     [t.start() for t in ts]
     [t.join() for t in ts]
-    assert not bad
+    assert not bad and len(done) == n * rounds
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])

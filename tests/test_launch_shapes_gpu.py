@@ -599,8 +599,9 @@ def test_write_call_threads_gpu():
 ])
 def test_direct_updates_gpu(B, H, hd, steps, dtype, monkeypatch):
     """update()'s one-launch form against the general one (quantize, then
-    append): rows, scales, sigma^2 and bitstreams, with K and V at their own
-    rates, from contiguous, transposed and misaligned tensors, zero heads."""
+    append), taken exactly where it should be: rows, scales, sigma^2 and
+    bitstreams, with K and V at their own rates, from contiguous, transposed and
+    misaligned tensors, zero heads."""
     from latticequant_amd.allocation.eval_alloc import VariableRateKVCache
     g = torch.Generator().manual_seed(hd)
     kv = []
@@ -616,9 +617,22 @@ def test_direct_updates_gpu(B, H, hd, steps, dtype, monkeypatch):
             k = torch.cat([k.new_zeros(1), k.reshape(-1)])[1:].view(k.shape)
         kv.append((k, v))
 
+    # the one-launch form takes heads of up to 1023 vectors, up to 2^14 in all, on
+    # 16-byte boundaries
+    bph = [k.shape[2] * hd // 8 for k, _ in kv]
+    want_direct = [n <= 1023 and n * B * H <= 1 << 14 and (not k.is_contiguous() or k.data_ptr() % 16 == 0)
+                   for n, (k, _) in zip(bph, kv)]
+    assert any(want_direct) and not all(want_direct)
+    took = []
+    update_direct = VariableRateKVCache._update_direct
+
+    def recorded(*a):
+        r = update_direct(*a)
+        took.append(r is not None)
+        return r
+
     def fill(direct):
-        if not direct:
-            monkeypatch.setattr(VariableRateKVCache, "_update_direct", lambda *a: None)
+        monkeypatch.setattr(VariableRateKVCache, "_update_direct", recorded if direct else lambda *a: None)
         c = VariableRateKVCache([{"K": 3, "V": 5}, {"K": 4, "V": 4}], eval_only_no_entropy=False)
         outs = []
         for k, v in kv:
@@ -627,6 +641,7 @@ def test_direct_updates_gpu(B, H, hd, steps, dtype, monkeypatch):
         return c, outs
 
     a, oa = fill(True)
+    assert took == [d for d in want_direct for _ in range(2)]   # two layers
     b, ob = fill(False)
     for (ka, va), (kb, vb) in zip(oa, ob):
         assert torch.equal(ka, kb) and torch.equal(va, vb)

@@ -369,9 +369,10 @@ int lq_build_tables(const int64_t *d_counts, const int64_t *d_count_off, const i
 /* rANS encode of n_streams streams of symbol indices (the tables are
  * lq_build_tables': frequencies in [1, L] summing to L).
  * Stream t: d_idx + d_sym_off[t], length d_n[t], table freqs/cum at
- * d_tab_off[t].  Words go to d_words + d_word_off[t] (capacity
- * 10*n/32 + 2 words each); state and n_bits per stream.
- * d_scratch: same total capacity as d_words.  Replaces core/gpu_ans.py:105-139. */
+ * d_tab_off[t].  Words go to d_words + d_word_off[t]; a stream has
+ * (10*n + 31)/32 + 2 words of its own there and as many from the same offset in
+ * d_scratch (every one of these may be written).  State and n_bits per stream.
+ * Replaces core/gpu_ans.py:105-139. */
 int lq_rans_encode_streams(const int32_t *d_idx, const int64_t *d_sym_off, const int64_t *d_n,
                            const int32_t *d_freqs, const int32_t *d_cum, const int64_t *d_tab_off,
                            int32_t n_streams, uint32_t *d_scratch, uint32_t *d_words, const int64_t *d_word_off,

@@ -205,10 +205,6 @@ def words_bound(n_chunks: int, n_vectors: int) -> int:
     return n_chunks * ((10 * 8 * n_vectors + 31) // 32 + 2 * L.LQ_STREAMS) + 2
 
 
-def _zeros(n, dtype, dev):
-    return torch.zeros(int(n), dtype=dtype, device=dev)
-
-
 def _empty(n, dtype, dev):
     return torch.empty(int(n), dtype=dtype, device=dev)
 
@@ -252,11 +248,10 @@ def _bits_tensor(bits, C, dev):
     return b.to(dev)
 
 
-def _head_scales(x: torch.Tensor, bits, scale32: Optional[torch.Tensor], rht_signs: Optional[torch.Tensor] = None):
+def _head_scales(x: torch.Tensor, bits, scale32: Optional[torch.Tensor]):
     """Per-head scales of a (C, B, H, T, hd) batch: from sigma^2 on the device
     (llm/compressed_kv_cache.py:188-196) or the caller's fp32 scales, plus the
-    fast-division flags of the quantizer.  rht_signs: sigma^2 of the rows
-    rotated in the kernel (the flags are then 0: rotated values are fp32)."""
+    fast-division flags of the quantizer."""
     lib = L.lib()
     C, B, H, T, hd = x.shape
     dev = x.device
@@ -271,21 +266,15 @@ def _head_scales(x: torch.Tensor, bits, scale32: Optional[torch.Tensor], rht_sig
         sigma2 = _empty(C * nh, torch.float32, dev)
         scale32 = _empty(C * nh, torch.float32, dev)
         scale16 = _empty(C * nh, torch.float16, dev)
-        if rht_signs is not None:
-            L.check(lib.lq_head_scales_rht(x.data_ptr(), dt, C, nh, bph, hd, rht_signs.data_ptr(), bits_t.data_ptr(),
-                                           work.data_ptr(), sigma2.data_ptr(), scale32.data_ptr(), scale16.data_ptr(),
-                                           fastdiv.data_ptr(), s), "lq_head_scales_rht")
-        else:
-            L.check(lib.lq_head_scales(x.data_ptr(), dt, C, nh, bph, bits_t.data_ptr(), work.data_ptr(),
-                                       sigma2.data_ptr(), scale32.data_ptr(), scale16.data_ptr(), fastdiv.data_ptr(), s),
-                    "lq_head_scales")
+        L.check(lib.lq_head_scales(x.data_ptr(), dt, C, nh, bph, bits_t.data_ptr(), work.data_ptr(),
+                                   sigma2.data_ptr(), scale32.data_ptr(), scale16.data_ptr(), fastdiv.data_ptr(), s),
+                "lq_head_scales")
     else:
         scale32 = scale32.to(device=dev, dtype=torch.float32).contiguous().view(-1)
         if scale32.numel() != C * nh:
             raise ValueError("scale32 must hold one scale per head of every chunk")
         scale16 = scale32.to(torch.float16)
-        fd_dt = L.LQ_F32 if rht_signs is not None else dt
-        L.check(lib.lq_scale_fastdiv(scale32.data_ptr(), C * nh, fd_dt, fastdiv.data_ptr(), s), "lq_scale_fastdiv")
+        L.check(lib.lq_scale_fastdiv(scale32.data_ptr(), C * nh, dt, fastdiv.data_ptr(), s), "lq_scale_fastdiv")
     return bits_t, scale32, scale16, sigma2, fastdiv
 
 

@@ -210,9 +210,9 @@ constexpr int kQBlocksPerWG = 8;   // at most (quant_blocks_per_wg)
 constexpr int kHRow = 256 + 8;
 constexpr int64_t kMaxBph = 1 << 30;   // vectors per head (2^27 tokens of 128 dims): in-head offsets stay int32
 
-// One workgroup quantizes bpw consecutive LQ_BLK-vector blocks of one chunk.  Per block it writes the coset bitmap (wave ballots, i.e. the
-// reference's LSB-first pack_coset_bits layout), the coset-1 count and the
-// symbols in the interleaved column layout of sym_pos (element index; int8
+// One workgroup quantizes bpw consecutive LQ_BLK-vector blocks of one chunk.  Per
+// block it writes the coset bitmap (wave ballots, i.e. the reference's LSB-first
+// pack_coset_bits layout), the coset-1 count and the symbols in the interleaved column layout of sym_pos (element index; int8
 // symbols, or int16 for the wide path), staged in LDS so the global stores are
 // 16-byte and contiguous.  int8: the 16 x 256 symbol histograms accumulate in
 // LDS and are flushed once per workgroup; a symbol outside int8 sets
@@ -290,14 +290,16 @@ __device__ __forceinline__ void stage_minmax(const uint4& w, int row16, int n0, 
 // by the scale as IEEE division rounds (div_exact where the row and the scale
 // lie in its range); no dequantised output, at least 5 waves per SIMD.
 // LDT >= 0: the input dtype as a compile-time constant (the lean launches),
-// so no dtype test is kept live across the block loop.
-// VALU issue bounds the lean launches (131072 blocks of fp16: about 300
-// operations per vector and lane; 581 us with both D8 roundings' flips
-// resolved and no load ahead, 558 us with only the chosen one's, 513 us with
-// the next block's rows in flight; the bytes alone take 326 us).  6 waves per
-// SIMD is what their 75 to 77 vector registers allow; forcing 7 spills.  LPR > 0: the rotation's
+// so no dtype test is kept live across the block loop.  LPR > 0: the rotation's
 // lanes per row as a compile-time constant, so the butterfly stages are
 // straight-line code (no per-stage branch and register copies).
+//
+// VALU issue bounds the lean launches: at 131072 blocks of fp16 339 instructions
+// per vector, 1.19 of the launch's cycles at 4 per instruction (some issue
+// faster).  581 us with both D8 roundings' flips resolved and no load ahead (340
+// instructions, 1.03), 558 us with only the chosen one's, 513 us with the next
+// block's rows in flight; the bytes alone take 326 us.  6 waves per SIMD is what
+// their 75 to 77 vector registers allow; forcing 7 spills.
 template <typename SymT, bool DITHER, bool LEAN = false, bool ROT = false, int LDT = -1, int LPR = 0>
 __global__ __launch_bounds__(kQThreads, ROT ? 5 : (LEAN ? 6 : 1)) void k_chunk_quantize(
     const void* __restrict__ x, int dtype, int64_t n_heads, int64_t bph, int64_t nblk,

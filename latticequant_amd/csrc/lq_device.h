@@ -83,7 +83,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {   // round to nearest even, 
     return (uint16_t)(u >> 16);
 }
 
-// Load one 8-dim vector (index v) of an fp16 / bf16 / fp32 array as fp32.
 // The eight 16-bit values (fp16 or bf16) of one 16-byte row.
 __device__ __forceinline__ void unpack8(const uint4& r, int dtype, float x[8]) {
     const uint32_t w[4] = {r.x, r.y, r.z, r.w};
@@ -102,6 +101,7 @@ __device__ __forceinline__ void unpack8(const uint4& r, int dtype, float x[8]) {
     }
 }
 
+// Load one 8-dim vector (index v) of an fp16 / bf16 / fp32 array as fp32.
 __device__ __forceinline__ void load8(const void* base, int dtype, int64_t v, float x[8]) {
     if (dtype == LQ_F32) {
         const float4* p = reinterpret_cast<const float4*>(base) + 2 * v;
@@ -205,8 +205,7 @@ __host__ __device__ __forceinline__ int e8_nearest(const float x[8], float ic[8]
 // path: what the reference needs two complete D8 roundings and two distance
 // sums for is decided from the roundings' remainders, and only the chosen
 // rounding's flip is looked for.  The kernels that call this are bound by VALU
-// issue, so the count of instructions is their time (the int8 quantizer at
-// 131072 blocks: see k_chunk_quantize).
+// issue (the int8 quantizer at 131072 blocks: see k_chunk_quantize).
 //
 // With e1 = x - r1 and e2 = y - r2 (y = RN(x - 1/2); both differences exact),
 //   d1 = sum e1^2 + odd1 (1 - 2 |e1_j|),  d2 = sum e2^2 + odd2 (1 - 2 |e2_k|)

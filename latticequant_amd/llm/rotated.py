@@ -15,10 +15,10 @@ a times the E8 Voronoi cell and independent of x (per-dimension MSE
 G(E8) a^2, G(E8) = 0.0716821).  Chunk seeds default to the HeadRHT-style
 layer*10000 + kv*10 + 7.
 
-Everything runs in the library's kernels: lq_head_scales_rht and
-lq_chunk_quantize_rht rotate each row in registers (no rotated copy in
-memory) before the scale sums and the nearest-point search, then tables,
-encode, pack; lq_chunk_decode_rht removes the dither and rotates each row back
+Everything runs in the library's kernels: lq_encode_chunks with sign rows (the
+launches of lq_head_scales_rht and lq_chunk_quantize_rht) rotates each row in
+registers (no rotated copy in memory) before the scale sums and the
+nearest-point search, then tables, encode, pack; lq_chunk_decode_rht removes the dither and rotates each row back
 before its fp16 store.  The rotation's fp32 arithmetic is the one lq_rht
 applies to a materialised copy, so the streams are the same either way.
 """
